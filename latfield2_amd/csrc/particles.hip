@@ -2792,8 +2792,8 @@ __global__ void fill_int_kernel(int *__restrict__ p, int64_t n, int v) {
 // ---------------------------------------------------------------- particle statistics
 // The output[] reductions of updateVel / moveParticles (particles/LATfield2_Particles.hpp:
 // 788-807, 846-885) in FP64.  Each workgroup folds a grid-stride share of the particles and
-// then its lanes by a fixed tree; one thread per quantity folds the workgroups' partials in
-// index order.  The summation order depends only on np, so results repeat exactly.
+// then its lanes by a fixed tree; one workgroup per quantity folds the workgroups' partials
+// in the same way.  The summation order depends only on np, so results repeat exactly.
 static constexpr int RED_Q = 8;        // quantities per call
 static constexpr int RED_WG = 256;
 static constexpr int RED_BLOCKS = 1024;
@@ -2862,15 +2862,27 @@ __global__ __launch_bounds__(RED_WG) void parts_reduce_kernel(RedArgs A, double 
     }
 }
 
-// out[k] = the reference's starting value folded with every workgroup's partial in order
-__global__ void parts_reduce_final_kernel(RedArgs A, const double *__restrict__ partial, int nblocks,
-                                          double *__restrict__ out) {
-    const int k = threadIdx.x;
-    if (k >= A.nq || A.op[k] == RED_NONE) return;
+// out[k] = the reference's starting value folded with every workgroup's partial: one workgroup
+// per quantity, each thread a fixed share of the partials, then a fixed tree (one thread
+// folding 1024 partials one after the other took 211 us, a chain of dependent loads)
+__global__ __launch_bounds__(RED_WG) void parts_reduce_final_kernel(RedArgs A, const double *__restrict__ partial,
+                                                                    int nblocks, double *__restrict__ out) {
+    const int k = blockIdx.x;
     const int op = A.op[k];
-    double r = op == RED_OP_SUM ? 0.0 : (op == RED_OP_MIN ? 9223372036854775807.0 : -9223372036854775807.0);
-    for (int b = 0; b < nblocks; ++b) r = red_fold(op, r, partial[(int64_t)b * RED_Q + k]);
-    out[k] = r;
+    if (op == RED_NONE) return;
+    __shared__ double lds[RED_WG];
+    double r = red_identity(op);
+    for (int b = threadIdx.x; b < nblocks; b += RED_WG) r = red_fold(op, r, partial[(int64_t)b * RED_Q + k]);
+    lds[threadIdx.x] = r;
+    __syncthreads();
+    for (int h = RED_WG / 2; h > 0; h >>= 1) {
+        if ((int)threadIdx.x < h) lds[threadIdx.x] = red_fold(op, lds[threadIdx.x], lds[threadIdx.x + h]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        const double init = op == RED_OP_SUM ? 0.0 : (op == RED_OP_MIN ? 9223372036854775807.0 : -9223372036854775807.0);
+        out[k] = red_fold(op, init, lds[0]);
+    }
 }
 
 }  // namespace lf2mi
@@ -4150,7 +4162,7 @@ int lf2mi_parts_reduce(lf2mi_parts p, int n, const int *quantity, const int *red
         parts_reduce_kernel<true><<<nb, RED_WG, 0, st>>>(A, p->red);
     }
     LF2MI_LAUNCHED();
-    parts_reduce_final_kernel<<<1, RED_Q, 0, st>>>(A, p->red, nb, res);
+    parts_reduce_final_kernel<<<n, RED_WG, 0, st>>>(A, p->red, nb, res);
     LF2MI_LAUNCHED();
     double host[RED_Q];
     LF2MI_HIP(hipMemcpyAsync(host, res, sizeof(double) * n, hipMemcpyDeviceToHost, st));
