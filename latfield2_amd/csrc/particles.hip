@@ -12,8 +12,9 @@
 // (histogram -> scan -> scatter into the second buffer).
 //
 // F64 representation (the plain path): absolute FP64 positions and velocities in upload
-// order; deposits are per-particle FP64 atomics into the field and the gather reads phi
-// directly.
+// order, with a brick index beside them (bricks.hpp): deposits sum a brick's particles in an
+// FP64 LDS window, the gather reads a brick's window of phi.  Where few particles fall into a
+// brick both go particle by particle: FP64 atomics into the field, phi straight from HBM.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -21,6 +22,7 @@
 #include <new>
 #include <vector>
 
+#include "bricks.hpp"
 #include "common.hpp"
 
 namespace lf2mi {
@@ -2641,6 +2643,151 @@ __global__ void deposit_f64_kernel(Dep64Args A) {
     }
 }
 
+// ---- brick windows
+// One workgroup per group of up to B64_MERGE items of a brick: every particle's terms (the
+// same products as deposit_f64_kernel's) go into FP64 LDS windows, one per component over the
+// component's own nodes, and the windows' non-zero nodes then go to the field, component
+// fastest, with one atomic each.
+static constexpr int B64_MERGE = 8;
+// below this many particles per brick the windows' zeroing and flush cost more than the
+// particles' own atomics
+static constexpr int64_t B64_OCC = 24;
+
+// first value of component COMP's window (constexpr recursion over the components before it)
+template <int KIND, int COMP> constexpr int b64_off() {
+    if constexpr (COMP == 0) return 0;
+    else {
+        constexpr int M = Comp<KIND, COMP - 1>::MASK, G = Comp<KIND, COMP - 1>::NGP;
+        return b64_off<KIND, COMP - 1>() + tc_w(M, G, 0) * tc_w(M, G, 1) * tc_w(M, G, 2);
+    }
+}
+template <int KIND> constexpr int b64_size() {
+    constexpr int L = KindC<KIND>::C - 1, M = Comp<KIND, L>::MASK, G = Comp<KIND, L>::NGP;
+    return b64_off<KIND, L>() + tc_w(M, G, 0) * tc_w(M, G, 1) * tc_w(M, G, 2);
+}
+
+struct B64Particle {
+    int l[3];                     // cell in the brick
+    double vw[3][2], lw[3][2];    // vertex and link weights
+    int llo[3];                   // the first link node's offset (-1 or 0)
+};
+
+template <int KIND, int COMP>
+__device__ __forceinline__ void b64_add(double *__restrict__ win, const B64Particle &P, double q) {
+    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP;
+    constexpr int WX = tc_w(M, G, 0), WY = tc_w(M, G, 1);
+    int b[3];
+    double w[3][2];
+    constexpr int n[3] = {(G & 1) ? 1 : 2, (G & 2) ? 1 : 2, (G & 4) ? 1 : 2};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        const bool link = (M >> d) & 1, ngp = (G >> d) & 1;
+        b[d] = P.l[d] + (link ? P.llo[d] + 1 : 0);
+        w[d][0] = ngp ? 1.0 : (link ? P.lw[d][0] : P.vw[d][0]);
+        w[d][1] = ngp ? 0.0 : (link ? P.lw[d][1] : P.vw[d][1]);
+    }
+    double *o = win + b64_off<KIND, COMP>() + b[0] + WX * (b[1] + WY * b[2]);
+#pragma unroll
+    for (int k = 0; k < n[2]; ++k)
+#pragma unroll
+        for (int j = 0; j < n[1]; ++j)
+#pragma unroll
+            for (int i = 0; i < n[0]; ++i) lds_add(&o[i + WX * (j + WY * k)], q * w[0][i] * w[1][j] * w[2][k]);
+}
+
+template <int KIND, int COMP>
+__device__ __forceinline__ bool b64_node(const double *__restrict__ win, int x, int y, int z, double &v) {
+    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP;
+    constexpr int LX = -tc_nl(M, 0), LY = -tc_nl(M, 1), LZ = -tc_nl(M, 2);
+    constexpr int WX = tc_w(M, G, 0), WY = tc_w(M, G, 1), WZ = tc_w(M, G, 2);
+    x -= LX;
+    y -= LY;
+    z -= LZ;
+    if (x < 0 || x >= WX || y < 0 || y >= WY || z < 0 || z >= WZ) return false;
+    v = win[b64_off<KIND, COMP>() + x + WX * (y + WY * z)];
+    return v != 0.0;
+}
+
+template <int KIND>
+__global__ __launch_bounds__(256) void deposit_brick64_kernel(Dep64Args A, BrickIndex V) {
+    constexpr int C = KindC<KIND>::C, LO = KindC<KIND>::LO, E = BRK + 1 - LO;
+    __shared__ double win[b64_size<KIND>()];
+    BrickRange r;
+    if (!brick_range<B64_MERGE>(V, blockIdx.x, r)) return;
+    for (int i = threadIdx.x; i < b64_size<KIND>(); i += 256) win[i] = 0.0;
+    __syncthreads();
+    const int N = A.N;
+    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += 256) {
+        const int p = V.list[j];
+        int c[3];
+        brick_decode(A.s.cell[p], N, V.lgN, c[0], c[1], c[2]);
+        const int o[3] = {r.ox, r.oy, r.oz};
+        B64Particle P;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            P.l[d] = c[d] - o[d];
+            const double t = A.s.pos[d][p] * (double)N;
+            const double u = t - floor(t);
+            P.vw[d][0] = 1.0 - u;
+            P.vw[d][1] = u;
+            const double s = u - 0.5;
+            if (s < 0) {
+                P.llo[d] = -1;
+                P.lw[d][0] = -s;
+                P.lw[d][1] = 1.0 - P.lw[d][0];
+            } else {
+                P.llo[d] = 0;
+                P.lw[d][1] = s;
+                P.lw[d][0] = 1.0 - P.lw[d][1];
+            }
+        }
+        const double m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
+        if constexpr (KIND == 0) {
+            b64_add<KIND, 0>(win, P, m);
+        } else {
+            const double v[3] = {A.s.vel[0][p], A.s.vel[1][p], A.s.vel[2][p]};
+            if constexpr (C == 3) {
+                b64_add<KIND, 0>(win, P, m * v[0]);
+                b64_add<KIND, 1>(win, P, m * v[1]);
+                b64_add<KIND, 2>(win, P, m * v[2]);
+            } else {
+                b64_add<KIND, 0>(win, P, m * v[0] * v[0]);
+                b64_add<KIND, 1>(win, P, m * v[0] * v[1]);
+                b64_add<KIND, 2>(win, P, m * v[0] * v[2]);
+                b64_add<KIND, 3>(win, P, m * v[1] * v[1]);
+                b64_add<KIND, 4>(win, P, m * v[1] * v[2]);
+                b64_add<KIND, 5>(win, P, m * v[2] * v[2]);
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < E * E * E * C; i += 256) {
+        const int c = i % C, n = i / C;
+        const int x = n % E + LO, y = (n / E) % E + LO, z = n / (E * E) + LO;
+        double v = 0.0;
+        bool any;
+        if constexpr (C == 1) any = b64_node<KIND, 0>(win, x, y, z, v);
+        else {
+            any = c == 0   ? b64_node<KIND, 0>(win, x, y, z, v)
+                  : c == 1 ? b64_node<KIND, 1>(win, x, y, z, v)
+                           : (c == 2 ? b64_node<KIND, 2>(win, x, y, z, v) : false);
+            if constexpr (C == 6)
+                if (c >= 3)
+                    any = c == 3   ? b64_node<KIND, 3>(win, x, y, z, v)
+                          : c == 4 ? b64_node<KIND, 4>(win, x, y, z, v)
+                                   : b64_node<KIND, 5>(win, x, y, z, v);
+        }
+        if (!any) continue;
+        int gx = r.ox + x, gy = r.oy + y, gz = r.oz + z;
+        if (A.tgt == LF2MI_DEP_PERIODIC) {
+            gx = wrapi(gx, N);
+            gy = wrapi(gy, N);
+            gz = wrapi(gz, N);
+        }
+        atomicAdd(&A.field[site_index(N, A.h, gx, gy, gz) * C + c], v);
+    }
+}
+
 struct Gkd64Args {
     Soa64 s;
     int64_t np;
@@ -2648,40 +2795,25 @@ struct Gkd64Args {
     const double *phi;
     double dt_kick, dt_drift;
     unsigned long long *vmax2;  // bits of max |v|^2 (non-negative double)
+    int drift;                  // 0: a kick only, positions and cells stay
+    int *count, *rank;          // brick index: counts of the new bricks and places (null: not kept)
 };
 
-__global__ void gkd_f64_kernel(Gkd64Args A) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= A.np) return;
+// kick with the gathered acceleration, drift and wrap (LATfield2_Particles.hpp:2028-2032);
+// returns the new cell
+__device__ __forceinline__ int kick_drift64(const Gkd64Args &A, int64_t p, int cell, const double a[3], double &v2) {
     const int N = A.N;
-    int c[3];
-    double u[3];
-    for (int d = 0; d < 3; ++d) {
-        const double t = A.s.pos[d][p] * (double)N;
-        c[d] = (int)floor(t) % N;
-        u[d] = t - (double)(int)floor(t);
-    }
-    const double hn = 0.5 * N;
-    double a[3] = {0.0, 0.0, 0.0};
-    if (A.phi)
-    for (int k = 0; k < 2; ++k)
-        for (int j = 0; j < 2; ++j)
-            for (int i = 0; i < 2; ++i) {
-                const double w = (i ? u[0] : 1.0 - u[0]) * (j ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
-                const int x = c[0] + i, y = c[1] + j, z = c[2] + k;
-                auto P = [&](int xx, int yy, int zz) {
-                    return A.phi[site_index(N, A.h, wrapi(xx, N), wrapi(yy, N), wrapi(zz, N))];
-                };
-                a[0] += w * (-(P(x + 1, y, z) - P(x - 1, y, z)) * hn);
-                a[1] += w * (-(P(x, y + 1, z) - P(x, y - 1, z)) * hn);
-                a[2] += w * (-(P(x, y, z + 1) - P(x, y, z - 1)) * hn);
-            }
-    double v2 = 0.0;
     int cn[3];
+    v2 = 0.0;
+#pragma unroll
     for (int d = 0; d < 3; ++d) {
-        const double v = add_rn(A.s.vel[d][p], mul_rn(A.dt_kick, a[d]));
-        A.s.vel[d][p] = v;
+        double v = A.s.vel[d][p];
+        if (A.phi) {
+            v = add_rn(v, mul_rn(A.dt_kick, a[d]));
+            A.s.vel[d][p] = v;
+        }
         v2 += v * v;
+        if (!A.drift) continue;
         double x = add_rn(A.s.pos[d][p], mul_rn(A.dt_drift, v));
         if (x < 0.0) x = add_rn(x, 1.0);
         if (x >= 1.0) x = sub_rn(x, 1.0);
@@ -2690,8 +2822,129 @@ __global__ void gkd_f64_kernel(Gkd64Args A) {
         A.s.pos[d][p] = x;
         cn[d] = (int)floor(x * (double)N) % N;
     }
-    A.s.cell[p] = cn[0] + N * (cn[1] + N * cn[2]);
-    if (A.vmax2) atomicMax(A.vmax2, (unsigned long long)__double_as_longlong(v2));
+    if (!A.drift) return cell;
+    const int nc = cn[0] + N * (cn[1] + N * cn[2]);
+    A.s.cell[p] = nc;
+    return nc;
+}
+
+// largest |v|^2 of the workgroup into vmax2, one atomic (256 threads)
+__device__ __forceinline__ void vmax64(const Gkd64Args &A, double v2) {
+    __shared__ double wm[4];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v2 = fmax(v2, __shfl_xor(v2, o));
+    if (lane_id() == 0) wm[threadIdx.x >> 6] = v2;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(A.vmax2, (unsigned long long)__double_as_longlong(fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]))));
+}
+
+// place in the new brick's list, for the index that follows (every lane of the wave calls it)
+__device__ __forceinline__ void rank64(const Gkd64Args &A, const BrickIndex &V, int64_t p, int cell, bool act) {
+    int x = 0, y = 0, z = 0;
+    if (act) brick_decode(cell, A.N, V.lgN, x, y, z);
+    const int k = brick_rank(A.count, brick_of(x, y, z, V.NB), act);
+    if (act) A.rank[p] = k;
+}
+
+// one workgroup per group of items of a brick: the brick's window of phi, then its force
+// nodes (the differences of gkd_f64_kernel, each formed once per node instead of once per
+// particle and corner), both in LDS
+static constexpr int G64_MERGE = 4;
+__global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickIndex V) {
+    constexpr int PW = BRK + 3, FW = BRK + 1;
+    __shared__ double phw[PW * PW * PW];
+    __shared__ double frc[3][FW * FW * FW];
+    BrickRange r;
+    if (!brick_range<G64_MERGE>(V, blockIdx.x, r)) return;
+    const int N = A.N;
+    for (int i = threadIdx.x; i < PW * PW * PW; i += 256)
+        phw[i] = A.phi[site_index(N, A.h, wrapi(r.ox - 1 + i % PW, N), wrapi(r.oy - 1 + (i / PW) % PW, N),
+                                  wrapi(r.oz - 1 + i / (PW * PW), N))];
+    __syncthreads();
+    const double hn = 0.5 * N;
+    for (int i = threadIdx.x; i < FW * FW * FW; i += 256) {
+        const int c = i % FW + 1 + PW * ((i / FW) % FW + 1 + PW * (i / (FW * FW) + 1));
+        frc[0][i] = -(phw[c + 1] - phw[c - 1]) * hn;
+        frc[1][i] = -(phw[c + PW] - phw[c - PW]) * hn;
+        frc[2][i] = -(phw[c + PW * PW] - phw[c - PW * PW]) * hn;
+    }
+    __syncthreads();
+    double vmax = 0.0;
+    for (int j0 = r.p0; j0 < r.p1; j0 += 256) {
+        const int j = j0 + (int)threadIdx.x;
+        const bool act = j < r.p1;
+        int p = 0, cell = 0;
+        if (act) {
+            p = V.list[j];
+            cell = A.s.cell[p];
+            int c[3];
+            brick_decode(cell, N, V.lgN, c[0], c[1], c[2]);
+            double u[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const double t = A.s.pos[d][p] * (double)N;
+                u[d] = t - (double)(int)floor(t);
+            }
+            const double *f = &frc[0][c[0] - r.ox + FW * (c[1] - r.oy + FW * (c[2] - r.oz))];
+            double a[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const double w = (i ? u[0] : 1.0 - u[0]) * (jj ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
+                        const int n = i + FW * (jj + FW * k);
+                        a[0] += w * f[n];
+                        a[1] += w * f[n + FW * FW * FW];
+                        a[2] += w * f[n + 2 * FW * FW * FW];
+                    }
+            double v2;
+            cell = kick_drift64(A, p, cell, a, v2);
+            vmax = fmax(vmax, v2);
+        }
+        if (A.drift) rank64(A, V, p, cell, act);
+    }
+    if (A.vmax2) vmax64(A, vmax);
+}
+
+// particle by particle, phi straight from HBM; also the drift without a potential
+__global__ __launch_bounds__(256) void gkd_f64_kernel(Gkd64Args A, BrickIndex V) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool act = p < A.np;
+    const int N = A.N;
+    int cell = 0;
+    double v2 = 0.0;
+    if (act) {
+        double a[3] = {0.0, 0.0, 0.0};
+        if (A.phi) {
+            int c[3];
+            double u[3];
+            for (int d = 0; d < 3; ++d) {
+                const double t = A.s.pos[d][p] * (double)N;
+                c[d] = (int)floor(t) % N;
+                u[d] = t - (double)(int)floor(t);
+            }
+            const double hn = 0.5 * N;
+            for (int k = 0; k < 2; ++k)
+                for (int j = 0; j < 2; ++j)
+                    for (int i = 0; i < 2; ++i) {
+                        const double w = (i ? u[0] : 1.0 - u[0]) * (j ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
+                        const int x = c[0] + i, y = c[1] + j, z = c[2] + k;
+                        auto P = [&](int xx, int yy, int zz) {
+                            return A.phi[site_index(N, A.h, wrapi(xx, N), wrapi(yy, N), wrapi(zz, N))];
+                        };
+                        a[0] += w * (-(P(x + 1, y, z) - P(x - 1, y, z)) * hn);
+                        a[1] += w * (-(P(x, y + 1, z) - P(x, y - 1, z)) * hn);
+                        a[2] += w * (-(P(x, y, z + 1) - P(x, y, z - 1)) * hn);
+                    }
+        }
+        if (!A.drift) cell = A.s.cell[p];
+        cell = kick_drift64(A, p, cell, a, v2);
+    }
+    if (A.drift && A.count) rank64(A, V, p, cell, act);
+    if (A.vmax2) vmax64(A, v2);
 }
 
 // ---------------------------------------------------------------- download / counts
@@ -2904,6 +3157,9 @@ struct lf2mi_parts_s {
     int *ndgroup;  // [number of entries, unused]
     int *ditems;   // work list of the item kernel after deposit_tiles_c_kernel (items of dense bricks)
     int *nditem;   // [number of entries, unused]
+    lf2mi::BrickBuild bb;  // brick index of an F64 container
+    int bricks;            // 1: kept (the lattice has a number of bricks that the scans serve)
+    int in_box;            // 1: every F64 position is in [0, 1) (a kick then leaves them alone)
     unsigned long long *fx;
     int64_t fx_n;
     void *shell;          // shell and seam buffers of the tiles deposit kernel (grown on demand)
@@ -2941,6 +3197,16 @@ static int fill_int(int *ptr, int64_t n, int v, hipStream_t st) {
     fill_int_kernel<<<(unsigned)std::min<int64_t>(grid1(n), 65536), 256, 0, st>>>(ptr, n, v);
     LF2MI_LAUNCHED();
     return LF2MI_OK;
+}
+
+static int64_t b64_bricks(int N) {
+    const int64_t nb = (N + BRK - 1) / BRK;
+    return nb * nb * nb;
+}
+// whether the F64 container's brick index is kept for its particles
+static bool b64_used(const lf2mi_parts_s *p) { return p->bricks && p->np >= B64_OCC * b64_bricks(p->N); }
+static int b64_index(lf2mi_parts_s *p, hipStream_t st) {
+    return b64_used(p) ? brick_build(p->b64.cell, p->np, p->N, p->bb, st) : LF2MI_OK;
 }
 
 // exclusive scans of bcount -> bstart, items -> istart
@@ -3157,8 +3423,10 @@ static int ic_common(lf2mi_parts_s *p, IcArgs &A, hipStream_t st) {
         LF2MI_LAUNCHED();
         if (p->plw && A.np > 0)
             LF2MI_HIP(hipMemsetAsync(p->b64.pl, 0, (size_t)A.np * p->plw * sizeof(unsigned long long), st));
-        LF2MI_HIP(hipStreamSynchronize(st));
         p->np = A.np;
+        p->in_box = 1;
+        if (int rc = b64_index(p, st)) return rc;
+        LF2MI_HIP(hipStreamSynchronize(st));
     }
     // synthetic particles: per-particle masses (when kept) are 1
     p->total_mass = (p->mass_src ? 1.0 : p->mass_global) * (double)p->np;
@@ -3320,6 +3588,18 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
         if (flags & LF2MI_PARTS_MASS) A((void **)&s.mass, cap * sizeof(double));
         if (flags & LF2MI_PARTS_ID) A((void **)&s.id, cap * sizeof(int64_t));
         A((void **)&p->vmax_f64, sizeof(unsigned long long));
+        // the windows need distinct images of a brick's nodes, the scans at most 4096 blocks
+        const int64_t nbk = b64_bricks(N);
+        p->bricks = N >= 16 && brick_blocks(nbk) <= 4096;
+        if (p->bricks) {
+            A((void **)&p->bb.start, (size_t)(nbk + 1) * sizeof(int));
+            A((void **)&p->bb.istart, (size_t)(nbk + 1) * sizeof(int));
+            A((void **)&p->bb.count, (size_t)nbk * sizeof(int));
+            A((void **)&p->bb.bsum, 2 * (size_t)brick_blocks(nbk) * sizeof(int));
+            A((void **)&p->bb.item, (size_t)brick_items(nbk, (int64_t)cap) * sizeof(int));
+            A((void **)&p->bb.list, cap * sizeof(int));
+            A((void **)&p->bb.rank, cap * sizeof(int));
+        }
     }
     A((void **)&p->red, (size_t)(RED_BLOCKS + 1) * RED_Q * sizeof(double));
     if (rc) {
@@ -3330,6 +3610,8 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
     if (dtype == LF2MI_F32) {
         hipMemset(p->bstart, 0, ((size_t)p->g.nbk + 1) * sizeof(int));
         hipMemset(p->istart, 0, ((size_t)p->g.nbk + 1) * sizeof(int));
+    } else if (p->bricks) {
+        hipMemset(p->bb.count, 0, (size_t)b64_bricks(N) * sizeof(int));
     }
     *out = p;
     return LF2MI_OK;
@@ -3376,10 +3658,13 @@ static int upload_impl(lf2mi_parts p, int64_t np, const double *pos, const doubl
     // so the device arrays hold only valid particles
     std::vector<int64_t> keep;
     keep.reserve((size_t)np);
+    int in_box = 1;
     for (int64_t i = 0; i < np; ++i) {
         bool ok = true;
-        for (int d = 0; d < 3; ++d)
+        for (int d = 0; d < 3; ++d) {
             if ((int)floor(pos[3 * i + d] * (double)p->N) % p->N < 0) ok = false;
+            if (!(pos[3 * i + d] >= 0.0 && pos[3 * i + d] < 1.0)) in_box = 0;
+        }
         if (ok) keep.push_back(i);
     }
     const int64_t nk = (int64_t)keep.size();
@@ -3440,8 +3725,10 @@ static int upload_impl(lf2mi_parts p, int64_t np, const double *pos, const doubl
                                       hipSuccess)
                     rc = hip_fail(e, "payload", __FILE__, __LINE__);
             }
+            p->np = rc ? 0 : nk;
+            p->in_box = in_box;
+            if (!rc) rc = b64_index(p, st);
             if (!rc && (e = hipStreamSynchronize(st)) != hipSuccess) rc = hip_fail(e, "sync", __FILE__, __LINE__);
-            p->np = nk;
         }
     }
     hipStreamSynchronize(st);
@@ -3897,6 +4184,19 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
         static const char *const names64[5] = {"deposit_f64_scalar", "deposit_f64_vector", "deposit_f64_vecvec",
                                                "deposit_f64_vector_ngp", "deposit_f64_symtensor_ngp"};
         LF2MI_PROF(names64[kind], st);
+        if (b64_used(p)) {
+            const BrickIndex V = brick_view(p->bb, N);
+            const unsigned gb = (unsigned)brick_items(V.nbk, p->np);
+            switch (kind) {
+                case 0: deposit_brick64_kernel<0><<<gb, 256, 0, st>>>(A, V); break;
+                case 1: deposit_brick64_kernel<1><<<gb, 256, 0, st>>>(A, V); break;
+                case 2: deposit_brick64_kernel<2><<<gb, 256, 0, st>>>(A, V); break;
+                case 3: deposit_brick64_kernel<3><<<gb, 256, 0, st>>>(A, V); break;
+                default: deposit_brick64_kernel<4><<<gb, 256, 0, st>>>(A, V); break;
+            }
+            LF2MI_LAUNCHED();
+            return LF2MI_OK;
+        }
         switch (kind) {
             case 0: deposit_f64_kernel<0><<<g, 256, 0, st>>>(A); break;
             case 1: deposit_f64_kernel<1><<<g, 256, 0, st>>>(A); break;
@@ -4062,10 +4362,28 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
         A.dt_kick = dt_kick;
         A.dt_drift = dt_drift;
         A.vmax2 = vmax2 ? p->vmax_f64 : nullptr;
+        // a kick alone leaves positions and cells as they are (in_box: none is due a wrap)
+        A.drift = dt_drift != 0.0 || !p->in_box;
+        const bool bricks = b64_used(p);
+        if (bricks) {
+            A.count = p->bb.count;
+            A.rank = p->bb.rank;
+        }
+        const BrickIndex V = brick_view(p->bb, p->N);
         if (vmax2) LF2MI_HIP(hipMemsetAsync(p->vmax_f64, 0, sizeof(unsigned long long), st));
-        LF2MI_PROF("gkd_f64", st);
-        gkd_f64_kernel<<<grid1(p->np), 256, 0, st>>>(A);
-        LF2MI_LAUNCHED();
+        {
+            LF2MI_PROF("gkd_f64", st);
+            if (bricks && phi) gkd_brick64_kernel<<<(unsigned)brick_items(V.nbk, p->np), 256, 0, st>>>(A, V);
+            else gkd_f64_kernel<<<grid1(p->np), 256, 0, st>>>(A, V);
+            LF2MI_LAUNCHED();
+        }
+        if (A.drift) {
+            p->in_box = 1;
+            if (bricks) {
+                LF2MI_PROF("brick_index", st);
+                if (int rc = brick_build_ranked(p->b64.cell, p->np, p->N, p->bb, st)) return rc;
+            }
+        }
         if (vmax2) {
             unsigned long long bits = 0;
             LF2MI_HIP(hipMemcpyAsync(&bits, p->vmax_f64, sizeof(bits), hipMemcpyDeviceToHost, st));
