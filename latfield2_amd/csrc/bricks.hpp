@@ -7,10 +7,14 @@
 // (1500 G FP64 LDS atomics/s on random nodes, against 200 for FP32 ones), only the window's
 // nodes go to the field, in rows (100 G atomics/s).  The index costs 12 bytes per particle.
 //
-// Building it: the kernel that sets the cells counts them (brick_rank: the particle's place
-// among its brick's, one global atomic per brick and wave), one or two scan kernels turn the
-// counts into starts (and clear them for the next time), and brick_list_kernel writes each
-// particle's number at start + place.  Bricks at the upper faces are partial when 8 does not
+// Building it: brick_count_kernel counts the cells in particle order (brick_rank: the
+// particle's place among its brick's, one global atomic per brick and wave), one or two scan
+// kernels turn the counts into starts (and clear them for the next time), and
+// brick_list_kernel writes each particle's number at start + place.  Counted in particle order
+// a list consists of runs of consecutive particles, which the kernels that walk it read in
+// whole lines; places given by a kernel that walks the old lists break the runs up from step
+// to step (256^3 FP64 particles in brick order: the gather went from 0.73 to 1.3 ms in 400
+// steps).  Bricks at the upper faces are partial when 8 does not
 // divide N.
 #pragma once
 

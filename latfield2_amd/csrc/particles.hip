@@ -11,15 +11,17 @@
 // of the brick's nodes.  After a drift the container is re-bucketed with a counting sort
 // (histogram -> scan -> scatter into the second buffer).
 //
-// F64 representation (the plain path): absolute FP64 positions and velocities in upload
-// order, with a brick index beside them (bricks.hpp): deposits sum a brick's particles in an
-// FP64 LDS window, the gather reads a brick's window of phi.  Where few particles fall into a
-// brick both go particle by particle: FP64 atomics into the field, phi straight from HBM.
+// F64 representation (the plain path): absolute FP64 positions and velocities, put into brick
+// order at upload and every few drifts, with a brick index beside them (bricks.hpp): deposits
+// sum a brick's particles in an FP64 LDS window, the gather reads a brick's window of phi.
+// Where few particles fall into a brick both go particle by particle in upload order: FP64
+// atomics into the field, phi straight from HBM.  Downloads come in upload order either way.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "bricks.hpp"
@@ -239,36 +241,112 @@ struct Soa64 {
     unsigned long long *pl;  // payload, as in Soa32
 };
 
-__global__ void ic_f64_kernel(IcArgs A, Soa64 dst, int N) {
+// cell of an FP64 position (Particles::getPartCoord)
+__device__ __forceinline__ int cell64(const double p[3], int N) {
+    int c[3];
+    for (int d = 0; d < 3; ++d) c[d] = (int)floor(p[d] * (double)N) % N;
+    return c[0] + N * (c[1] + N * c[2]);
+}
+
+// Where the F64 container keeps a brick index its particles lie in brick order as they were
+// uploaded (place `start of the brick + rank` for each), so that the lists of later steps,
+// whose particles have moved little, still read memory nearly in order: with particles left
+// in lattice order a brick's list touches 64 8-particle runs per array, and after a few
+// hundred steps single particles of them (256^3 step: gather 1.1 -> 1.8 ms).  `slot` maps the
+// upload order to the place.  (256^3 step in brick order, lists in particle order: gather
+// 0.44 ms, 2.0 GB moved at 4.5 TB/s.)
+struct Order64 {
+    const int *start, *rank;  // null: upload order
+    int *slot;
+    int N, NB, lgN;
+};
+__device__ __forceinline__ int64_t order64(const Order64 &O, int64_t i, int cell) {
+    if (!O.start) return i;
+    int x, y, z;
+    brick_decode(cell, O.N, O.lgN, x, y, z);
+    const int j = O.start[brick_of(x, y, z, O.NB)] + O.rank[i];
+    O.slot[i] = j;
+    return j;
+}
+
+// One array (or one word of the payload: `stride` words per particle) into list order through
+// `tmp`, and back in place.  The container's pointers stay, so that a captured step can be
+// replayed any number of times.
+template <typename T>
+__global__ void reorder_gather_kernel(int64_t np, const T *__restrict__ src, int stride, const int *__restrict__ list,
+                                      T *__restrict__ tmp) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < np) tmp[j] = src[(int64_t)list[j] * stride];
+}
+template <typename T>
+__global__ void reorder_store_kernel(int64_t np, const T *__restrict__ tmp, T *__restrict__ dst, int stride) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < np) dst[j * stride] = tmp[j];
+}
+// the places after a reorder: inverse of the list, then the uploaded particles' places
+// through it (and the list becomes the identity)
+__global__ void reorder_inverse_kernel(int64_t np, const int *__restrict__ list, int *__restrict__ place) {
+    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < np) place[list[j]] = (int)j;
+}
+__global__ void reorder_slot_kernel(int64_t np, const int *__restrict__ place, int *__restrict__ slot,
+                                    int *__restrict__ list) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    slot[i] = place[slot[i]];
+    list[i] = (int)i;
+}
+
+// the cells of staged positions (pos: AoS) or, without them, of the synthetic particles
+__global__ void cells64_kernel(int64_t np, const double *__restrict__ pos, IcArgs A, int N, int *__restrict__ cell) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    double p[3], v[3];
+    if (pos) {
+        for (int d = 0; d < 3; ++d) p[d] = pos[3 * i + d];
+    } else {
+        ic_particle(A, i, p, v);
+    }
+    cell[i] = cell64(p, N);
+}
+
+__global__ void iota_kernel(int *__restrict__ p, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = (int)i;
+}
+
+__global__ void ic_f64_kernel(IcArgs A, Soa64 dst, int N, Order64 O) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= A.np) return;
     double p[3], v[3];
     ic_particle(A, i, p, v);
-    int c[3];
+    const int cell = cell64(p, N);
+    const int64_t j = order64(O, i, cell);
     for (int d = 0; d < 3; ++d) {
-        dst.pos[d][i] = p[d];
-        dst.vel[d][i] = v[d];
-        c[d] = (int)floor(p[d] * (double)N) % N;
+        dst.pos[d][j] = p[d];
+        dst.vel[d][j] = v[d];
     }
-    dst.cell[i] = c[0] + N * (c[1] + N * c[2]);
-    if (dst.mass) dst.mass[i] = 1.0;
-    if (dst.id) dst.id[i] = i;
+    dst.cell[j] = cell;
+    if (dst.mass) dst.mass[j] = 1.0;
+    if (dst.id) dst.id[j] = i;
 }
 
 __global__ void upload_f64_kernel(int64_t np, const double *__restrict__ pos, const double *__restrict__ vel,
-                                  const double *__restrict__ mass, const int64_t *__restrict__ id, Soa64 dst, int N) {
+                                  const double *__restrict__ mass, const int64_t *__restrict__ id,
+                                  const unsigned long long *__restrict__ pl, int plw, Soa64 dst, int N, Order64 O) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
-    int c[3];
+    const double p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+    const int cell = cell64(p, N);
+    const int64_t j = order64(O, i, cell);
     for (int d = 0; d < 3; ++d) {
-        const double p = pos[3 * i + d];
-        dst.pos[d][i] = p;
-        dst.vel[d][i] = vel[3 * i + d];
-        c[d] = (int)floor(p * (double)N) % N;
+        dst.pos[d][j] = p[d];
+        dst.vel[d][j] = vel[3 * i + d];
     }
-    dst.cell[i] = c[0] + N * (c[1] + N * c[2]);
-    if (dst.mass) dst.mass[i] = mass ? mass[i] : 1.0;
-    if (dst.id) dst.id[i] = id ? id[i] : i;
+    dst.cell[j] = cell;
+    if (dst.mass) dst.mass[j] = mass ? mass[i] : 1.0;
+    if (dst.id) dst.id[j] = id ? id[i] : i;
+    for (int w = 0; w < plw; ++w) dst.pl[j * plw + w] = pl[i * plw + w];
 }
 
 // ---------------------------------------------------------------- scans
@@ -2719,14 +2797,12 @@ __global__ __launch_bounds__(256) void deposit_brick64_kernel(Dep64Args A, Brick
     const int N = A.N;
     for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += 256) {
         const int p = V.list[j];
-        int c[3];
-        brick_decode(A.s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const int o[3] = {r.ox, r.oy, r.oz};
         B64Particle P;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            P.l[d] = c[d] - o[d];
             const double t = A.s.pos[d][p] * (double)N;
+            P.l[d] = (int)floor(t) % N - o[d];  // the cell as the index took it
             const double u = t - floor(t);
             P.vw[d][0] = 1.0 - u;
             P.vw[d][1] = u;
@@ -2796,25 +2872,24 @@ struct Gkd64Args {
     double dt_kick, dt_drift;
     unsigned long long *vmax2;  // bits of max |v|^2 (non-negative double)
     int drift;                  // 0: a kick only, positions and cells stay
-    int *count, *rank;          // brick index: counts of the new bricks and places (null: not kept)
 };
 
-// kick with the gathered acceleration, drift and wrap (LATfield2_Particles.hpp:2028-2032);
-// returns the new cell
-__device__ __forceinline__ int kick_drift64(const Gkd64Args &A, int64_t p, int cell, const double a[3], double &v2) {
+// kick with the gathered acceleration, drift and wrap (LATfield2_Particles.hpp:2028-2032)
+__device__ __forceinline__ void kick_drift64(const Gkd64Args &A, int64_t p, const double xin[3], const double vin[3],
+                                             const double a[3], double &v2) {
     const int N = A.N;
     int cn[3];
     v2 = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        double v = A.s.vel[d][p];
+        double v = vin[d];
         if (A.phi) {
             v = add_rn(v, mul_rn(A.dt_kick, a[d]));
             A.s.vel[d][p] = v;
         }
         v2 += v * v;
         if (!A.drift) continue;
-        double x = add_rn(A.s.pos[d][p], mul_rn(A.dt_drift, v));
+        double x = add_rn(xin[d], mul_rn(A.dt_drift, v));
         if (x < 0.0) x = add_rn(x, 1.0);
         if (x >= 1.0) x = sub_rn(x, 1.0);
         // beyond the reference's range (|dt v| >= box) wrap fully so the cell stays valid
@@ -2822,10 +2897,7 @@ __device__ __forceinline__ int kick_drift64(const Gkd64Args &A, int64_t p, int c
         A.s.pos[d][p] = x;
         cn[d] = (int)floor(x * (double)N) % N;
     }
-    if (!A.drift) return cell;
-    const int nc = cn[0] + N * (cn[1] + N * cn[2]);
-    A.s.cell[p] = nc;
-    return nc;
+    if (A.drift) A.s.cell[p] = cn[0] + N * (cn[1] + N * cn[2]);
 }
 
 // largest |v|^2 of the workgroup into vmax2, one atomic (256 threads)
@@ -2839,28 +2911,54 @@ __device__ __forceinline__ void vmax64(const Gkd64Args &A, double v2) {
         atomicMax(A.vmax2, (unsigned long long)__double_as_longlong(fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]))));
 }
 
-// place in the new brick's list, for the index that follows (every lane of the wave calls it)
-__device__ __forceinline__ void rank64(const Gkd64Args &A, const BrickIndex &V, int64_t p, int cell, bool act) {
-    int x = 0, y = 0, z = 0;
-    if (act) brick_decode(cell, A.N, V.lgN, x, y, z);
-    const int k = brick_rank(A.count, brick_of(x, y, z, V.NB), act);
-    if (act) A.rank[p] = k;
-}
-
 // one workgroup per group of items of a brick: the brick's window of phi, then its force
 // nodes (the differences of gkd_f64_kernel, each formed once per node instead of once per
 // particle and corner), both in LDS
 static constexpr int G64_MERGE = 4;
+static constexpr int G64_PER = 2;  // particles per thread and round, their loads issued together
 __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickIndex V) {
-    constexpr int PW = BRK + 3, FW = BRK + 1;
+    constexpr int PW = BRK + 3, FW = BRK + 1, RP = 256 * G64_PER;
     __shared__ double phw[PW * PW * PW];
     __shared__ double frc[3][FW * FW * FW];
     BrickRange r;
     if (!brick_range<G64_MERGE>(V, blockIdx.x, r)) return;
     const int N = A.N;
-    for (int i = threadIdx.x; i < PW * PW * PW; i += 256)
-        phw[i] = A.phi[site_index(N, A.h, wrapi(r.ox - 1 + i % PW, N), wrapi(r.oy - 1 + (i / PW) % PW, N),
-                                  wrapi(r.oz - 1 + i / (PW * PW), N))];
+    int p[G64_PER];
+    double x[G64_PER][3], vin[G64_PER][3];
+    auto fetch = [&](int j0) {
+#pragma unroll
+        for (int k = 0; k < G64_PER; ++k) {
+            const int j = j0 + (int)threadIdx.x + 256 * k;
+            p[k] = j < r.p1 ? V.list[j] : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < G64_PER; ++k)
+            if (p[k] >= 0) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    x[k][d] = A.s.pos[d][p[k]];
+                    vin[k][d] = A.s.vel[d][p[k]];
+                }
+            }
+    };
+    // the first round's particles in flight while the window loads
+    fetch(r.p0);
+    {
+        constexpr int WK = (PW * PW * PW + 255) / 256;
+        double w[WK];
+#pragma unroll
+        for (int k = 0; k < WK; ++k) {
+            const int i = threadIdx.x + 256 * k;
+            if (i < PW * PW * PW)
+                w[k] = A.phi[site_index(N, A.h, wrapi(r.ox - 1 + i % PW, N), wrapi(r.oy - 1 + (i / PW) % PW, N),
+                                        wrapi(r.oz - 1 + i / (PW * PW), N))];
+        }
+#pragma unroll
+        for (int k = 0; k < WK; ++k) {
+            const int i = threadIdx.x + 256 * k;
+            if (i < PW * PW * PW) phw[i] = w[k];
+        }
+    }
     __syncthreads();
     const double hn = 0.5 * N;
     for (int i = threadIdx.x; i < FW * FW * FW; i += 256) {
@@ -2871,19 +2969,18 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
     }
     __syncthreads();
     double vmax = 0.0;
-    for (int j0 = r.p0; j0 < r.p1; j0 += 256) {
-        const int j = j0 + (int)threadIdx.x;
-        const bool act = j < r.p1;
-        int p = 0, cell = 0;
-        if (act) {
-            p = V.list[j];
-            cell = A.s.cell[p];
+    for (int j0 = r.p0; j0 < r.p1; j0 += RP) {
+        if (j0 != r.p0) fetch(j0);
+#pragma unroll
+        for (int q = 0; q < G64_PER; ++q) {
+            if (p[q] < 0) continue;
             int c[3];
-            brick_decode(cell, N, V.lgN, c[0], c[1], c[2]);
             double u[3];
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
-                const double t = A.s.pos[d][p] * (double)N;
+                // the cell as the index took it (same expression on the same position)
+                const double t = x[q][d] * (double)N;
+                c[d] = (int)floor(t) % N;
                 u[d] = t - (double)(int)floor(t);
             }
             const double *f = &frc[0][c[0] - r.ox + FW * (c[1] - r.oy + FW * (c[2] - r.oz))];
@@ -2891,38 +2988,40 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
 #pragma unroll
             for (int k = 0; k < 2; ++k)
 #pragma unroll
-                for (int jj = 0; jj < 2; ++jj)
+                for (int j = 0; j < 2; ++j)
 #pragma unroll
                     for (int i = 0; i < 2; ++i) {
-                        const double w = (i ? u[0] : 1.0 - u[0]) * (jj ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
-                        const int n = i + FW * (jj + FW * k);
+                        const double w = (i ? u[0] : 1.0 - u[0]) * (j ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
+                        const int n = i + FW * (j + FW * k);
                         a[0] += w * f[n];
                         a[1] += w * f[n + FW * FW * FW];
                         a[2] += w * f[n + 2 * FW * FW * FW];
                     }
             double v2;
-            cell = kick_drift64(A, p, cell, a, v2);
+            kick_drift64(A, p[q], x[q], vin[q], a, v2);
             vmax = fmax(vmax, v2);
         }
-        if (A.drift) rank64(A, V, p, cell, act);
     }
     if (A.vmax2) vmax64(A, vmax);
 }
 
 // particle by particle, phi straight from HBM; also the drift without a potential
-__global__ __launch_bounds__(256) void gkd_f64_kernel(Gkd64Args A, BrickIndex V) {
+__global__ __launch_bounds__(256) void gkd_f64_kernel(Gkd64Args A) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool act = p < A.np;
     const int N = A.N;
-    int cell = 0;
     double v2 = 0.0;
     if (act) {
-        double a[3] = {0.0, 0.0, 0.0};
+        double a[3] = {0.0, 0.0, 0.0}, x[3], vin[3];
+        for (int d = 0; d < 3; ++d) {
+            x[d] = A.s.pos[d][p];
+            vin[d] = A.s.vel[d][p];
+        }
         if (A.phi) {
             int c[3];
             double u[3];
             for (int d = 0; d < 3; ++d) {
-                const double t = A.s.pos[d][p] * (double)N;
+                const double t = x[d] * (double)N;
                 c[d] = (int)floor(t) % N;
                 u[d] = t - (double)(int)floor(t);
             }
@@ -2931,19 +3030,17 @@ __global__ __launch_bounds__(256) void gkd_f64_kernel(Gkd64Args A, BrickIndex V)
                 for (int j = 0; j < 2; ++j)
                     for (int i = 0; i < 2; ++i) {
                         const double w = (i ? u[0] : 1.0 - u[0]) * (j ? u[1] : 1.0 - u[1]) * (k ? u[2] : 1.0 - u[2]);
-                        const int x = c[0] + i, y = c[1] + j, z = c[2] + k;
+                        const int nx = c[0] + i, ny = c[1] + j, nz = c[2] + k;
                         auto P = [&](int xx, int yy, int zz) {
                             return A.phi[site_index(N, A.h, wrapi(xx, N), wrapi(yy, N), wrapi(zz, N))];
                         };
-                        a[0] += w * (-(P(x + 1, y, z) - P(x - 1, y, z)) * hn);
-                        a[1] += w * (-(P(x, y + 1, z) - P(x, y - 1, z)) * hn);
-                        a[2] += w * (-(P(x, y, z + 1) - P(x, y, z - 1)) * hn);
+                        a[0] += w * (-(P(nx + 1, ny, nz) - P(nx - 1, ny, nz)) * hn);
+                        a[1] += w * (-(P(nx, ny + 1, nz) - P(nx, ny - 1, nz)) * hn);
+                        a[2] += w * (-(P(nx, ny, nz + 1) - P(nx, ny, nz - 1)) * hn);
                     }
         }
-        if (!A.drift) cell = A.s.cell[p];
-        cell = kick_drift64(A, p, cell, a, v2);
+        kick_drift64(A, p, x, vin, a, v2);
     }
-    if (A.drift && A.count) rank64(A, V, p, cell, act);
     if (A.vmax2) vmax64(A, v2);
 }
 
@@ -2961,13 +3058,25 @@ __global__ void download_f32_kernel(int64_t np, Soa32 s, int N, double *__restri
     if (mass) mass[i] = s.mass ? (double)s.mass[i] : mass_global;
 }
 
-__global__ void download_f64_kernel(int64_t np, Soa64 s, double *__restrict__ pos, double *__restrict__ vel) {
+__global__ void download_f64_kernel(int64_t np, Soa64 s, const int *__restrict__ slot, double *__restrict__ pos,
+                                    double *__restrict__ vel) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
+    const int64_t j = slot ? slot[i] : i;
     for (int d = 0; d < 3; ++d) {
-        if (pos) pos[3 * i + d] = s.pos[d][i];
-        if (vel) vel[3 * i + d] = s.vel[d][i];
+        if (pos) pos[3 * i + d] = s.pos[d][j];
+        if (vel) vel[3 * i + d] = s.vel[d][j];
     }
+}
+
+// `words` values per particle into upload order
+template <typename T>
+__global__ void unsort_kernel(int64_t np, const T *__restrict__ src, int words, const int *__restrict__ slot,
+                              T *__restrict__ dst) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const int64_t j = slot[i];
+    for (int w = 0; w < words; ++w) dst[i * words + w] = src[j * words + w];
 }
 
 // particles whose cell lies in the box [lo, hi) per axis, compacted through a cursor
@@ -3059,6 +3168,7 @@ struct RedArgs {
     const double *vel64[3];
     const double *mass64;  // per-particle masses (F64 container) or null
     double mass;           // the global mass, when no per-particle one is used
+    const int *slot;       // F64: place of each uploaded particle (null: upload order)
     int nq;
     int q[RED_Q];
     int op[RED_Q];
@@ -3080,8 +3190,9 @@ __global__ __launch_bounds__(RED_WG) void parts_reduce_kernel(RedArgs A, double 
     for (int64_t i = (int64_t)blockIdx.x * RED_WG + threadIdx.x; i < A.np; i += stride) {
         double v[3], m;
         if (F64) {
-            for (int d = 0; d < 3; ++d) v[d] = A.vel64[d][i];
-            m = A.mass64 ? A.mass64[i] : A.mass;
+            const int64_t j = A.slot ? A.slot[i] : i;
+            for (int d = 0; d < 3; ++d) v[d] = A.vel64[d][j];
+            m = A.mass64 ? A.mass64[j] : A.mass;
         } else {
             for (int d = 0; d < 3; ++d) v[d] = (double)A.vel32[d][i];
             m = A.mass32 ? (double)A.mass32[i] : A.mass;
@@ -3159,6 +3270,10 @@ struct lf2mi_parts_s {
     int *nditem;   // [number of entries, unused]
     lf2mi::BrickBuild bb;  // brick index of an F64 container
     int bricks;            // 1: kept (the lattice has a number of bricks that the scans serve)
+    int *slot;             // F64: place of each uploaded particle
+    int sorted;            // 1: the places are in brick order (else upload order, slot unused)
+    void *tmp;             // F64: one 8-byte value per particle (reordering)
+    int moves;             // F64: drifts since the particles were last put into brick order
     int in_box;            // 1: every F64 position is in [0, 1) (a kick then leaves them alone)
     unsigned long long *fx;
     int64_t fx_n;
@@ -3205,8 +3320,74 @@ static int64_t b64_bricks(int N) {
 }
 // whether the F64 container's brick index is kept for its particles
 static bool b64_used(const lf2mi_parts_s *p) { return p->bricks && p->np >= B64_OCC * b64_bricks(p->N); }
-static int b64_index(lf2mi_parts_s *p, hipStream_t st) {
-    return b64_used(p) ? brick_build(p->b64.cell, p->np, p->N, p->bb, st) : LF2MI_OK;
+template <typename T> static int reorder_one(lf2mi_parts_s *p, T *a, int stride, hipStream_t st) {
+    const unsigned g = grid1(p->np);
+    reorder_gather_kernel<T><<<g, 256, 0, st>>>(p->np, a, stride, p->bb.list, (T *)p->tmp);
+    LF2MI_LAUNCHED();
+    reorder_store_kernel<T><<<g, 256, 0, st>>>(p->np, (const T *)p->tmp, a, stride);
+    LF2MI_LAUNCHED();
+    return LF2MI_OK;
+}
+
+// The index after a drift; every B64_REORDER drifts the particles are put into its order as
+// well.  A particle that has left the brick whose place it lies in costs whole lines for
+// single values: at 256^3 the gather slows from 0.45 to 0.9 ms over 400 steps without this;
+// a reorder takes 0.9 ms.
+static constexpr int B64_REORDER = 32;
+static int b64_moved(lf2mi_parts_s *p, hipStream_t st) {
+    Soa64 &s = p->b64;
+    if (int rc = brick_build(s.cell, p->np, p->N, p->bb, st)) return rc;
+    if (++p->moves < B64_REORDER) return LF2MI_OK;
+    p->moves = 0;
+    int rc = reorder_one(p, s.cell, 1, st);
+    for (int d = 0; d < 3 && !rc; ++d) {
+        rc = reorder_one(p, s.pos[d], 1, st);
+        if (!rc) rc = reorder_one(p, s.vel[d], 1, st);
+    }
+    if (!rc && s.mass) rc = reorder_one(p, s.mass, 1, st);
+    if (!rc && s.id) rc = reorder_one(p, s.id, 1, st);
+    for (int w = 0; w < p->plw && !rc; ++w) rc = reorder_one(p, s.pl + w, p->plw, st);
+    if (rc) return rc;
+    const unsigned g = grid1(p->np);
+    reorder_inverse_kernel<<<g, 256, 0, st>>>(p->np, p->bb.list, p->bb.rank);
+    LF2MI_LAUNCHED();
+    reorder_slot_kernel<<<g, 256, 0, st>>>(p->np, p->bb.rank, p->slot, p->bb.list);
+    LF2MI_LAUNCHED();
+    return LF2MI_OK;
+}
+
+// new contents of the F64 container (p->np particles): staged arrays (`pos` and the rest,
+// device) or, without `pos`, the synthetic particles of A; their brick order and index where
+// the container keeps one
+static int b64_fill(lf2mi_parts_s *p, const double *pos, const double *vel, const double *mass, const int64_t *id,
+                    const unsigned long long *pl, const IcArgs &A, hipStream_t st) {
+    const int N = p->N;
+    const unsigned g = grid1(p->np);
+    Order64 O{};
+    p->sorted = b64_used(p);
+    p->moves = 0;
+    if (p->sorted) {
+        const BrickIndex V = brick_view(p->bb, N);
+        cells64_kernel<<<g, 256, 0, st>>>(p->np, pos, A, N, p->bb.list);  // the list is written last
+        LF2MI_LAUNCHED();
+        brick_count_kernel<<<g, 256, 0, st>>>(p->np, p->bb.list, N, V.NB, V.lgN, p->bb.count, p->bb.rank);
+        LF2MI_LAUNCHED();
+        if (int rc = brick_scan(p->bb.count, V.nbk, p->bb.bsum, p->bb.start, p->bb.istart, p->bb.item, st)) return rc;
+        O.start = p->bb.start;
+        O.rank = p->bb.rank;
+        O.slot = p->slot;
+        O.N = N;
+        O.NB = V.NB;
+        O.lgN = V.lgN;
+    }
+    if (pos) upload_f64_kernel<<<g, 256, 0, st>>>(p->np, pos, vel, mass, id, pl, p->plw, p->b64, N, O);
+    else ic_f64_kernel<<<g, 256, 0, st>>>(A, p->b64, N, O);
+    LF2MI_LAUNCHED();
+    if (p->sorted) {
+        iota_kernel<<<g, 256, 0, st>>>(p->bb.list, p->np);
+        LF2MI_LAUNCHED();
+    }
+    return LF2MI_OK;
 }
 
 // exclusive scans of bcount -> bstart, items -> istart
@@ -3419,13 +3600,15 @@ static int ic_common(lf2mi_parts_s *p, IcArgs &A, hipStream_t st) {
         if (int rc = sort_into_other(p, src, A.np, st)) return rc;
         if (int rc = read_total(p, st, &p->np)) return rc;
     } else {
-        ic_f64_kernel<<<grid1(A.np), 256, 0, st>>>(A, p->b64, p->N);
-        LF2MI_LAUNCHED();
-        if (p->plw && A.np > 0)
-            LF2MI_HIP(hipMemsetAsync(p->b64.pl, 0, (size_t)A.np * p->plw * sizeof(unsigned long long), st));
         p->np = A.np;
         p->in_box = 1;
-        if (int rc = b64_index(p, st)) return rc;
+        if (A.np > 0)
+            if (int rc = b64_fill(p, nullptr, nullptr, nullptr, nullptr, nullptr, A, st)) {
+                p->np = 0;
+                return rc;
+            }
+        if (p->plw && A.np > 0)
+            LF2MI_HIP(hipMemsetAsync(p->b64.pl, 0, (size_t)A.np * p->plw * sizeof(unsigned long long), st));
         LF2MI_HIP(hipStreamSynchronize(st));
     }
     // synthetic particles: per-particle masses (when kept) are 1
@@ -3444,11 +3627,13 @@ namespace lf2mi {
 // run to run
 template <typename T>
 __global__ __launch_bounds__(RED_WG) void mass_partial_kernel(int64_t np, const T *__restrict__ mass,
+                                                              const int *__restrict__ slot,
                                                               double *__restrict__ partial) {
     __shared__ double lds[RED_WG];
     double m = 0.0;
     const int64_t stride = (int64_t)gridDim.x * RED_WG;
-    for (int64_t i = (int64_t)blockIdx.x * RED_WG + threadIdx.x; i < np; i += stride) m += (double)mass[i];
+    for (int64_t i = (int64_t)blockIdx.x * RED_WG + threadIdx.x; i < np; i += stride)
+        m += (double)mass[slot ? slot[i] : i];
     lds[threadIdx.x] = m;
     __syncthreads();
     for (int h = RED_WG / 2; h > 0; h >>= 1) {
@@ -3599,6 +3784,8 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
             A((void **)&p->bb.item, (size_t)brick_items(nbk, (int64_t)cap) * sizeof(int));
             A((void **)&p->bb.list, cap * sizeof(int));
             A((void **)&p->bb.rank, cap * sizeof(int));
+            A((void **)&p->slot, cap * sizeof(int));
+            A((void **)&p->tmp, cap * sizeof(double));
         }
     }
     A((void **)&p->red, (size_t)(RED_BLOCKS + 1) * RED_Q * sizeof(double));
@@ -3718,16 +3905,10 @@ static int upload_impl(lf2mi_parts p, int64_t np, const double *pos, const doubl
             if (!rc) rc = sort_into_other(p, src, nk, st);
             if (!rc) rc = read_total(p, st, &p->np);
         } else {
-            if (nk > 0) {
-                upload_f64_kernel<<<grid1(nk), 256, 0, st>>>(nk, dpos, dvel, dmass, did, p->b64, p->N);
-                if ((e = hipGetLastError()) != hipSuccess) rc = hip_fail(e, "upload_f64_kernel", __FILE__, __LINE__);
-                if (!rc && plb && (e = hipMemcpyAsync(p->b64.pl, dpl, plb * (size_t)nk, hipMemcpyDeviceToDevice, st)) !=
-                                      hipSuccess)
-                    rc = hip_fail(e, "payload", __FILE__, __LINE__);
-            }
-            p->np = rc ? 0 : nk;
+            p->np = nk;
             p->in_box = in_box;
-            if (!rc) rc = b64_index(p, st);
+            if (nk > 0) rc = b64_fill(p, dpos, dvel, dmass, did, dpl, IcArgs{}, st);
+            if (rc) p->np = 0;
             if (!rc && (e = hipStreamSynchronize(st)) != hipSuccess) rc = hip_fail(e, "sync", __FILE__, __LINE__);
         }
     }
@@ -3775,19 +3956,32 @@ int lf2mi_parts_download(lf2mi_parts p, double *pos, double *vel, double *mass, 
         if (e != hipSuccess) rc = hip_fail(e, "download", __FILE__, __LINE__);
     } else {
         const Soa64 &s = p->b64;
-        download_f64_kernel<<<grid1(np), 256, 0, st>>>(np, s, dpos, dvel);
+        const int *slot = p->sorted ? p->slot : nullptr;
+        download_f64_kernel<<<grid1(np), 256, 0, st>>>(np, s, slot, dpos, dvel);
         hipError_t e = hipGetLastError();
         if (e == hipSuccess && pos) e = hipMemcpyAsync(pos, dpos, np * 3 * sizeof(double), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess && vel) e = hipMemcpyAsync(vel, dvel, np * 3 * sizeof(double), hipMemcpyDeviceToHost, st);
+        // the other arrays go through dmass, which holds 8 bytes per particle, in upload order
+        auto out = [&](auto *host, const auto *dev) {
+            using T = std::remove_cv_t<std::remove_pointer_t<decltype(host)>>;
+            static_assert(sizeof(T) <= sizeof(double), "staged in dmass");
+            const T *from = dev;
+            if (slot) {
+                unsort_kernel<T><<<grid1(np), 256, 0, st>>>(np, dev, 1, slot, (T *)dmass);
+                if ((e = hipGetLastError()) != hipSuccess) return;
+                from = (const T *)dmass;
+            }
+            e = hipMemcpyAsync(host, from, np * sizeof(T), hipMemcpyDeviceToHost, st);
+        };
         if (e == hipSuccess && mass) {
-            if (s.mass && p->mass_src) e = hipMemcpyAsync(mass, s.mass, np * sizeof(double), hipMemcpyDeviceToHost, st);
+            if (s.mass && p->mass_src) out(mass, s.mass);
             else for (int64_t i = 0; i < np; ++i) mass[i] = p->mass_global;
         }
         if (e == hipSuccess && id) {
-            if (s.id) e = hipMemcpyAsync(id, s.id, np * sizeof(int64_t), hipMemcpyDeviceToHost, st);
+            if (s.id) out(id, s.id);
             else rc = fail(LF2MI_EINVAL, "container keeps no IDs");
         }
-        if (e == hipSuccess && cell) e = hipMemcpyAsync(cell, s.cell, np * sizeof(int32_t), hipMemcpyDeviceToHost, st);
+        if (e == hipSuccess && cell) out(cell, s.cell);
         if (e != hipSuccess) rc = hip_fail(e, "download", __FILE__, __LINE__);
     }
     hipStreamSynchronize(st);
@@ -3887,8 +4081,17 @@ int lf2mi_parts_download_aos(lf2mi_parts p, void *base, int64_t n_room, int64_t 
     unsigned char *b = static_cast<unsigned char *>(base);
     if (p->plw) {
         const unsigned long long *pl = p->dtype == LF2MI_F32 ? p->b32[p->cur].pl : p->b64.pl;
-        LF2MI_HIP(hipMemcpyAsync(b, pl, (size_t)np * p->plw * 8, hipMemcpyDeviceToHost, st));
-        LF2MI_HIP(hipStreamSynchronize(st));
+        unsigned long long *tmp = nullptr;
+        if (p->dtype == LF2MI_F64 && p->sorted) {
+            LF2MI_HIP(hipMalloc((void **)&tmp, (size_t)np * p->plw * 8));
+            unsort_kernel<unsigned long long><<<grid1(np), 256, 0, st>>>(np, pl, p->plw, p->slot, tmp);
+            pl = tmp;
+        }
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipMemcpyAsync(b, pl, (size_t)np * p->plw * 8, hipMemcpyDeviceToHost, st);
+        const hipError_t e2 = hipStreamSynchronize(st);
+        if (tmp) hipFree(tmp);
+        if (e != hipSuccess || e2 != hipSuccess) return hip_fail(e != hipSuccess ? e : e2, "payload", __FILE__, __LINE__);
     }
     for (int64_t i = 0; i < np; ++i) {
         unsigned char *q = b + i * stride;
@@ -3947,8 +4150,9 @@ int lf2mi_parts_mass_from(lf2mi_parts p, int where, int64_t offset, void *stream
         }
         LF2MI_LAUNCHED();
     }
-    if (p->dtype == LF2MI_F32) mass_partial_kernel<float><<<nb, RED_WG, 0, st>>>(p->np, p->b32[p->cur].mass, p->red);
-    else mass_partial_kernel<double><<<nb, RED_WG, 0, st>>>(p->np, p->b64.mass, p->red);
+    if (p->dtype == LF2MI_F32) mass_partial_kernel<float><<<nb, RED_WG, 0, st>>>(p->np, p->b32[p->cur].mass, nullptr, p->red);
+    else
+        mass_partial_kernel<double><<<nb, RED_WG, 0, st>>>(p->np, p->b64.mass, p->sorted ? p->slot : nullptr, p->red);
     LF2MI_LAUNCHED();
     mass_total_kernel<<<1, 1, 0, st>>>(p->red, nb, res);
     LF2MI_LAUNCHED();
@@ -4365,23 +4569,19 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
         // a kick alone leaves positions and cells as they are (in_box: none is due a wrap)
         A.drift = dt_drift != 0.0 || !p->in_box;
         const bool bricks = b64_used(p);
-        if (bricks) {
-            A.count = p->bb.count;
-            A.rank = p->bb.rank;
-        }
         const BrickIndex V = brick_view(p->bb, p->N);
         if (vmax2) LF2MI_HIP(hipMemsetAsync(p->vmax_f64, 0, sizeof(unsigned long long), st));
         {
             LF2MI_PROF("gkd_f64", st);
             if (bricks && phi) gkd_brick64_kernel<<<(unsigned)brick_items(V.nbk, p->np), 256, 0, st>>>(A, V);
-            else gkd_f64_kernel<<<grid1(p->np), 256, 0, st>>>(A, V);
+            else gkd_f64_kernel<<<grid1(p->np), 256, 0, st>>>(A);
             LF2MI_LAUNCHED();
         }
         if (A.drift) {
             p->in_box = 1;
             if (bricks) {
                 LF2MI_PROF("brick_index", st);
-                if (int rc = brick_build_ranked(p->b64.cell, p->np, p->N, p->bb, st)) return rc;
+                if (int rc = b64_moved(p, st)) return rc;
             }
         }
         if (vmax2) {
@@ -4477,6 +4677,7 @@ int lf2mi_parts_reduce(lf2mi_parts p, int n, const int *quantity, const int *red
     } else {
         for (int d = 0; d < 3; ++d) A.vel64[d] = p->b64.vel[d];
         A.mass64 = p->mass_src ? p->b64.mass : nullptr;
+        A.slot = p->sorted ? p->slot : nullptr;
         parts_reduce_kernel<true><<<nb, RED_WG, 0, st>>>(A, p->red);
     }
     LF2MI_LAUNCHED();

@@ -70,3 +70,52 @@ def test_f64_steps_and_projections_match_oracle(N, n):
     a = parts.reduce(q, [lf.SUM, lf.SUM, lf.MAX])
     assert a == parts.reduce(q, [lf.SUM, lf.SUM, lf.MAX])
     assert abs(a[1] - 0.5 * mass * np.sum(e["vel"] ** 2)) <= 1e-12 * a[1]
+
+
+def test_f64_reordering_keeps_structs_and_upload_order():
+    """more drifts than the container waits between two reorderings, with IDs, masses and a
+    payload: everything comes back in upload order, and a captured run of steps that holds a
+    reordering replays like eager steps"""
+    N, n, dt, mass = 16, 5003, 0.01, 1.0 / 5003
+    announce(f"F64 reorder N={N} n={n}")
+    rng = np.random.default_rng(3)
+    part = np.dtype([("ID", "<i8"), ("pos", "<f8", 3), ("vel", "<f8", 3), ("tag", "<f8")])
+    a = np.zeros(n, dtype=part)
+    a["ID"] = rng.permutation(n)
+    a["pos"] = rng.random((n, 3))
+    a["vel"] = 0.5 * rng.standard_normal((n, 3))
+    a["tag"] = rng.random(n)
+    lat = lf.Lattice(3, N, 1)
+
+    def fresh():
+        q = lf.Particles(N, n, lf.F64, ids=True, mass=mass)
+        q.set_payload(part.itemsize)
+        q.upload_structs(a)
+        f = lf.Field(lat, 1, lf.F64)
+        return q, f, lf.Field(lat, 1, lf.F64), lf.PlanFFT(f, None)
+
+    eager, rho, phi, plan = fresh()
+    for _ in range(70):
+        lf.pm_step(eager, plan, rho, phi, dt, dt)
+    e = eager.download_structs(part)
+    p, v = a["pos"].copy(), a["vel"].copy()
+    for _ in range(70):
+        orc.pm_step(p, v, N, dt, dt, mass_global=mass)
+    assert np.array_equal(e["ID"], a["ID"]) and np.array_equal(e["tag"], a["tag"])
+    off = np.abs(e["pos"] - p)
+    # 70 steps amplify the rounding of the sums' order; a wrong particle would be off by a cell
+    assert np.max(np.minimum(off, 1.0 - off)) <= 1e-6
+    captured, rho2, phi2, plan2 = fresh()
+    side = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(35):  # the 32nd reorders
+                lf.pm_step(captured, plan2, rho2, phi2, dt, dt)
+        for _ in range(2):
+            g.replay()
+            torch.cuda.synchronize()
+    c = captured.download_structs(part)
+    assert np.array_equal(c["ID"], a["ID"]) and np.array_equal(c["tag"], a["tag"])
+    off = np.abs(c["pos"] - p)
+    assert np.max(np.minimum(off, 1.0 - off)) <= 1e-6
