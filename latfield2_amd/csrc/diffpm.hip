@@ -16,8 +16,8 @@
 //                        phi-bar = sum_d D_d F-bar_d          (D_d is antisymmetric)
 //                        rho-bar = G phi-bar                  (G is symmetric: the same FFT solve)
 //                        lambda_x += q N grad_X interp(rho-bar)(X_p)   (deposit weights)
-// Particles keep their order (no bucketing) so gradients stay attached to them.  The
-// starting state of every step is checkpointed in HBM and the fields are recomputed
+// Particles keep their order so gradients stay attached to them; a brick index (bricks.hpp)
+// of the state at hand lets the deposits and gathers work brick by brick.  The starting state of every step is checkpointed in HBM and the fields are recomputed
 // on the way back.  Positions are kept as (cell, offset in cell units) and re-anchored
 // in FP64 after each drift, as in the PM step.  T = float or double selects the
 // precision of the whole path (fields, FFTs, offsets, velocities, adjoints).
@@ -25,6 +25,7 @@
 #include <cmath>
 #include <new>
 
+#include "bricks.hpp"
 #include "common.hpp"
 
 namespace lf2mi {
@@ -102,79 +103,113 @@ template <typename T, typename I> __global__ void dp_state_out_kernel(DpState<T>
     }
 }
 
-template <typename T> __global__ void dp_density_kernel(DpState<T> s, T *__restrict__ rho, T q) {
+// ---- brick windows (bricks.hpp): one workgroup per group of items of a brick
+static constexpr int DP_MERGE = 4;
+static constexpr int DP_FW = BRK + 1, DP_F3 = DP_FW * DP_FW * DP_FW;  // nodes [o, o + 8]
+static constexpr int DP_PW = BRK + 3, DP_P3 = DP_PW * DP_PW * DP_PW;  // nodes [o - 1, o + 9]
+
+// density: the brick's terms q w summed in an FP64 window, its nodes added to rho (128^3 FP32
+// particles in lattice order: 390 us with 8 global atomics per particle)
+template <typename T>
+__global__ __launch_bounds__(DP_WG) void dp_density_kernel(DpState<T> s, BrickIndex V, T *__restrict__ rho, T q) {
+    __shared__ double win[DP_F3];
+    BrickRange r;
+    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
     const int N = s.N;
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
+    for (int i = threadIdx.x; i < DP_F3; i += DP_WG) win[i] = 0.0;
+    __syncthreads();
+    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
+        const int p = V.list[j];
         int c[3];
-        decode(s.cell[p], N, c);
+        brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};
+        double *o = win + (c[0] - r.ox + DP_FW * (c[1] - r.oy + DP_FW * (c[2] - r.oz)));
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j2 = 0; j2 < 2; ++j2)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const T w = wsel(i, u[0]) * wsel(j, u[1]) * wsel(k, u[2]);
-                    atomicAdd(&rho[site_index(N, 1, wrapn(c[0] + i, N), wrapn(c[1] + j, N), wrapn(c[2] + k, N))], q * w);
-                }
+                for (int i = 0; i < 2; ++i)
+                    lds_add(&o[i + DP_FW * (j2 + DP_FW * k)], (double)(q * (wsel(i, u[0]) * wsel(j2, u[1]) * wsel(k, u[2]))));
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < DP_F3; i += DP_WG) {
+        const double w = win[i];
+        if (w == 0.0) continue;
+        const int x = r.ox + i % DP_FW, y = r.oy + (i / DP_FW) % DP_FW, z = r.oz + i / (DP_FW * DP_FW);
+        atomicAdd(&rho[site_index(N, 1, wrapn(x, N), wrapn(y, N), wrapn(z, N))], (T)w);
     }
 }
 
-// F = -D phi at the 8 corners of a cell from the 32 surrounding values: Fc[d][k][j][i]
+// the brick's window of phi into LDS (every load issued before the stores), then the force
+// F = -D phi on its nodes; barriers inside
 template <typename T>
-__device__ __forceinline__ void corner_forces(const T *__restrict__ phi, int N, const int c[3], T Fc[3][2][2][2]) {
-    int xs[4], ys[4], zs[4];
+__device__ __forceinline__ void brick_forces(const T *__restrict__ phi, int N, const BrickRange &r, T *__restrict__ phw,
+                                             T (*__restrict__ frc)[DP_F3]) {
+    constexpr int WK = (DP_P3 + DP_WG - 1) / DP_WG;
+    T w[WK];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-        xs[a] = wrapn(c[0] - 1 + a, N);
-        ys[a] = wrapn(c[1] - 1 + a, N);
-        zs[a] = wrapn(c[2] - 1 + a, N);
+    for (int k = 0; k < WK; ++k) {
+        const int i = threadIdx.x + DP_WG * k;
+        if (i < DP_P3)
+            w[k] = phi[site_index(N, 1, wrapn(r.ox - 1 + i % DP_PW, N), wrapn(r.oy - 1 + (i / DP_PW) % DP_PW, N),
+                                  wrapn(r.oz - 1 + i / (DP_PW * DP_PW), N))];
     }
+#pragma unroll
+    for (int k = 0; k < WK; ++k) {
+        const int i = threadIdx.x + DP_WG * k;
+        if (i < DP_P3) phw[i] = w[k];
+    }
+    __syncthreads();
     const T hn = (T)0.5 * (T)N;
-    auto P = [&](int a, int b, int e) { return phi[site_index(N, 1, xs[a], ys[b], zs[e])]; };
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                Fc[0][k][j][i] = -(P(i + 2, j + 1, k + 1) - P(i, j + 1, k + 1)) * hn;
-                Fc[1][k][j][i] = -(P(i + 1, j + 2, k + 1) - P(i + 1, j, k + 1)) * hn;
-                Fc[2][k][j][i] = -(P(i + 1, j + 1, k + 2) - P(i + 1, j + 1, k)) * hn;
-            }
+    for (int i = threadIdx.x; i < DP_F3; i += DP_WG) {
+        const int c = i % DP_FW + 1 + DP_PW * ((i / DP_FW) % DP_FW + 1 + DP_PW * (i / (DP_FW * DP_FW) + 1));
+        frc[0][i] = -(phw[c + 1] - phw[c - 1]) * hn;
+        frc[1][i] = -(phw[c + DP_PW] - phw[c - DP_PW]) * hn;
+        frc[2][i] = -(phw[c + DP_PW * DP_PW] - phw[c - DP_PW * DP_PW]) * hn;
+    }
+    __syncthreads();
 }
 
-// v += dt a(X); X += dt N v; re-anchor
-template <typename T> __global__ void dp_step_kernel(DpState<T> s, const T *__restrict__ phi, T dt) {
+// v += dt a(X); X += dt N v; re-anchor: state s -> state t (the particles keep their numbers)
+template <typename T>
+__global__ __launch_bounds__(DP_WG) void dp_step_kernel(DpState<T> s, DpState<T> t, BrickIndex V,
+                                                        const T *__restrict__ phi, T dt) {
+    __shared__ T phw[DP_P3];
+    __shared__ T frc[3][DP_F3];
+    BrickRange r;
+    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
     const int N = s.N;
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
+    brick_forces(phi, N, r, phw, frc);
+    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
+        const int p = V.list[j];
         int c[3];
-        decode(s.cell[p], N, c);
+        brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};
-        T Fc[3][2][2][2];
-        corner_forces(phi, N, c, Fc);
+        const T vin[3] = {s.vel[0][p], s.vel[1][p], s.vel[2][p]};
+        const int o = c[0] - r.ox + DP_FW * (c[1] - r.oy + DP_FW * (c[2] - r.oz));
         T a[3] = {(T)0, (T)0, (T)0};
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j2 = 0; j2 < 2; ++j2)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const T w = wsel(i, u[0]) * wsel(j, u[1]) * wsel(k, u[2]);
+                    const T w = wsel(i, u[0]) * wsel(j2, u[1]) * wsel(k, u[2]);
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) a[d] += w * Fc[d][k][j][i];
+                    for (int d = 0; d < 3; ++d) a[d] += w * frc[d][o + i + DP_FW * (j2 + DP_FW * k)];
                 }
         int cn[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const T v = s.vel[d][p] + dt * a[d];
-            s.vel[d][p] = v;
+            const T v = vin[d] + dt * a[d];
+            t.vel[d][p] = v;
             const double X = add_nc(add_nc((double)c[d], (double)u[d]), mul_nc(mul_nc((double)dt, (double)v), (double)N));
-            T o;
-            anchor<T>(X, N, cn[d], o);
-            s.off[d][p] = o;
+            T on;
+            anchor<T>(X, N, cn[d], on);
+            t.off[d][p] = on;
         }
-        s.cell[p] = cn[0] + N * (cn[1] + N * cn[2]);
+        t.cell[p] = cn[0] + N * (cn[1] + N * cn[2]);
     }
 }
 
@@ -235,56 +270,70 @@ __global__ void dp_pos_grad_kernel(DpState<T> s, const T *__restrict__ g, T qN, 
     }
 }
 
-// particle part of one backward step; fbar is a 3-component AoS field
+// One backward step's particle part, and phi-bar = sum_d D_d F-bar_d with
+// F-bar_d = sum_p mu_d W: F-bar is summed per brick in three FP64 LDS windows and its
+// differences are formed there, so that a brick adds one value to each node of its
+// [o - 1, o + 9] window of phi-bar instead of 24 terms per particle to a three-component
+// field (128^3 FP32 particles: 1960 us with global atomics, and a pass over the field for the
+// differences).
 template <typename T>
-__global__ void dp_adj_particles_kernel(DpState<T> s, const T *__restrict__ phi, T dt, T *__restrict__ lx,
-                                        T *__restrict__ lv, T *__restrict__ fbar) {
+__global__ __launch_bounds__(DP_WG) void dp_adj_kernel(DpState<T> s, BrickIndex V, const T *__restrict__ phi, T dt,
+                                                       T *__restrict__ lx, T *__restrict__ lv, T *__restrict__ phib) {
+    __shared__ T frc[3][DP_F3];
+    __shared__ double fb[3][DP_F3];  // the window of phi before
+    static_assert(sizeof(double) * 3 * DP_F3 >= sizeof(T) * DP_P3, "the window of phi fits");
+    BrickRange r;
+    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
     const int N = s.N;
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
+    brick_forces(phi, N, r, reinterpret_cast<T *>(&fb[0][0]), frc);
+    for (int i = threadIdx.x; i < 3 * DP_F3; i += DP_WG) (&fb[0][0])[i] = 0.0;
+    __syncthreads();
+    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
+        const int p = V.list[j];
         int c[3];
-        decode(s.cell[p], N, c);
+        brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};
-        T mu[3];
+        T mu[3], l[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const T v = lv[3 * p + d] + dt * lx[3 * p + d];
-            lv[3 * p + d] = v;
+            l[d] = lx[3 * (int64_t)p + d];
+            const T v = lv[3 * (int64_t)p + d] + dt * l[d];
+            lv[3 * (int64_t)p + d] = v;
             mu[d] = dt * v;
         }
-        T Fc[3][2][2][2];
-        corner_forces(phi, N, c, Fc);
+        const int o = c[0] - r.ox + DP_FW * (c[1] - r.oy + DP_FW * (c[2] - r.oz));
         T add[3] = {(T)0, (T)0, (T)0};
 #pragma unroll
         for (int k = 0; k < 2; ++k)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j2 = 0; j2 < 2; ++j2)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    const T wx = wsel(i, u[0]), wy = wsel(j, u[1]), wz = wsel(k, u[2]);
-                    const T mf = mu[0] * Fc[0][k][j][i] + mu[1] * Fc[1][k][j][i] + mu[2] * Fc[2][k][j][i];
+                    const int n = o + i + DP_FW * (j2 + DP_FW * k);
+                    const T wx = wsel(i, u[0]), wy = wsel(j2, u[1]), wz = wsel(k, u[2]);
+                    const T mf = mu[0] * frc[0][n] + mu[1] * frc[1][n] + mu[2] * frc[2][n];
                     add[0] += (i ? mf : -mf) * wy * wz;
-                    add[1] += wx * (j ? mf : -mf) * wz;
+                    add[1] += wx * (j2 ? mf : -mf) * wz;
                     add[2] += wx * wy * (k ? mf : -mf);
-                    const int64_t node = site_index(N, 1, wrapn(c[0] + i, N), wrapn(c[1] + j, N), wrapn(c[2] + k, N));
                     const T w = wx * wy * wz;
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) atomicAdd(&fbar[3 * node + d], mu[d] * w);
+                    for (int d = 0; d < 3; ++d) lds_add(&fb[d][n], (double)(mu[d] * w));
                 }
 #pragma unroll
-        for (int d = 0; d < 3; ++d) lx[3 * p + d] += (T)N * add[d];
+        for (int d = 0; d < 3; ++d) lx[3 * (int64_t)p + d] = l[d] + (T)N * add[d];
     }
-}
-
-// phi-bar = sum_d D_d F-bar_d on the interior, periodic
-template <typename T> __global__ void dp_divergence_kernel(const T *__restrict__ fbar, T *__restrict__ phib, int N) {
-    const int64_t n = (int64_t)N * N * N;
-    const T hn = (T)0.5 * (T)N;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
-        const int x = (int)(t % N), y = (int)((t / N) % N), z = (int)(t / ((int64_t)N * N));
-        auto F = [&](int xx, int yy, int zz, int d) { return fbar[3 * site_index(N, 1, wrapn(xx, N), wrapn(yy, N), wrapn(zz, N)) + d]; };
-        phib[site_index(N, 1, x, y, z)] = (F(x + 1, y, z, 0) - F(x - 1, y, z, 0)) * hn +
-                                          (F(x, y + 1, z, 1) - F(x, y - 1, z, 1)) * hn +
-                                          (F(x, y, z + 1, 2) - F(x, y, z - 1, 2)) * hn;
+    __syncthreads();
+    const double hn = 0.5 * (double)N;
+    for (int i = threadIdx.x; i < DP_P3; i += DP_WG) {
+        const int x = i % DP_PW - 1, y = (i / DP_PW) % DP_PW - 1, z = i / (DP_PW * DP_PW) - 1;
+        auto F = [&](int d, int xx, int yy, int zz) {
+            const bool in = xx >= 0 && xx < DP_FW && yy >= 0 && yy < DP_FW && zz >= 0 && zz < DP_FW;
+            return in ? fb[d][xx + DP_FW * (yy + DP_FW * zz)] : 0.0;
+        };
+        const double w = (F(0, x + 1, y, z) - F(0, x - 1, y, z)) + (F(1, x, y + 1, z) - F(1, x, y - 1, z)) +
+                         (F(2, x, y, z + 1) - F(2, x, y, z - 1));
+        if (w == 0.0) continue;
+        atomicAdd(&phib[site_index(N, 1, wrapn(r.ox + x, N), wrapn(r.oy + y, N), wrapn(r.oz + z, N))], (T)(w * hn));
     }
 }
 
@@ -306,7 +355,10 @@ struct lf2mi_diffpm_s {
     lf2mi_fft_plan plan;
     size_t tsize;   // sizeof(T)
     void *ck_mem;   // nsteps + 1 particle states (cell, off[3], vel[3])
-    void *rho, *phi, *resid, *fbar, *phib, *rhob;  // (N+2)^3 fields of T (fbar: 3 components)
+    void *rho, *phi, *resid, *phib, *rhob;  // (N+2)^3 fields of T
+    void *index_mem;  // brick index of one state (rebuilt for every state it is needed for)
+    size_t index_bytes;
+    lf2mi::BrickBuild bricks;
     void *lx, *lv;  // adjoints, np*3 of T
     double *loss_dev;
     bool forward_done;
@@ -339,34 +391,46 @@ int dp_malloc(void **p, size_t bytes) {
     return LF2MI_OK;
 }
 
-template <typename T> int dp_forces(lf2mi_diffpm_s *m, const DpState<T> &s, hipStream_t st) {
+unsigned dp_bricks_grid(const lf2mi_diffpm_s *m) {
+    const int64_t nb = (m->N + BRK - 1) / BRK;
+    return (unsigned)brick_items(nb * nb * nb, m->np);
+}
+
+// the brick index of state s and its density in m->rho
+template <typename T> int dp_density(lf2mi_diffpm_s *m, const DpState<T> &s, hipStream_t st) {
+    if (int rc = brick_build(s.cell, m->np, m->N, m->bricks, st)) return rc;
     dp_fill_kernel<T><<<dp_grid(m->G3), DP_WG, 0, st>>>((T *)m->rho, m->G3);
     LF2MI_LAUNCHED();
     const double n3 = (double)m->N * m->N * m->N;
-    dp_density_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(s, (T *)m->rho, (T)(m->mass * n3));
+    dp_density_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(s, brick_view(m->bricks, m->N), (T *)m->rho,
+                                                              (T)(m->mass * n3));
     LF2MI_LAUNCHED();
+    return LF2MI_OK;
+}
+
+// index, density and potential of state s
+template <typename T> int dp_potential(lf2mi_diffpm_s *m, const DpState<T> &s, hipStream_t st) {
+    if (int rc = dp_density<T>(m, s, st)) return rc;
+    const double n3 = (double)m->N * m->N * m->N;
     return lf2mi_poisson_solve(m->plan, m->rho, m->phi, m->mass * (double)m->np, 1.0 / n3, st);
 }
 
 template <typename T, typename I>
 int dp_forward(lf2mi_diffpm_s *m, const I *pos0, const I *vel0, const I *target, I *rho_out, double *loss, hipStream_t st) {
-    const size_t sb = dp_state_bytes(m->np, sizeof(T));
     dp_init_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, 0), pos0, vel0);
     LF2MI_LAUNCHED();
     for (int s = 0; s < m->nsteps; ++s) {
-        const DpState<T> nx = dp_view<T>(m, s + 1);
-        LF2MI_HIP(hipMemcpyAsync(nx.cell, dp_view<T>(m, s).cell, sb, hipMemcpyDeviceToDevice, st));
-        if (int rc = dp_forces<T>(m, nx, st)) return rc;
-        dp_step_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(nx, (const T *)m->phi, (T)m->dt);
+        const DpState<T> xs = dp_view<T>(m, s);
+        if (int rc = dp_potential<T>(m, xs, st)) return rc;
+        dp_step_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, dp_view<T>(m, s + 1), brick_view(m->bricks, m->N),
+                                                               (const T *)m->phi, (T)m->dt);
         LF2MI_LAUNCHED();
     }
     const DpState<T> fin = dp_view<T>(m, m->nsteps);
-    dp_fill_kernel<T><<<dp_grid(m->G3), DP_WG, 0, st>>>((T *)m->rho, m->G3);
+    if (int rc = dp_density<T>(m, fin, st)) return rc;
     dp_fill_kernel<double><<<1, DP_WG, 0, st>>>(m->loss_dev, 1);
     LF2MI_LAUNCHED();
     const double n3 = (double)m->N * m->N * m->N;
-    dp_density_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(fin, (T *)m->rho, (T)(m->mass * n3));
-    LF2MI_LAUNCHED();
     dp_resid_kernel<T, I><<<std::min<unsigned>(dp_grid((int64_t)n3), 1024), DP_WG, 0, st>>>(
         (const T *)m->rho, target, (T *)m->resid, rho_out, m->N, m->loss_dev);
     LF2MI_LAUNCHED();
@@ -387,12 +451,11 @@ template <typename T, typename I> int dp_backward(lf2mi_diffpm_s *m, I *grad_pos
     LF2MI_LAUNCHED();
     for (int s = m->nsteps - 1; s >= 0; --s) {
         const DpState<T> xs = dp_view<T>(m, s);
-        if (int rc = dp_forces<T>(m, xs, st)) return rc;  // recompute phi of step s
-        dp_fill_kernel<T><<<dp_grid(3 * m->G3), DP_WG, 0, st>>>((T *)m->fbar, 3 * m->G3);
+        if (int rc = dp_potential<T>(m, xs, st)) return rc;  // recompute phi of step s
+        dp_fill_kernel<T><<<dp_grid(m->G3), DP_WG, 0, st>>>((T *)m->phib, m->G3);
         LF2MI_LAUNCHED();
-        dp_adj_particles_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(xs, (const T *)m->phi, (T)m->dt, lx, lv, (T *)m->fbar);
-        LF2MI_LAUNCHED();
-        dp_divergence_kernel<T><<<dp_grid((int64_t)n3), DP_WG, 0, st>>>((const T *)m->fbar, (T *)m->phib, m->N);
+        dp_adj_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, brick_view(m->bricks, m->N), (const T *)m->phi,
+                                                              (T)m->dt, lx, lv, (T *)m->phib);
         LF2MI_LAUNCHED();
         if (int rc = lf2mi_poisson_solve(m->plan, m->phib, m->rhob, 0.0, 1.0 / n3, st)) return rc;
         dp_pos_grad_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(xs, (const T *)m->rhob, qN, lx, 0);
@@ -424,7 +487,7 @@ int lf2mi_diffpm_bytes(lf2mi_diffpm m, int64_t *bytes) {
     if (!m || !bytes) return fail(LF2MI_EINVAL, "lf2mi_diffpm_bytes: null argument");
     int64_t fft = 0;
     if (int rc = lf2mi_fft_plan_bytes(m->plan, &fft)) return rc;
-    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + 8 * (size_t)m->G3 * m->tsize +
+    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + 5 * (size_t)m->G3 * m->tsize + m->index_bytes +
                        6 * (size_t)m->np * m->tsize + sizeof(double)) + fft;
     return LF2MI_OK;
 }
@@ -451,7 +514,27 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     if (!rc) rc = dp_malloc(&m->rho, fb);
     if (!rc) rc = dp_malloc(&m->phi, fb);
     if (!rc) rc = dp_malloc(&m->resid, fb);
-    if (!rc) rc = dp_malloc(&m->fbar, 3 * fb);
+    const int64_t nb = (N + BRK - 1) / BRK, nbk = nb * nb * nb, items = brick_items(nbk, np);
+    // starts, item starts, counts, block totals, items, list, places
+    m->index_bytes = sizeof(int) * (size_t)(2 * (nbk + 1) + nbk + 2 * brick_blocks(nbk) + items + 2 * np);
+    if (!rc) rc = dp_malloc(&m->index_mem, m->index_bytes);
+    if (!rc) {
+        int *q = (int *)m->index_mem;
+        auto take = [&q](int64_t n) {
+            int *r = q;
+            q += n;
+            return r;
+        };
+        m->bricks.start = take(nbk + 1);
+        m->bricks.istart = take(nbk + 1);
+        m->bricks.count = take(nbk);
+        m->bricks.bsum = take(2 * brick_blocks(nbk));
+        m->bricks.item = take(items);
+        m->bricks.list = take(np);
+        m->bricks.rank = take(np);
+        hipError_t e = hipMemset(m->bricks.count, 0, sizeof(int) * (size_t)nbk);
+        if (e != hipSuccess) rc = hip_fail(e, "hipMemset(diffpm)", __FILE__, __LINE__);
+    }
     if (!rc) rc = dp_malloc(&m->phib, fb);
     if (!rc) rc = dp_malloc(&m->rhob, fb);
     if (!rc) rc = dp_malloc(&m->lx, (size_t)np * 3 * m->tsize);
@@ -478,7 +561,7 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
 int lf2mi_diffpm_destroy(lf2mi_diffpm m) {
     if (!m) return LF2MI_OK;
     if (m->plan) lf2mi_fft_plan_destroy(m->plan);
-    for (void *p : {m->ck_mem, m->rho, m->phi, m->resid, m->fbar, m->phib, m->rhob, m->lx, m->lv, (void *)m->loss_dev})
+    for (void *p : {m->ck_mem, m->index_mem, m->rho, m->phi, m->resid, m->phib, m->rhob, m->lx, m->lv, (void *)m->loss_dev})
         if (p) (void)hipFree(p);
     delete m;
     return LF2MI_OK;
