@@ -606,50 +606,22 @@ __device__ __forceinline__ bool item_range(int item, const int *__restrict__ sta
 // ---------------------------------------------------------------- deposit (F32)
 // The reference accumulates, per cell, the contributions of the cell's particles to the
 // nodes around it (localCube[8] / vi[36] / tii[24] + tij[54], particles/projections.hpp:
-// 140-179, :1034-1122, :1421-1521) and then adds them to the field.  Here one workgroup
-// takes an item (a chunk of at most ITEM_P particles of one brick) and
-//   A. counting-sorts the chunk by cell in LDS (one int LDS atomic per particle);
-//   B. each lane takes a run of DEP_PER consecutive sorted particles and sums their node
-//      terms per cell in registers; a run's inner cells go to the LDS node window with LDS
-//      atomics, its last cell is combined across the wave with a segmented DPP sum (equal
-//      cells are adjacent lanes after the sort) and added once per run of lanes, so a
-//      crowded cell costs the same as a sparse one.  The window holds 64-bit fixed point
-//      (integer LDS atomics: the FP32 LDS atomic add is many times slower on gfx950): per
-//      item and component a power-of-two scale puts the bound sum_p |q_p| (from the item's
-//      maxima of |q| and |v|) just below 2^51, so the window sums are exact and the only
-//      rounding past the FP32 run sums is the quantum 2^-51 of that bound;
-//   C. the node window (all components, component-fastest) is added into the field with
-//      one global atomic per non-zero value (periodic wrap or the unfolded ghost layer).
-// Node offsets per axis: {0, 1} on the vertex grid, {-1, 0, +1} on the link grid (nodes at
-// n + 1/2) and {0} on a nearest-grid-point axis, so 8 (scalar, T_ii), 12 (vector component),
-// 18 (T_ij), 4 (CIC-NGP vector component) or 2 (CIC-NGP T_ij) terms per particle and
-// component; the window spans nodes [LO, B] per axis, LO = -1 when a component of the kind
-// sits on links.
+// 140-179, :1034-1122, :1421-1521) and then adds them to the field.  Here a brick's particles
+// are summed in a window of its nodes in LDS first: tiles of bricks that store their nodes
+// once (deposit_tiles_kernel, deposit_tiles_c_kernel), or one brick per workgroup and atomics
+// into the field (deposit_brick32_kernel, dense_body).
+// A particle has two non-zero weights per axis on the vertex grid (nodes 0, 1) and on the link
+// grid (nodes -1, 0 or 0, 1 of the nodes at n + 1/2, the branch at the link midpoint of
+// projections.hpp:1058-1071, whose third weight is zero), and one on a nearest-grid-point axis:
+// 8 terms per component, or 4 (CIC-NGP vector) or 2 (CIC-NGP T_ij).  C: components; a window
+// spans nodes [LO, B] per axis, LO = -1 when a component of the kind sits on links.
 template <int KIND> struct KindC;
-// CW: components the node window holds at a time (VecVec runs two passes of three, which
-// keeps its LDS at the vector kind's)
-template <> struct KindC<0> { static constexpr int C = 1, CW = 1, LO = 0; };
-template <> struct KindC<1> { static constexpr int C = 3, CW = 3, LO = -1; };
-template <> struct KindC<2> { static constexpr int C = 6, CW = 3, LO = -1; };
+template <> struct KindC<0> { static constexpr int C = 1, LO = 0; };
+template <> struct KindC<1> { static constexpr int C = 3, LO = -1; };
+template <> struct KindC<2> { static constexpr int C = 6, LO = -1; };
 // the CIC-NGP hybrids (vertex and nearest-grid-point axes only)
-template <> struct KindC<3> { static constexpr int C = 3, CW = 3, LO = 0; };
-template <> struct KindC<4> { static constexpr int C = 6, CW = 3, LO = 0; };
-
-// link-grid weights of one axis as a 3-vector over node offsets {-1, 0, +1}
-// (projections.hpp:1058-1071: the branch at the link midpoint)
-__device__ __forceinline__ void link3(float u, float &wm, float &w0, float &wp) {
-    const float t = u - 0.5f;
-    if (t < 0.0f) {
-        const float a = -t;
-        wm = a;
-        w0 = 1.0f - a;
-        wp = 0.0f;
-    } else {
-        wm = 0.0f;
-        w0 = 1.0f - t;
-        wp = t;
-    }
-}
+template <> struct KindC<3> { static constexpr int C = 3, LO = 0; };
+template <> struct KindC<4> { static constexpr int C = 6, LO = 0; };
 
 // component c of kind KIND: stagger mask (bit d: link grid along axis d), nearest-grid-point
 // mask (bit d: the single node of the particle's cell along axis d, weight 1) and velocity
@@ -678,12 +650,6 @@ template <> struct Comp<4, 3> { static constexpr int MASK = 0, NGP = 0, VA = 1, 
 template <> struct Comp<4, 4> { static constexpr int MASK = 0, NGP = 6, VA = 1, VB = 2; };  // (1,2)
 template <> struct Comp<4, 5> { static constexpr int MASK = 0, NGP = 0, VA = 2, VB = 2; };  // (2,2)
 
-// nodes per axis d of a component: 3 on links, 1 for NGP, 2 on vertices
-template <int MASK, int NGP, int D>
-__host__ __device__ constexpr int axis_nodes() {
-    return (MASK >> D) & 1 ? 3 : ((NGP >> D) & 1 ? 1 : 2);
-}
-
 struct DepArgs {
     Soa32 s;
     const int *start;
@@ -697,549 +663,19 @@ struct DepArgs {
                              // fixed point counts dimensionless weights)
     int h;
     int tgt;
-    const int *dlist;        // deposit_f32_kernel: a list of items (with its count at dcount)
-    const int *dcount;       // instead of one item per workgroup
 };
 
-template <typename ACC> struct AccOps;
-template <> struct AccOps<float> {
-    static __device__ __forceinline__ float term(float q, float w, double) { return q * w; }
-    static __device__ __forceinline__ void flush(const DepArgs &A, int64_t idx, float v) {
-        atomicAdd(&A.field[idx], v);
-    }
-};
-template <> struct AccOps<unsigned long long> {
-    // each particle's term is quantised on its own, so the integer sums do not depend on order
-    static __device__ __forceinline__ unsigned long long term(float q, float w, double fxscale) {
-        return (unsigned long long)llrint((double)(q * w) * fxscale);
-    }
-    static __device__ __forceinline__ void flush(const DepArgs &A, int64_t idx, unsigned long long v) {
-        atomicAdd(&A.fx[idx], v);
-    }
-};
-
-// ---- segmented sum over the lanes of a wave (DPP)
-// update_dpp with bound_ctrl off: lanes whose source is outside the row, or whose row the
-// row mask leaves out, get `old`.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ int dpp_i32(int old, int v) {
-    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWMASK, 0xf, false);
-}
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ float dpp_val(float v) {
-    return __int_as_float(dpp_i32<CTRL, ROWMASK>(0, __float_as_int(v)));
-}
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ unsigned long long dpp_val(unsigned long long v) {
-    const unsigned lo = (unsigned)dpp_i32<CTRL, ROWMASK>(0, (int)(unsigned)v);
-    const unsigned hi = (unsigned)dpp_i32<CTRL, ROWMASK>(0, (int)(unsigned)(v >> 32));
-    return ((unsigned long long)hi << 32) | lo;
-}
-template <int CTRL, int ROWMASK, typename T, int NS>
-__device__ __forceinline__ void seg_step(int key, T (&v)[NS]) {
-    const bool same = dpp_i32<CTRL, ROWMASK>(-2, key) == key;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-        const T s = dpp_val<CTRL, ROWMASK>(v[k]);
-        v[k] += same ? s : T(0);
-    }
-}
-// Inclusive segmented scan over the 64 lanes (all active): lanes with equal keys must be
-// adjacent (keys >= 0, the sentinel -2 never matches); afterwards the last lane of each run
-// of equal keys holds the run's sum.  Within rows of 16: shifts by 1, 2, 4, 8; then lane 15
-// of rows 0 and 2 into rows 1 and 3, and lane 31 into rows 2 and 3.
-template <typename T, int NS>
-__device__ __forceinline__ void seg_scan(int key, T (&v)[NS]) {
-    seg_step<0x111, 0xf>(key, v);  // row_shr:1
-    seg_step<0x112, 0xf>(key, v);  // row_shr:2
-    seg_step<0x114, 0xf>(key, v);  // row_shr:4
-    seg_step<0x118, 0xf>(key, v);  // row_shr:8
-    seg_step<0x142, 0xa>(key, v);  // row_bcast:15
-    seg_step<0x143, 0xc>(key, v);  // row_bcast:31
+// each particle's term of a fixed-point deposit is quantised on its own, so the integer sums do
+// not depend on order
+__device__ __forceinline__ unsigned long long fx_term(float q, float w, double fxscale) {
+    return (unsigned long long)llrint((double)(q * w) * fxscale);
 }
 
-static constexpr int DEP_PER = ITEM_P / DEP_WG;  // sorted particles per lane run
-
-// window value of a run sum: FP32 sums in the item's fixed point (nearest), fixed-point terms
-// as they are.  |x scale| < 2^51, so adding 1.5 2^52 leaves the rounded integer in the low
-// mantissa bits of the sum (two's complement once the constant's bits are taken off).
-__device__ __forceinline__ unsigned long long to_window(float x, double scale) {
-    const double t = fma((double)x, scale, 0x1.8p52);
-    return (unsigned long long)(__double_as_longlong(t) - 0x4338000000000000ll);
-}
-__device__ __forceinline__ unsigned long long to_window(unsigned long long x, double) { return x; }
-
-// add a cell's NS node terms into the LDS node window of one component (edge NWE,
-// origin LO): node offsets per axis start at -1 on link axes, 0 on the others
-template <int MASK, int NGP, int LO, typename ACC, int NS>
-__device__ __forceinline__ void window_add(unsigned long long *nd, int cell, int B, int NWE, const ACC (&acc)[NS],
-                                           double scale) {
-    constexpr int SX = axis_nodes<MASK, NGP, 0>(), SY = axis_nodes<MASK, NGP, 1>(), SZ = axis_nodes<MASK, NGP, 2>();
-    const int lx = cell % B, ly = (cell / B) % B, lz = cell / (B * B);
-    const int base = (lx + ((MASK & 1) ? -1 : 0) - LO) + NWE * ((ly + ((MASK & 2) ? -1 : 0) - LO) +
-                                                              NWE * (lz + ((MASK & 4) ? -1 : 0) - LO));
-#pragma unroll
-    for (int kz = 0; kz < SZ; ++kz)
-#pragma unroll
-        for (int ky = 0; ky < SY; ++ky)
-#pragma unroll
-            for (int kx = 0; kx < SX; ++kx)
-                atomicAdd(&nd[base + kx + NWE * (ky + NWE * kz)], to_window(acc[kx + SX * (ky + SY * kz)], scale));
-}
-
-// phase B for one component: the lane's run of sorted particles (cells key[k], -1 past the
-// item's end), its last cell carried across the wave
-template <int KIND, int COMP, typename ACC, int BC, int PER = DEP_PER>
-__device__ __forceinline__ void deposit_component(const DepArgs &A, int B, int NWE, const int (&key)[PER],
-                                                  const float4 (&pd)[PER], const float4 (&pv)[PER],
-                                                  int ckey, bool any_shared, bool carry_end, unsigned long long *nodes,
-                                                  double scale) {
-    constexpr int MASK = Comp<KIND, COMP>::MASK, NGP = Comp<KIND, COMP>::NGP;
-    constexpr int VA = Comp<KIND, COMP>::VA, VB = Comp<KIND, COMP>::VB;
-    constexpr int SX = axis_nodes<MASK, NGP, 0>(), SY = axis_nodes<MASK, NGP, 1>(), SZ = axis_nodes<MASK, NGP, 2>();
-    constexpr int NS = SX * SY * SZ;
-    constexpr int LO = KindC<KIND>::LO;
-    constexpr int NWMAX = MAXB + 1 - LO;
-    unsigned long long *nd = nodes + (COMP % KindC<KIND>::CW) * NWMAX * NWMAX * NWMAX;
-    ACC acc[NS];
-#pragma unroll
-    for (int k = 0; k < NS; ++k) acc[k] = ACC(0);
-    int cur = -1;
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-        const int c = key[p];
-        if (c < 0) continue;  // past the end: every later particle of the run is too
-        if (c != cur) {
-            if (cur >= 0) {
-                window_add<MASK, NGP, LO>(nd, cur, B, NWE, acc, scale);
-#pragma unroll
-                for (int k = 0; k < NS; ++k) acc[k] = ACC(0);
-            }
-            cur = c;
-        }
-        const float4 d = pd[p];
-        float q = d.w;
-        if constexpr (VA >= 0) {
-            const float4 v = pv[p];
-            q *= VA == 0 ? v.x : (VA == 1 ? v.y : v.z);
-            if constexpr (VB >= 0) q *= (VB == 0 ? v.x : (VB == 1 ? v.y : v.z));
-        }
-        float wx[3], wy[3], wz[3];
-        if constexpr (MASK & 1) link3(d.x, wx[0], wx[1], wx[2]);
-        else if constexpr (NGP & 1) wx[0] = 1.0f;
-        else { wx[0] = 1.0f - d.x; wx[1] = d.x; }
-        if constexpr (MASK & 2) link3(d.y, wy[0], wy[1], wy[2]);
-        else if constexpr (NGP & 2) wy[0] = 1.0f;
-        else { wy[0] = 1.0f - d.y; wy[1] = d.y; }
-        if constexpr (MASK & 4) link3(d.z, wz[0], wz[1], wz[2]);
-        else if constexpr (NGP & 4) wz[0] = 1.0f;
-        else { wz[0] = 1.0f - d.z; wz[1] = d.z; }
-#pragma unroll
-        for (int kz = 0; kz < SZ; ++kz)
-#pragma unroll
-            for (int ky = 0; ky < SY; ++ky)
-#pragma unroll
-                for (int kx = 0; kx < SX; ++kx)
-                    acc[kx + SX * (ky + SY * kz)] += AccOps<ACC>::term(q, wx[kx] * wy[ky] * wz[kz], A.fxs[COMP]);
-    }
-    // the run's last cell: summed over the lanes that share it (uniform branch)
-    if (any_shared) seg_scan(ckey, acc);
-    if (carry_end) window_add<MASK, NGP, LO>(nd, cur, B, NWE, acc, scale);
-}
-
-// item maxima: |q| and |v_d| as the bits of non-negative floats (ordered like the values)
-struct DepMax {
-    unsigned int q, v[3];
-};
-
-// per-item fixed-point scale of one component: 2^(51 - e) with sum_p |q_p v_a v_b| < 2^e
-template <int KIND, int COMP>
-__device__ __forceinline__ double window_scale(int n, const DepMax &m) {
-    constexpr int VA = Comp<KIND, COMP>::VA, VB = Comp<KIND, COMP>::VB;
-    double bound = (double)n * (double)__uint_as_float(m.q);
-    if constexpr (VA >= 0) bound *= (double)__uint_as_float(m.v[VA]);
-    if constexpr (VB >= 0) bound *= (double)__uint_as_float(m.v[VB]);
-    if (!(bound > 0.0) || !(bound < 1e300)) return 1.0;  // all zero (or not finite)
-    int e;
-    frexp(bound, &e);
-    return ldexp(1.0, 51 - e);
-}
-
-// grid: one workgroup per item.  LDS is what limits the workgroups per CU (the kernel
-// slows down steeply with fewer), so the sorted particles are kept as planes of floats
-// without a mass plane when the mass is global (PM false), with 16-bit cell keys, and the
-// cell counts turn into starts in place.
-template <int KIND, typename ACC, int BC, bool PM>
-__device__ __forceinline__ void deposit_item(const DepArgs &A, int item) {
-    constexpr int C = KindC<KIND>::C, CW = KindC<KIND>::CW;
-    constexpr int LO = KindC<KIND>::LO;
-    constexpr int NWMAX = MAXB + 1 - LO;
-    constexpr int NW3 = NWMAX * NWMAX * NWMAX;
-    constexpr int NCMAX = MAXB * MAXB * MAXB;
-    constexpr bool FX = sizeof(ACC) == 8;  // global fixed point: terms quantised per particle
-    static_assert(2 * DEP_WG >= NCMAX, "two cells per thread in the scan");
-    static_assert(C % CW == 0, "whole window passes");
-    // the sorted particles (offset planes, mass plane if PM, velocity planes if KIND > 0,
-    // keys), then (aliased) the node window
-    constexpr size_t PL_B = sizeof(float) * ITEM_P;
-    constexpr int NPL = 3 + (PM ? 1 : 0) + (KIND > 0 ? 3 : 0);
-    constexpr size_t SK_B = sizeof(unsigned short) * ITEM_P;
-    constexpr size_t ND_B = sizeof(unsigned long long) * CW * NW3;
-    constexpr size_t POOL_B = NPL * PL_B + SK_B > ND_B ? NPL * PL_B + SK_B : ND_B;
-    __shared__ int cst[NCMAX];  // counts, then (in place) exclusive starts
-    __shared__ int scan_sh[DEP_WG / 64];
-    __shared__ DepMax smax;
-    __shared__ __align__(16) unsigned char pool[POOL_B];
-    float *pl = reinterpret_cast<float *>(pool);  // plane k at pl + k * ITEM_P: u.x u.y u.z [q] [v.x v.y v.z]
-    constexpr int QPL = 3, VPL = PM ? 4 : 3;
-    unsigned short *skey = reinterpret_cast<unsigned short *>(pool + NPL * PL_B);
-    unsigned long long *nodes = reinterpret_cast<unsigned long long *>(pool);
-    ItemRange r;
-    if (!item_range(item, A.start, A.istart, A.item_bucket, A.g, r)) return;
-    const int p0 = r.p0, n = r.p1 - r.p0;
-    const int B = BC ? BC : A.g.B, N = A.g.N;
-    const int NC = B * B * B, NWE = B + 1 - LO;
-    const int lane = lane_id();
-    for (int i = threadIdx.x; i < NC; i += DEP_WG) cst[i] = 0;
-    if (threadIdx.x == 0) smax = DepMax{0u, {0u, 0u, 0u}};
-    __syncthreads();
-    // A. load and rank by cell; item maxima of |q| and |v|
-    {
-        int lc[DEP_PER], rk[DEP_PER];
-        float4 qd[DEP_PER], qv[DEP_PER];
-        float mq = 0.0f, mv[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int k = 0; k < DEP_PER; ++k) {
-            const int i = threadIdx.x + k * DEP_WG;
-            lc[k] = -1;
-            if (i < n) {
-                const int p = p0 + i;
-                const int cell = A.s.cell[p];
-                int lx, ly, lz;
-                decode_cell(cell, A.g, lx, ly, lz);
-                lc[k] = (lx - r.ox) + B * ((ly - r.oy) + B * (lz - r.oz));
-                qd[k] = make_float4(A.s.off[0][p], A.s.off[1][p], A.s.off[2][p],
-                                    PM ? A.s.mass[p] * A.mass_nv : A.mass_nv);
-                mq = fmaxf(mq, fabsf(qd[k].w));
-                if constexpr (KIND > 0) {
-                    qv[k] = make_float4(A.s.vel[0][p], A.s.vel[1][p], A.s.vel[2][p], 0.0f);
-                    mv[0] = fmaxf(mv[0], fabsf(qv[k].x));
-                    mv[1] = fmaxf(mv[1], fabsf(qv[k].y));
-                    mv[2] = fmaxf(mv[2], fabsf(qv[k].z));
-                }
-                rk[k] = atomicAdd(&cst[lc[k]], 1);
-            }
-        }
-        if constexpr (!FX) {
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                mq = fmaxf(mq, __shfl_xor(mq, o));
-                if constexpr (KIND > 0) {
-                    mv[0] = fmaxf(mv[0], __shfl_xor(mv[0], o));
-                    mv[1] = fmaxf(mv[1], __shfl_xor(mv[1], o));
-                    mv[2] = fmaxf(mv[2], __shfl_xor(mv[2], o));
-                }
-            }
-            if (lane == 0) {
-                atomicMax(&smax.q, __float_as_uint(mq));
-                if constexpr (KIND > 0) {
-                    atomicMax(&smax.v[0], __float_as_uint(mv[0]));
-                    atomicMax(&smax.v[1], __float_as_uint(mv[1]));
-                    atomicMax(&smax.v[2], __float_as_uint(mv[2]));
-                }
-            }
-        }
-        __syncthreads();
-        // exclusive scan of the NC <= 512 counts in place, two cells per thread (the scan's
-        // first barrier orders every read before any write)
-        {
-            const int c0 = 2 * threadIdx.x, c1 = c0 + 1;
-            const int a0 = c0 < NC ? cst[c0] : 0, a1 = c1 < NC ? cst[c1] : 0;
-            int total;
-            const int ex = block_excl_scan_fast(a0 + a1, scan_sh, total);
-            if (c0 < NC) cst[c0] = ex;
-            if (c1 < NC) cst[c1] = ex + a0;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < DEP_PER; ++k) {
-            if (lc[k] >= 0) {
-                const int j = cst[lc[k]] + rk[k];
-                skey[j] = (unsigned short)lc[k];
-                pl[0 * ITEM_P + j] = qd[k].x;
-                pl[1 * ITEM_P + j] = qd[k].y;
-                pl[2 * ITEM_P + j] = qd[k].z;
-                if constexpr (PM) pl[QPL * ITEM_P + j] = qd[k].w;
-                if constexpr (KIND > 0) {
-                    pl[(VPL + 0) * ITEM_P + j] = qv[k].x;
-                    pl[(VPL + 1) * ITEM_P + j] = qv[k].y;
-                    pl[(VPL + 2) * ITEM_P + j] = qv[k].z;
-                }
-            }
-        }
-    }
-    __syncthreads();
-    // B. lane runs of DEP_PER consecutive sorted particles, held in registers (the node
-    // window then takes over their LDS)
-    // (whole 16-byte rows of each plane: the run starts at a multiple of DEP_PER = 4; values
-    // past the item's end are masked by their key)
-    static_assert(DEP_PER == 4, "runs are read as 16-byte rows");
-    int key[DEP_PER];
-    float4 pd[DEP_PER], pv[DEP_PER];
-    const int j0 = DEP_PER * threadIdx.x;
-    {
-        const float4 ux = *reinterpret_cast<const float4 *>(pl + 0 * ITEM_P + j0);
-        const float4 uy = *reinterpret_cast<const float4 *>(pl + 1 * ITEM_P + j0);
-        const float4 uz = *reinterpret_cast<const float4 *>(pl + 2 * ITEM_P + j0);
-        float4 uq = make_float4(A.mass_nv, A.mass_nv, A.mass_nv, A.mass_nv);
-        if constexpr (PM) uq = *reinterpret_cast<const float4 *>(pl + QPL * ITEM_P + j0);
-        const ushort4 kk = *reinterpret_cast<const ushort4 *>(skey + j0);
-        pd[0] = make_float4(ux.x, uy.x, uz.x, uq.x);
-        pd[1] = make_float4(ux.y, uy.y, uz.y, uq.y);
-        pd[2] = make_float4(ux.z, uy.z, uz.z, uq.z);
-        pd[3] = make_float4(ux.w, uy.w, uz.w, uq.w);
-        key[0] = j0 + 0 < n ? (int)kk.x : -1;
-        key[1] = j0 + 1 < n ? (int)kk.y : -1;
-        key[2] = j0 + 2 < n ? (int)kk.z : -1;
-        key[3] = j0 + 3 < n ? (int)kk.w : -1;
-        if constexpr (KIND > 0) {
-            const float4 vx = *reinterpret_cast<const float4 *>(pl + (VPL + 0) * ITEM_P + j0);
-            const float4 vy = *reinterpret_cast<const float4 *>(pl + (VPL + 1) * ITEM_P + j0);
-            const float4 vz = *reinterpret_cast<const float4 *>(pl + (VPL + 2) * ITEM_P + j0);
-            pv[0] = make_float4(vx.x, vy.x, vz.x, 0.f);
-            pv[1] = make_float4(vx.y, vy.y, vz.y, 0.f);
-            pv[2] = make_float4(vx.z, vy.z, vz.z, 0.f);
-            pv[3] = make_float4(vx.w, vy.w, vz.w, 0.f);
-        }
-    }
-    const DepMax m = smax;
-    __syncthreads();
-    for (int i = threadIdx.x; i < CW * NW3; i += DEP_WG) nodes[i] = 0ull;
-    int ckey = -1;  // the run's last cell
-#pragma unroll
-    for (int k = 0; k < DEP_PER; ++k) ckey = key[k] >= 0 ? key[k] : ckey;
-    const int next = __shfl_down(ckey, 1);
-    const int prev = __shfl_up(ckey, 1);
-    const bool any_shared = __ballot(lane > 0 && ckey >= 0 && prev == ckey) != 0ull;
-    const bool carry_end = ckey >= 0 && (lane == 63 || next != ckey);
-    __syncthreads();
-    double sc[C];
-#define LF2MI_DEP_COMP(K, I)                                                                               \
-    sc[I] = FX ? 1.0 : window_scale<K, I>(n, m);                                                           \
-    deposit_component<K, I, ACC, BC>(A, B, NWE, key, pd, pv, ckey, any_shared, carry_end, nodes, sc[I]);
-    if constexpr (KIND == 0) {
-        LF2MI_DEP_COMP(0, 0)
-    } else {
-        LF2MI_DEP_COMP(KIND, 0)
-        LF2MI_DEP_COMP(KIND, 1)
-        LF2MI_DEP_COMP(KIND, 2)
-    }
-    __syncthreads();
-    // C. the node window into the field, component-fastest (consecutive addresses of the
-    // interleaved field), zeros skipped; components c0 .. c0 + CW - 1
-    const int nn = NWE * NWE * NWE;
-    auto flush = [&](int c0) {
-        for (int i = threadIdx.x; i < CW * nn; i += DEP_WG) {
-            const int mnode = i / CW, cw = i - mnode * CW, c = c0 + cw;
-            const unsigned long long w = nodes[cw * NW3 + mnode];
-            if (w == 0ull) continue;
-            const int ax = mnode % NWE + LO, ay = (mnode / NWE) % NWE + LO, az = mnode / (NWE * NWE) + LO;
-            int gx = r.ox + ax, gy = r.oy + ay, gz = r.oz + az;
-            if (A.tgt == LF2MI_DEP_PERIODIC) {
-                gx = wrapi(gx, N);
-                gy = wrapi(gy, N);
-                gz = wrapi(gz, N);
-            }
-            const int64_t idx = site_index(N, A.h, gx, gy, gz) * C + c;
-            if constexpr (FX) {
-                AccOps<ACC>::flush(A, idx, w);
-            } else {
-                double inv = 1.0;
-#pragma unroll
-                for (int k = 0; k < C; ++k)
-                    if (k == c) inv = 1.0 / sc[k];
-                atomicAdd(&A.field[idx], (float)((double)(long long)w * inv));
-            }
-        }
-    };
-    flush(0);
-    if constexpr (C == 6) {
-        // the window's second pass: T_11, T_12, T_22
-        __syncthreads();
-        for (int i = threadIdx.x; i < CW * NW3; i += DEP_WG) nodes[i] = 0ull;
-        __syncthreads();
-        LF2MI_DEP_COMP(KIND, 3)
-        LF2MI_DEP_COMP(KIND, 4)
-        LF2MI_DEP_COMP(KIND, 5)
-        __syncthreads();
-        flush(3);
-    }
-#undef LF2MI_DEP_COMP
-}
-
-// one item per workgroup, or (A.dlist) the items of a work list, grid-stride
-template <int KIND, typename ACC, int BC, bool PM>
-__global__ __launch_bounds__(DEP_WG) void deposit_f32_kernel(DepArgs A) {
-    if (A.dlist) {
-        const int cnt = *A.dcount;
-        for (int it = blockIdx.x; it < cnt; it += gridDim.x) {
-            deposit_item<KIND, ACC, BC, PM>(A, A.dlist[it]);
-            __syncthreads();  // the LDS is reused
-        }
-    } else {
-        deposit_item<KIND, ACC, BC, PM>(A, blockIdx.x);
-    }
-}
-
-// Scalar deposit with a global mass: a workgroup takes up to DEP_MERGE consecutive items of
-// one brick (the first of each group; the others exit) and sorts them one after the other
-// into the same node window, so a dense brick's nodes are added to the field once per group
-// rather than once per item.  With one mass the fixed-point bound is n m, known before any
-// particle is read.  Phases as in deposit_f32_kernel; the window has its own LDS here.
-static constexpr int DEP_MERGE = 8;
-// consecutive items of a group sorted together (a lane's run holds DEP_SORT * DEP_PER sorted
-// particles): 1, since the larger LDS planes of 2 or 4 cost more occupancy than the longer
-// runs save
-static constexpr int DEP_SORT = 1;
-
-template <typename ACC, int BC>
-__global__ __launch_bounds__(DEP_WG) void deposit_merged_kernel(DepArgs A) {
-    constexpr int NWMAX = MAXB + 1;
-    constexpr int NW3 = NWMAX * NWMAX * NWMAX;
-    constexpr int NCMAX = MAXB * MAXB * MAXB;
-    constexpr bool FX = sizeof(ACC) == 8;
-    constexpr int SP = DEP_SORT * ITEM_P;  // particles per sort
-    constexpr int PER = SP / DEP_WG;       // sorted particles per lane run
-    static_assert(PER % 4 == 0, "runs are read as 16-byte rows");
-    static_assert(DEP_MERGE % DEP_SORT == 0, "whole sorts per group");
-    static_assert(2 * DEP_WG >= NCMAX, "two cells per thread in the scan");
-    __shared__ int cst[NCMAX];
-    __shared__ int scan_sh[DEP_WG / 64];
-    __shared__ __align__(16) float pl[3][SP];
-    __shared__ __align__(16) unsigned short skey[SP];
-    __shared__ unsigned long long nodes[NW3];
-    ItemRange r;
-    if (!item_range(blockIdx.x, A.start, A.istart, A.item_bucket, A.g, r)) return;
-    const int bstart = A.start[r.b], bend = A.start[r.b + 1];
-    if (((r.p0 - bstart) / ITEM_P) % DEP_MERGE != 0) return;  // taken by the group's first item
-    const int end = min(bend, r.p0 + DEP_MERGE * ITEM_P);
-    const int B = BC ? BC : A.g.B, N = A.g.N;
-    const int NC = B * B * B, NWE = B + 1;
-    const int lane = lane_id();
-    const DepMax m{__float_as_uint(A.mass_nv), {0u, 0u, 0u}};
-    const double sc = FX ? 1.0 : window_scale<0, 0>(end - r.p0, m);
-    for (int i = threadIdx.x; i < NW3; i += DEP_WG) nodes[i] = 0ull;
-    // the next sort's particles are loaded before the current sort's lane runs
-    int nc[PER];
-    float3 nq[PER];
-    auto fetch = [&](int q0) {
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-            const int p = q0 + threadIdx.x + k * DEP_WG;
-            nc[k] = -1;
-            if (p < end) {
-                nc[k] = A.s.cell[p];
-                nq[k] = make_float3(A.s.off[0][p], A.s.off[1][p], A.s.off[2][p]);
-            }
-        }
-    };
-    fetch(r.p0);
-    for (int p0 = r.p0; p0 < end; p0 += SP) {
-        const int n = min(SP, end - p0);
-        for (int i = threadIdx.x; i < NC; i += DEP_WG) cst[i] = 0;
-        __syncthreads();
-        // A. rank by cell
-        {
-            int lc[PER], rk[PER];
-            float3 qd[PER];
-#pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                lc[k] = -1;
-                qd[k] = nq[k];
-                if (nc[k] >= 0) {
-                    int lx, ly, lz;
-                    decode_cell(nc[k], A.g, lx, ly, lz);
-                    lc[k] = (lx - r.ox) + B * ((ly - r.oy) + B * (lz - r.oz));
-                    rk[k] = atomicAdd(&cst[lc[k]], 1);
-                }
-            }
-            __syncthreads();
-            {
-                const int c0 = 2 * threadIdx.x, c1 = c0 + 1;
-                const int a0 = c0 < NC ? cst[c0] : 0, a1 = c1 < NC ? cst[c1] : 0;
-                int total;
-                const int ex = block_excl_scan_fast(a0 + a1, scan_sh, total);
-                if (c0 < NC) cst[c0] = ex;
-                if (c1 < NC) cst[c1] = ex + a0;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < PER; ++k) {
-                if (lc[k] >= 0) {
-                    const int j = cst[lc[k]] + rk[k];
-                    skey[j] = (unsigned short)lc[k];
-                    pl[0][j] = qd[k].x;
-                    pl[1][j] = qd[k].y;
-                    pl[2][j] = qd[k].z;
-                }
-            }
-        }
-        __syncthreads();
-        // B. lane runs into the window (16-byte rows of each plane; values past the end
-        // are masked by their key)
-        int key[PER];
-        float4 pd[PER], pv[PER];
-        const int j0 = PER * threadIdx.x;
-        const float q = A.mass_nv;
-#pragma unroll
-        for (int h = 0; h < PER / 4; ++h) {
-            const int jr = j0 + 4 * h;
-            const float4 ux = *reinterpret_cast<const float4 *>(&pl[0][jr]);
-            const float4 uy = *reinterpret_cast<const float4 *>(&pl[1][jr]);
-            const float4 uz = *reinterpret_cast<const float4 *>(&pl[2][jr]);
-            const ushort4 kk = *reinterpret_cast<const ushort4 *>(&skey[jr]);
-            pd[4 * h + 0] = make_float4(ux.x, uy.x, uz.x, q);
-            pd[4 * h + 1] = make_float4(ux.y, uy.y, uz.y, q);
-            pd[4 * h + 2] = make_float4(ux.z, uy.z, uz.z, q);
-            pd[4 * h + 3] = make_float4(ux.w, uy.w, uz.w, q);
-            key[4 * h + 0] = jr + 0 < n ? (int)kk.x : -1;
-            key[4 * h + 1] = jr + 1 < n ? (int)kk.y : -1;
-            key[4 * h + 2] = jr + 2 < n ? (int)kk.z : -1;
-            key[4 * h + 3] = jr + 3 < n ? (int)kk.w : -1;
-        }
-        if (p0 + SP < end) fetch(p0 + SP);
-        int ckey = -1;
-#pragma unroll
-        for (int k = 0; k < PER; ++k) ckey = key[k] >= 0 ? key[k] : ckey;
-        const int next = __shfl_down(ckey, 1);
-        const int prev = __shfl_up(ckey, 1);
-        const bool any_shared = __ballot(lane > 0 && ckey >= 0 && prev == ckey) != 0ull;
-        const bool carry_end = ckey >= 0 && (lane == 63 || next != ckey);
-        deposit_component<0, 0, ACC, BC, PER>(A, B, NWE, key, pd, pv, ckey, any_shared, carry_end, nodes, sc);
-        __syncthreads();  // the planes and counts are reused by the next sort
-    }
-    // C. the window into the field
-    const int nn = NWE * NWE * NWE;
-    const double inv = 1.0 / sc;
-    for (int i = threadIdx.x; i < nn; i += DEP_WG) {
-        const unsigned long long w = nodes[i];
-        if (w == 0ull) continue;
-        const int ax = i % NWE, ay = (i / NWE) % NWE, az = i / (NWE * NWE);
-        int gx = r.ox + ax, gy = r.oy + ay, gz = r.oz + az;
-        if (A.tgt == LF2MI_DEP_PERIODIC) {
-            gx = wrapi(gx, N);
-            gy = wrapi(gy, N);
-            gz = wrapi(gz, N);
-        }
-        const int64_t idx = site_index(N, A.h, gx, gy, gz);
-        if constexpr (FX) AccOps<ACC>::flush(A, idx, w);
-        else atomicAdd(&A.field[idx], (float)((double)(long long)w * inv));
-    }
-}
+static constexpr int DEP_MERGE = 8;  // items one deposit workgroup takes
 
 // ---------------------------------------------------------------- scalar deposit, periodic target
-// Three kernels replace the item kernels when the target is periodic, the brick edge 8, the
-// number of bricks per row a multiple of TILE_B and the mass global (the PM step's deposit).
+// Three kernels, when the target is periodic, the brick edge 8, the number of bricks per row a
+// multiple of TILE_B and the mass global (the PM step's deposit).
 // A brick's nodes are [0,8)^3 relative to its origin; its particles also reach the first
 // node layer of the bricks above it along x, y and z.
 //  * deposit_tiles_kernel: one workgroup per tile of TILE_B bricks along x, one wave per
@@ -1267,12 +703,13 @@ static constexpr int TILE_B = 8;           // bricks per tile (one wave each)
 static constexpr int TILE_X = 8 * TILE_B;  // nodes per tile row
 
 // a particle's term for node weight w: float accumulation takes q w times the window scale
-// in FP64 (qsc = q * scale, one FMA against 1.5 2^52 as in to_window); the fixed point
+// in FP64 (qsc = q * scale, one FMA against 1.5 2^52: |term| < 2^51 leaves the rounded integer in the low
+// mantissa bits of the sum, two's complement once the constant's bits are taken off); the fixed point
 // quantises fl(q w) to the global scale on its own
 template <typename ACC>
 __device__ __forceinline__ unsigned long long dep_term(float q, float w, double qsc, double fxs) {
     if constexpr (sizeof(ACC) == 8) {
-        return AccOps<ACC>::term(q, w, fxs);
+        return fx_term(q, w, fxs);
     } else {
         const double t = fma((double)w, qsc, 0x1.8p52);
         return (unsigned long long)(__double_as_longlong(t) - 0x4338000000000000ll);
@@ -1491,43 +928,6 @@ __global__ __launch_bounds__(DG_WG) void dense_groups_kernel(const int *__restri
     for (int k = 0; k < g; ++k) groups[base + k] = make_int2((int)b, k);
 }
 
-// work list of the item kernel: the items of the bricks with dense_min or more particles
-// (one atomic per workgroup of DG_WG threads)
-__global__ __launch_bounds__(DG_WG) void dense_items_kernel(const int *__restrict__ start,
-                                                            const int *__restrict__ istart, int64_t nbk,
-                                                            int dense_min, int *__restrict__ items,
-                                                            int *__restrict__ nitems) {
-    __shared__ int wsum[DG_WG / 64];
-    __shared__ int wbase;
-    const int64_t b = (int64_t)blockIdx.x * DG_WG + threadIdx.x;
-    int g = 0, i0 = 0;
-    if (b < nbk && start[b + 1] - start[b] >= dense_min) {
-        i0 = istart[b];
-        g = istart[b + 1] - i0;
-    }
-    const int lane = lane_id(), wave = threadIdx.x >> 6;
-    int incl = g;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const int v = __shfl_up(incl, o);
-        if (lane >= o) incl += v;
-    }
-    if (lane == 63) wsum[wave] = incl;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tot = 0;
-        for (int w = 0; w < DG_WG / 64; ++w) {
-            const int v = wsum[w];
-            wsum[w] = tot;
-            tot += v;
-        }
-        wbase = tot > 0 ? atomicAdd(nitems, tot) : 0;
-    }
-    __syncthreads();
-    const int base = wbase + wsum[wave] + incl - g;
-    for (int k = 0; k < g; ++k) items[base + k] = i0 + k;
-}
-
 static constexpr int DENSE_PER = 4;  // particles per thread and round
 
 // persistent: workgroup w takes entries w, w + grid, ... of the work list (full groups are
@@ -1605,7 +1005,7 @@ __device__ __forceinline__ void dense_body(const DepArgs &A, const int2 *__restr
             if (w == 0ull) continue;
             const int ax = i % NWE, ay = (i / NWE) % NWE, az = i / (NWE * NWE);
             const int64_t idx = site_index(N, A.h, wrapi(ox + ax, N), wrapi(oy + ay, N), wrapi(oz + az, N));
-            if constexpr (FX) AccOps<ACC>::flush(A, idx, w);
+            if constexpr (FX) atomicAdd(&A.fx[idx], w);
             else atomicAdd(&A.field[idx], (float)((double)(long long)w * inv));
         }
         __syncthreads();  // the window is reused
@@ -1654,8 +1054,7 @@ __global__ __launch_bounds__(DEP_WG) void deposit_dense_fold_kernel(DepArgs A, c
 // (projections.hpp:1058-1071, whose third weight is zero), so LO = -1 and HI = 8; a vertex
 // axis spans [0, 8], a nearest-grid-point axis [0, 7].
 // Bricks with dense_min or more particles are left out (their windows stay zero) and are
-// deposited afterwards by the item kernel over a work list of their items
-// (dense_items_kernel, deposit_f32_kernel with A.dlist).
+// deposited afterwards by deposit_brick32_kernel over a work list of their groups.
 // (measured at 1024^3 with about 512 particles per brick: 4 bricks per tile and 2 particles
 // per lane in registers, at most 128 VGPRs, against 8 bricks per tile or 8 particles per
 // lane: within 5 %, the bricks' own nodes written once per line being what counted)
@@ -1877,7 +1276,7 @@ __global__ __launch_bounds__(64 * TB, 4) void deposit_tiles_c_kernel(DepArgs A, 
     const int64_t brick = (int64_t)row * NB + tile * TB + wave;  // bricks are numbered x fastest
     const int a = A.start[brick];
     int n = A.start[brick + 1] - a;
-    if (n >= dense_min) n = 0;  // the item kernel's
+    if (n >= dense_min) n = 0;  // deposit_brick32_kernel's
     TcRegs R;
     float m[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -2722,146 +2121,203 @@ __global__ void deposit_f64_kernel(Dep64Args A) {
 }
 
 // ---- brick windows
-// One workgroup per group of up to B64_MERGE items of a brick: every particle's terms (the
-// same products as deposit_f64_kernel's) go into FP64 LDS windows, one per component over the
-// component's own nodes, and the windows' non-zero nodes then go to the field, component
-// fastest, with one atomic each.
-static constexpr int B64_MERGE = 8;
-// below this many particles per brick the windows' zeroing and flush cost more than the
-// particles' own atomics
-static constexpr int64_t B64_OCC = 24;
+// One workgroup per group of consecutive particles of a brick: every particle's terms go into
+// an LDS window of the brick's nodes, all components interleaved as in the field, and the
+// window's non-zero values then go to the field with one atomic each, consecutive lanes on
+// consecutive addresses.  The window sums are FP64 (W = double), or int64 of terms quantised
+// one by one (W = unsigned long long, the fixed-point deposit).  No sort: a wave's particles
+// rarely share a node.  int64 windows of scaled sums, whose LDS atomics are twice as fast but
+// need a pass for the scale and conversions, measured equal to 25 % slower: the flush bounds
+// it, at 300-350 G atomics/s.  (FP32
+// container at 256^3, 512 particles per brick, microseconds, against sorting a brick's items
+// by cell and summing runs in registers first: scalar 247 -> 218, vector 710 -> 466, VecVec
+// 1572 -> 893, CIC-NGP 580 -> 387 / 1188 -> 692.)
+// 512 threads for six components, whose window leaves room for three workgroups per CU.
+template <int KIND> constexpr int bw_wg() { return KindC<KIND>::C == 6 ? 512 : 256; }
+template <int KIND> constexpr int bw_edge() { return BRK + 1 - KindC<KIND>::LO; }
+template <int KIND> constexpr int bw_size() {
+    return bw_edge<KIND>() * bw_edge<KIND>() * bw_edge<KIND>() * KindC<KIND>::C;
+}
 
-// first value of component COMP's window (constexpr recursion over the components before it)
-template <int KIND, int COMP> constexpr int b64_off() {
-    if constexpr (COMP == 0) return 0;
-    else {
-        constexpr int M = Comp<KIND, COMP - 1>::MASK, G = Comp<KIND, COMP - 1>::NGP;
-        return b64_off<KIND, COMP - 1>() + tc_w(M, G, 0) * tc_w(M, G, 1) * tc_w(M, G, 2);
+template <typename T> struct BwParticle {
+    int l[3];                // cell in the brick
+    T vw[3][2], lw[3][2];    // vertex and link weights
+    int llo[3];              // the first link node's offset (-1 or 0)
+};
+template <typename T> __device__ __forceinline__ void bw_weights(BwParticle<T> &P, int d, T u) {
+    P.vw[d][0] = (T)1 - u;
+    P.vw[d][1] = u;
+    const T s = u - (T)0.5;
+    if (s < 0) {
+        P.llo[d] = -1;
+        P.lw[d][0] = -s;
+        P.lw[d][1] = (T)1 - P.lw[d][0];
+    } else {
+        P.llo[d] = 0;
+        P.lw[d][1] = s;
+        P.lw[d][0] = (T)1 - P.lw[d][1];
     }
 }
-template <int KIND> constexpr int b64_size() {
-    constexpr int L = KindC<KIND>::C - 1, M = Comp<KIND, L>::MASK, G = Comp<KIND, L>::NGP;
-    return b64_off<KIND, L>() + tc_w(M, G, 0) * tc_w(M, G, 1) * tc_w(M, G, 2);
+
+// a term into the window: q w0 w1 w2, multiplied in the order of the per-particle path (FP64)
+// or the weights first (FP32); fxs: the fixed point's scale
+__device__ __forceinline__ void bw_term(double *p, double q, double w0, double w1, double w2, double) {
+    lds_add(p, q * w0 * w1 * w2);
+}
+__device__ __forceinline__ void bw_term(double *p, float q, float w0, float w1, float w2, double) {
+    lds_add(p, (double)(q * (w0 * w1 * w2)));
+}
+__device__ __forceinline__ void bw_term(unsigned long long *p, float q, float w0, float w1, float w2, double fxs) {
+    atomicAdd(p, fx_term(q, w0 * w1 * w2, fxs));
 }
 
-struct B64Particle {
-    int l[3];                     // cell in the brick
-    double vw[3][2], lw[3][2];    // vertex and link weights
-    int llo[3];                   // the first link node's offset (-1 or 0)
-};
-
-template <int KIND, int COMP>
-__device__ __forceinline__ void b64_add(double *__restrict__ win, const B64Particle &P, double q) {
-    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP;
-    constexpr int WX = tc_w(M, G, 0), WY = tc_w(M, G, 1);
+template <int KIND, int COMP, typename W, typename T>
+__device__ __forceinline__ void bw_add(W *__restrict__ win, const BwParticle<T> &P, T q, const double *fxs) {
+    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP, C = KindC<KIND>::C, E = bw_edge<KIND>();
     int b[3];
-    double w[3][2];
+    T w[3][2];
     constexpr int n[3] = {(G & 1) ? 1 : 2, (G & 2) ? 1 : 2, (G & 4) ? 1 : 2};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const bool link = (M >> d) & 1, ngp = (G >> d) & 1;
-        b[d] = P.l[d] + (link ? P.llo[d] + 1 : 0);
-        w[d][0] = ngp ? 1.0 : (link ? P.lw[d][0] : P.vw[d][0]);
-        w[d][1] = ngp ? 0.0 : (link ? P.lw[d][1] : P.vw[d][1]);
+        b[d] = P.l[d] - KindC<KIND>::LO + (link ? P.llo[d] : 0);
+        w[d][0] = ngp ? (T)1 : (link ? P.lw[d][0] : P.vw[d][0]);
+        w[d][1] = ngp ? (T)0 : (link ? P.lw[d][1] : P.vw[d][1]);
     }
-    double *o = win + b64_off<KIND, COMP>() + b[0] + WX * (b[1] + WY * b[2]);
+    W *o = win + C * (b[0] + E * (b[1] + E * b[2])) + COMP;
 #pragma unroll
     for (int k = 0; k < n[2]; ++k)
 #pragma unroll
         for (int j = 0; j < n[1]; ++j)
 #pragma unroll
-            for (int i = 0; i < n[0]; ++i) lds_add(&o[i + WX * (j + WY * k)], q * w[0][i] * w[1][j] * w[2][k]);
+            for (int i = 0; i < n[0]; ++i)
+                bw_term(&o[C * (i + E * (j + E * k))], q, w[0][i], w[1][j], w[2][k], fxs[COMP]);
 }
 
-template <int KIND, int COMP>
-__device__ __forceinline__ bool b64_node(const double *__restrict__ win, int x, int y, int z, double &v) {
-    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP;
-    constexpr int LX = -tc_nl(M, 0), LY = -tc_nl(M, 1), LZ = -tc_nl(M, 2);
-    constexpr int WX = tc_w(M, G, 0), WY = tc_w(M, G, 1), WZ = tc_w(M, G, 2);
-    x -= LX;
-    y -= LY;
-    z -= LZ;
-    if (x < 0 || x >= WX || y < 0 || y >= WY || z < 0 || z >= WZ) return false;
-    v = win[b64_off<KIND, COMP>() + x + WX * (y + WY * z)];
-    return v != 0.0;
-}
-
-template <int KIND>
-__global__ __launch_bounds__(256) void deposit_brick64_kernel(Dep64Args A, BrickIndex V) {
-    constexpr int C = KindC<KIND>::C, LO = KindC<KIND>::LO, E = BRK + 1 - LO;
-    __shared__ double win[b64_size<KIND>()];
-    BrickRange r;
-    if (!brick_range<B64_MERGE>(V, blockIdx.x, r)) return;
-    for (int i = threadIdx.x; i < b64_size<KIND>(); i += 256) win[i] = 0.0;
-    __syncthreads();
-    const int N = A.N;
-    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += 256) {
-        const int p = V.list[j];
-        const int o[3] = {r.ox, r.oy, r.oz};
-        B64Particle P;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const double t = A.s.pos[d][p] * (double)N;
-            P.l[d] = (int)floor(t) % N - o[d];  // the cell as the index took it
-            const double u = t - floor(t);
-            P.vw[d][0] = 1.0 - u;
-            P.vw[d][1] = u;
-            const double s = u - 0.5;
-            if (s < 0) {
-                P.llo[d] = -1;
-                P.lw[d][0] = -s;
-                P.lw[d][1] = 1.0 - P.lw[d][0];
-            } else {
-                P.llo[d] = 0;
-                P.lw[d][1] = s;
-                P.lw[d][0] = 1.0 - P.lw[d][1];
-            }
-        }
-        const double m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
-        if constexpr (KIND == 0) {
-            b64_add<KIND, 0>(win, P, m);
-        } else {
-            const double v[3] = {A.s.vel[0][p], A.s.vel[1][p], A.s.vel[2][p]};
-            if constexpr (C == 3) {
-                b64_add<KIND, 0>(win, P, m * v[0]);
-                b64_add<KIND, 1>(win, P, m * v[1]);
-                b64_add<KIND, 2>(win, P, m * v[2]);
-            } else {
-                b64_add<KIND, 0>(win, P, m * v[0] * v[0]);
-                b64_add<KIND, 1>(win, P, m * v[0] * v[1]);
-                b64_add<KIND, 2>(win, P, m * v[0] * v[2]);
-                b64_add<KIND, 3>(win, P, m * v[1] * v[1]);
-                b64_add<KIND, 4>(win, P, m * v[1] * v[2]);
-                b64_add<KIND, 5>(win, P, m * v[2] * v[2]);
-            }
-        }
+// a particle's terms of every component
+template <int KIND, typename W, typename T>
+__device__ __forceinline__ void bw_particle(W *__restrict__ win, const BwParticle<T> &P, T m, const T (&v)[3],
+                                            const double *fxs) {
+    if constexpr (KIND == 0) {
+        bw_add<KIND, 0>(win, P, m, fxs);
+    } else if constexpr (KindC<KIND>::C == 3) {
+        bw_add<KIND, 0>(win, P, m * v[0], fxs);
+        bw_add<KIND, 1>(win, P, m * v[1], fxs);
+        bw_add<KIND, 2>(win, P, m * v[2], fxs);
+    } else {
+        bw_add<KIND, 0>(win, P, m * v[0] * v[0], fxs);
+        bw_add<KIND, 1>(win, P, m * v[0] * v[1], fxs);
+        bw_add<KIND, 2>(win, P, m * v[0] * v[2], fxs);
+        bw_add<KIND, 3>(win, P, m * v[1] * v[1], fxs);
+        bw_add<KIND, 4>(win, P, m * v[1] * v[2], fxs);
+        bw_add<KIND, 5>(win, P, m * v[2] * v[2], fxs);
     }
-    __syncthreads();
-    for (int i = threadIdx.x; i < E * E * E * C; i += 256) {
+}
+
+// the window's non-zero values into the field
+template <int KIND, typename W, typename F>
+__device__ __forceinline__ void bw_flush(const W *__restrict__ win, F *__restrict__ field, int N, int h, int tgt,
+                                         int ox, int oy, int oz) {
+    constexpr int C = KindC<KIND>::C, LO = KindC<KIND>::LO, E = bw_edge<KIND>();
+    for (int i = threadIdx.x; i < bw_size<KIND>(); i += bw_wg<KIND>()) {
+        const W v = win[i];
+        if (v == W(0)) continue;
         const int c = i % C, n = i / C;
-        const int x = n % E + LO, y = (n / E) % E + LO, z = n / (E * E) + LO;
-        double v = 0.0;
-        bool any;
-        if constexpr (C == 1) any = b64_node<KIND, 0>(win, x, y, z, v);
-        else {
-            any = c == 0   ? b64_node<KIND, 0>(win, x, y, z, v)
-                  : c == 1 ? b64_node<KIND, 1>(win, x, y, z, v)
-                           : (c == 2 ? b64_node<KIND, 2>(win, x, y, z, v) : false);
-            if constexpr (C == 6)
-                if (c >= 3)
-                    any = c == 3   ? b64_node<KIND, 3>(win, x, y, z, v)
-                          : c == 4 ? b64_node<KIND, 4>(win, x, y, z, v)
-                                   : b64_node<KIND, 5>(win, x, y, z, v);
-        }
-        if (!any) continue;
-        int gx = r.ox + x, gy = r.oy + y, gz = r.oz + z;
-        if (A.tgt == LF2MI_DEP_PERIODIC) {
+        int gx = ox + n % E + LO, gy = oy + (n / E) % E + LO, gz = oz + n / (E * E) + LO;
+        if (tgt == LF2MI_DEP_PERIODIC) {
             gx = wrapi(gx, N);
             gy = wrapi(gy, N);
             gz = wrapi(gz, N);
         }
-        atomicAdd(&A.field[site_index(N, A.h, gx, gy, gz) * C + c], v);
+        atomicAdd(&field[site_index(N, h, gx, gy, gz) * C + c], (F)v);
     }
+}
+
+// below this many particles per brick the index, the windows' zeroing and their flush cost an
+// FP64 container more than its particles' own atomics
+static constexpr int64_t B64_OCC = 24;
+static constexpr int B64_MERGE = 8;  // items per workgroup
+
+template <int KIND>
+__global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Args A, BrickIndex V) {
+    constexpr int WG = bw_wg<KIND>();
+    __shared__ double win[bw_size<KIND>()];
+    BrickRange r;
+    if (!brick_range<B64_MERGE>(V, blockIdx.x, r)) return;
+    for (int i = threadIdx.x; i < bw_size<KIND>(); i += WG) win[i] = 0.0;
+    __syncthreads();
+    const int N = A.N;
+    const double none[6] = {};
+    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += WG) {
+        const int p = V.list[j];
+        const int o[3] = {r.ox, r.oy, r.oz};
+        BwParticle<double> P;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            // rounded like the per-particle path's: a product fused into the difference would
+            // give other weights
+            const double t = mul_rn(A.s.pos[d][p], (double)N);
+            P.l[d] = (int)floor(t) % N - o[d];  // the cell as the index took it
+            bw_weights(P, d, sub_rn(t, floor(t)));
+        }
+        const double m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
+        double v[3] = {0.0, 0.0, 0.0};
+        if constexpr (KIND > 0)
+            for (int d = 0; d < 3; ++d) v[d] = A.s.vel[d][p];
+        bw_particle<KIND>(win, P, m, v, none);
+    }
+    __syncthreads();
+    bw_flush<KIND>(win, A.field, N, A.h, A.tgt, r.ox, r.oy, r.oz);
+}
+
+// The same windows for the FP32 container, whose buckets are its bricks (any edge up to 8):
+// one workgroup per group of up to DEP_MERGE items of a brick, or a share of the groups of a
+// work list (dense_groups_kernel).  The terms' products are FP32.
+template <int KIND, typename ACC>
+__global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs A, const int2 *__restrict__ groups,
+                                                                        const int *__restrict__ ngroups) {
+    constexpr int WG = bw_wg<KIND>(), GP = DEP_MERGE * ITEM_P;
+    constexpr bool FX = sizeof(ACC) == 8;
+    using W = std::conditional_t<FX, unsigned long long, double>;
+    __shared__ W win[bw_size<KIND>()];
+    const int N = A.g.N, NB = A.g.NB, B = A.g.B;
+    auto group = [&](int b, int p0) {
+        const int p1 = min(A.start[b + 1], p0 + GP);
+        const int o[3] = {(b % NB) * B, ((b / NB) % NB) * B, (b / (NB * NB)) * B};
+        for (int i = threadIdx.x; i < bw_size<KIND>(); i += WG) win[i] = W(0);
+        __syncthreads();
+        for (int p = p0 + (int)threadIdx.x; p < p1; p += WG) {
+            int c[3];
+            decode_cell(A.s.cell[p], A.g, c[0], c[1], c[2]);
+            BwParticle<float> P;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                P.l[d] = c[d] - o[d];
+                bw_weights(P, d, A.s.off[d][p]);
+            }
+            const float m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
+            float v[3] = {0.f, 0.f, 0.f};
+            if constexpr (KIND > 0)
+                for (int d = 0; d < 3; ++d) v[d] = A.s.vel[d][p];
+            bw_particle<KIND>(win, P, m, v, A.fxs);
+        }
+        __syncthreads();
+        if constexpr (FX) bw_flush<KIND>(win, A.fx, N, A.h, A.tgt, o[0], o[1], o[2]);
+        else bw_flush<KIND>(win, A.field, N, A.h, A.tgt, o[0], o[1], o[2]);
+    };
+    if (groups) {
+        const int total = ngroups[0];
+        for (int gi = blockIdx.x; gi < total; gi += gridDim.x) {
+            const int2 gr = groups[gi];
+            group(gr.x, A.start[gr.x] + gr.y * GP);
+            __syncthreads();  // the window is reused
+        }
+        return;
+    }
+    const int it = blockIdx.x;
+    if (it >= A.istart[A.g.nbk]) return;
+    const int b = A.item_bucket[it], k = it - A.istart[b];
+    if (k % DEP_MERGE == 0) group(b, A.start[b] + k * ITEM_P);
 }
 
 struct Gkd64Args {
@@ -2979,9 +2435,9 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 // the cell as the index took it (same expression on the same position)
-                const double t = x[q][d] * (double)N;
+                const double t = mul_rn(x[q][d], (double)N);
                 c[d] = (int)floor(t) % N;
-                u[d] = t - (double)(int)floor(t);
+                u[d] = sub_rn(t, (double)(int)floor(t));
             }
             const double *f = &frc[0][c[0] - r.ox + FW * (c[1] - r.oy + FW * (c[2] - r.oz))];
             double a[3] = {0.0, 0.0, 0.0};
@@ -3266,8 +2722,6 @@ struct lf2mi_parts_s {
     int *nchunk;   // [number of chunks, claim counter]
     int2 *dgroups; // work list of the dense deposit kernel (at most cap / group + bricks)
     int *ndgroup;  // [number of entries, unused]
-    int *ditems;   // work list of the item kernel after deposit_tiles_c_kernel (items of dense bricks)
-    int *nditem;   // [number of entries, unused]
     lf2mi::BrickBuild bb;  // brick index of an F64 container
     int bricks;            // 1: kept (the lattice has a number of bricks that the scans serve)
     int *slot;             // F64: place of each uploaded particle
@@ -3429,22 +2883,10 @@ static int read_total(lf2mi_parts_s *p, hipStream_t st, int64_t *out) {
 
 static int64_t item_grid(const lf2mi_parts_s *p) { return p->g.nbk + p->np / ITEM_P + 1; }
 
-// deposit kernel for brick edge 8 or any, with or without per-particle masses
+// the brick window deposit: every brick, or (groups) those of a work list of dense ones
 template <int KIND, typename ACC>
-static void launch_deposit(const DepArgs &A, bool b8, unsigned grid, hipStream_t st) {
-    const bool pm = A.s.mass != nullptr;
-    if (KIND == 0 && !pm) {
-        if (b8) deposit_merged_kernel<ACC, 8><<<grid, DEP_WG, 0, st>>>(A);
-        else deposit_merged_kernel<ACC, 0><<<grid, DEP_WG, 0, st>>>(A);
-        return;
-    }
-    if (b8) {
-        if (pm) deposit_f32_kernel<KIND, ACC, 8, true><<<grid, DEP_WG, 0, st>>>(A);
-        else deposit_f32_kernel<KIND, ACC, 8, false><<<grid, DEP_WG, 0, st>>>(A);
-    } else {
-        if (pm) deposit_f32_kernel<KIND, ACC, 0, true><<<grid, DEP_WG, 0, st>>>(A);
-        else deposit_f32_kernel<KIND, ACC, 0, false><<<grid, DEP_WG, 0, st>>>(A);
-    }
+static void launch_bricks(const DepArgs &A, unsigned grid, const int2 *groups, const int *ngroups, hipStream_t st) {
+    deposit_brick32_kernel<KIND, ACC><<<grid, bw_wg<KIND>(), 0, st>>>(A, groups, ngroups);
 }
 
 // bricks with fewer particles are deposited by deposit_tiles_kernel, the others by
@@ -3499,15 +2941,18 @@ static int launch_tiles_dense(lf2mi_parts_s *p, const DepArgs &A, bool overwrite
     return LF2MI_OK;
 }
 
-// the other kinds (and the scalar kind with per-particle masses) into a periodic target
-// with 8^3 bricks
+// the other kinds (and the scalar kind with per-particle masses) into a periodic target with
+// 8^3 bricks, four to a tile, where the tiles beat the brick windows: large lattices and, from
+// 192, sparse ones (microseconds, tiles / windows, at 1 and 1/4 particle per cell: vector
+// 160^3 149 / 119 and 106 / 99, 256^3 500 / 466 and 336 / 384, 512^3 3519 / 3643 and 2273 / 3008;
+// VecVec 256^3 977 / 893 and 659 / 664, 512^3 7135 / 7074 and 4573 / 5111)
 static bool tiles_c_path(const lf2mi_parts_s *p, int kind, int target, bool pm) {
     return (kind != LF2MI_PROJ_SCALAR || pm) && target == LF2MI_DEP_PERIODIC && p->g.B == 8 &&
-           p->g.NB % TC_TB == 0 && p->N <= 1024;
+           p->g.NB % TC_TB == 0 && p->N <= 1024 && p->N >= 192 && (p->N >= 512 || p->np < 256 * p->g.nbk);
 }
 
 // the shell buffer of deposit_tiles_c_kernel (grown on demand), its layout, the fold and the
-// item deposit of the dense bricks
+// window deposit of the dense bricks
 template <int KIND>
 static int launch_tiles_c(lf2mi_parts_s *p, DepArgs A, bool pm, bool overwrite, hipStream_t st) {
     constexpr int C = KindC<KIND>::C, TB = TC_TB;
@@ -3577,13 +3022,10 @@ static int launch_tiles_c(lf2mi_parts_s *p, DepArgs A, bool pm, bool overwrite, 
         fold_edges_kernel<C><<<grid1(edges), 256, 0, st>>>(A.field, (int)N, A.h, (int)NB, F, shell, edges);
         LF2MI_LAUNCHED();
     }
-    if (int rc = fill_int(p->nditem, 2, 0, st)) return rc;
-    dense_items_kernel<<<grid1(p->g.nbk, DG_WG), DG_WG, 0, st>>>(p->bstart, p->istart, p->g.nbk, DENSE_MIN, p->ditems,
-                                                                 p->nditem);
+    if (int rc = fill_int(p->ndgroup, 2, 0, st)) return rc;
+    dense_groups_kernel<<<grid1(p->g.nbk, DG_WG), DG_WG, 0, st>>>(p->bstart, p->g.nbk, DENSE_MIN, p->dgroups, p->ndgroup);
     LF2MI_LAUNCHED();
-    A.dlist = p->ditems;
-    A.dcount = p->nditem;
-    launch_deposit<KIND, float>(A, true, (unsigned)std::min<int64_t>(item_grid(p), DENSE_WORKERS), st);
+    launch_bricks<KIND, float>(A, (unsigned)std::min<int64_t>(item_grid(p), DENSE_WORKERS), p->dgroups, p->ndgroup, st);
     LF2MI_LAUNCHED();
     return LF2MI_OK;
 }
@@ -3758,8 +3200,6 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
         A((void **)&p->nchunk, 2 * sizeof(int));
         A((void **)&p->dgroups, (size_t)(cap / (DEP_MERGE * ITEM_P) + p->g.nbk + 1) * sizeof(int2));
         A((void **)&p->ndgroup, 2 * sizeof(int));
-        A((void **)&p->ditems, (size_t)(p->g.nbk + cap / ITEM_P + 1) * sizeof(int));
-        A((void **)&p->nditem, 2 * sizeof(int));
     } else {
         Soa64 &s = p->b64;
         A((void **)&s.cell, cap * sizeof(int32_t));
@@ -4392,11 +3832,11 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
             const BrickIndex V = brick_view(p->bb, N);
             const unsigned gb = (unsigned)brick_items(V.nbk, p->np);
             switch (kind) {
-                case 0: deposit_brick64_kernel<0><<<gb, 256, 0, st>>>(A, V); break;
-                case 1: deposit_brick64_kernel<1><<<gb, 256, 0, st>>>(A, V); break;
-                case 2: deposit_brick64_kernel<2><<<gb, 256, 0, st>>>(A, V); break;
-                case 3: deposit_brick64_kernel<3><<<gb, 256, 0, st>>>(A, V); break;
-                default: deposit_brick64_kernel<4><<<gb, 256, 0, st>>>(A, V); break;
+                case 0: deposit_brick64_kernel<0><<<gb, bw_wg<0>(), 0, st>>>(A, V); break;
+                case 1: deposit_brick64_kernel<1><<<gb, bw_wg<1>(), 0, st>>>(A, V); break;
+                case 2: deposit_brick64_kernel<2><<<gb, bw_wg<2>(), 0, st>>>(A, V); break;
+                case 3: deposit_brick64_kernel<3><<<gb, bw_wg<3>(), 0, st>>>(A, V); break;
+                default: deposit_brick64_kernel<4><<<gb, bw_wg<4>(), 0, st>>>(A, V); break;
             }
             LF2MI_LAUNCHED();
             return LF2MI_OK;
@@ -4487,17 +3927,16 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
                                                    "deposit_f32_vecvec_fixed64", "deposit_f32_vector_ngp_fixed64",
                                                    "deposit_f32_symtensor_ngp_fixed64"};
             LF2MI_PROF(namesfx[kind], st);
-            const bool b8 = p->g.B == 8;
             if (tiles_path(p, kind, target, pm)) {
                 // the fixed-point buffer starts cleared, so its interior can be stored
                 if (int rc = launch_tiles_dense<unsigned long long>(p, A, true, st)) return rc;
             } else {
                 switch (kind) {
-                    case 0: launch_deposit<0, unsigned long long>(A, b8, g, st); break;
-                    case 1: launch_deposit<1, unsigned long long>(A, b8, g, st); break;
-                    case 2: launch_deposit<2, unsigned long long>(A, b8, g, st); break;
-                    case 3: launch_deposit<3, unsigned long long>(A, b8, g, st); break;
-                    default: launch_deposit<4, unsigned long long>(A, b8, g, st); break;
+                    case 0: launch_bricks<0, unsigned long long>(A, g, nullptr, nullptr, st); break;
+                    case 1: launch_bricks<1, unsigned long long>(A, g, nullptr, nullptr, st); break;
+                    case 2: launch_bricks<2, unsigned long long>(A, g, nullptr, nullptr, st); break;
+                    case 3: launch_bricks<3, unsigned long long>(A, g, nullptr, nullptr, st); break;
+                    default: launch_bricks<4, unsigned long long>(A, g, nullptr, nullptr, st); break;
                 }
             }
             LF2MI_LAUNCHED();
@@ -4517,7 +3956,6 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
     static const char *const names32[5] = {"deposit_f32_scalar", "deposit_f32_vector", "deposit_f32_vecvec",
                                            "deposit_f32_vector_ngp", "deposit_f32_symtensor_ngp"};
     LF2MI_PROF(names32[kind], st);
-    const bool b8 = p->g.B == 8;
     if (tiles_path(p, kind, target, pm)) return launch_tiles_dense<float>(p, A, overwrite, st);
     if (tiles_c_path(p, kind, target, pm)) {
         switch (kind) {
@@ -4529,11 +3967,11 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
         }
     }
     switch (kind) {
-        case 0: launch_deposit<0, float>(A, b8, g, st); break;
-        case 1: launch_deposit<1, float>(A, b8, g, st); break;
-        case 2: launch_deposit<2, float>(A, b8, g, st); break;
-        case 3: launch_deposit<3, float>(A, b8, g, st); break;
-        default: launch_deposit<4, float>(A, b8, g, st); break;
+        case 0: launch_bricks<0, float>(A, g, nullptr, nullptr, st); break;
+        case 1: launch_bricks<1, float>(A, g, nullptr, nullptr, st); break;
+        case 2: launch_bricks<2, float>(A, g, nullptr, nullptr, st); break;
+        case 3: launch_bricks<3, float>(A, g, nullptr, nullptr, st); break;
+        default: launch_bricks<4, float>(A, g, nullptr, nullptr, st); break;
     }
     LF2MI_LAUNCHED();
     return LF2MI_OK;
