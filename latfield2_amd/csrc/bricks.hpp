@@ -34,12 +34,37 @@ struct BrickIndex {
     const int *list;      // particle numbers, brick by brick
 };
 
+// the arrays of a scan of the brick counts (brick_scan)
+struct BrickScan {
+    int *count;                  // cleared
+    int *bsum;                   // scratch, 3 per block
+    int *start, *istart, *item;
+    int *cursor;                 // copy of the starts, or null
+    int2 *group;                 // (brick, k): particles [k group_p, (k + 1) group_p) of a brick with
+    int *ngroup;                 // dense_min or more, and their number; null without
+    int dense_min, group_p;
+    // runs of sparse bricks along x: (first particle, past the last, first brick, bricks), at
+    // most chunk_w bricks of a row with 1 to sparse_max - 1 particles each; null without
+    int4 *chunk;
+    int *nchunk;                 // their number, and a counter of claims (cleared)
+    int NB, sparse_max, chunk_w;
+};
+
 // writable side, with the scratch of the build
 struct BrickBuild {
     int *start, *istart, *item, *list;
     int *count;           // [nbk], zero between builds
     int *rank;            // [np] place of a particle in its brick
-    int *bsum;            // [2 * blocks] totals of the scan's blocks
+    int *bsum;            // [3 * blocks] totals of the scan's blocks
+    BrickScan scan() const {
+        BrickScan S{};
+        S.count = count;
+        S.bsum = bsum;
+        S.start = start;
+        S.istart = istart;
+        S.item = item;
+        return S;
+    }
 };
 
 __device__ __forceinline__ void brick_decode(int cell, int N, int lgN, int &x, int &y, int &z) {
@@ -91,31 +116,30 @@ __device__ __forceinline__ int wave_scan(int v) {
     }
     return v;
 }
-// exclusive scans of two values over a workgroup of WG threads; totals in ta, tb
-template <int WG>
-__device__ __forceinline__ void block_scan2(int &a, int &b, int &ta, int &tb, int *sh) {
+// exclusive scans of K values over a workgroup of WG threads; totals in tot
+template <int WG, int K>
+__device__ __forceinline__ void block_scan(int (&v)[K], int (&tot)[K], int *sh) {
     const int lane = __lane_id(), wave = threadIdx.x >> 6;
-    const int ia = wave_scan(a), ib = wave_scan(b);
-    if (lane == 63) {
-        sh[wave] = ia;
-        sh[WG / 64 + wave] = ib;
-    }
-    __syncthreads();
-    int pa = 0, pb = 0;
-    ta = tb = 0;
+    int incl[K];
 #pragma unroll
-    for (int w = 0; w < WG / 64; ++w) {
-        const int va = sh[w], vb = sh[WG / 64 + w];
-        if (w < wave) {
-            pa += va;
-            pb += vb;
-        }
-        ta += va;
-        tb += vb;
+    for (int k = 0; k < K; ++k) {
+        incl[k] = wave_scan(v[k]);
+        if (lane == 63) sh[k * (WG / 64) + wave] = incl[k];
     }
     __syncthreads();
-    a = pa + ia - a;
-    b = pb + ib - b;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        int before = 0, t = 0;
+#pragma unroll
+        for (int w = 0; w < WG / 64; ++w) {
+            const int x = sh[k * (WG / 64) + w];
+            if (w < wave) before += x;
+            t += x;
+        }
+        tot[k] = t;
+        v[k] = before + incl[k] - v[k];
+    }
+    __syncthreads();
 }
 
 // ---- scans of the brick counts
@@ -123,74 +147,138 @@ __device__ __forceinline__ void block_scan2(int &a, int &b, int &ta, int &tb, in
 // the first kernel leaves each block's totals and every block of the second sums those before
 // its own (at most 4096 blocks).  The second kernel writes starts, item starts and the
 // item -> brick table (threads over the block's items, whose brick a binary search in LDS
-// finds: a brick of thousands of items is written by the whole block) and clears the counts.
+// finds: a brick of thousands of items is written by the whole block, where one thread per
+// brick took 106 us at 512^3 with dense blobs) and clears the counts.  A container that
+// scatters its particles also gets a copy of the starts to claim places from and a list of the
+// dense bricks' groups, and chunks of sparse bricks.  (Five launches, a list kernel for each of
+// the two and four fills before: 51 us a step at 256^3, 190 us at 512^3 with dense blobs.)
 static constexpr int BS_WG = 256, BS_PER = 4, BS_CHUNK = BS_WG * BS_PER;
 
-static __global__ __launch_bounds__(BS_WG) void brick_sums_kernel(const int *__restrict__ count, int n,
-                                                                  int *__restrict__ bsum) {
-    __shared__ int sh[2 * BS_WG / 64];
-    const int base = blockIdx.x * BS_CHUNK + threadIdx.x * BS_PER;
-    int a = 0, b = 0, ta, tb;
-#pragma unroll
-    for (int k = 0; k < BS_PER; ++k) {
-        const int c = base + k < n ? count[base + k] : 0;
-        a += c;
-        b += (c + BRK_ITEM - 1) / BRK_ITEM;
-    }
-    block_scan2<BS_WG>(a, b, ta, tb, sh);
-    if (threadIdx.x == 0) {
-        bsum[2 * blockIdx.x] = ta;
-        bsum[2 * blockIdx.x + 1] = tb;
-    }
+__device__ __forceinline__ void brick_sizes(const BrickScan &S, int c, int (&v)[3]) {
+    v[0] = c;
+    v[1] = (c + BRK_ITEM - 1) / BRK_ITEM;
+    v[2] = S.group && c >= S.dense_min ? (c + S.group_p - 1) / S.group_p : 0;
 }
 
-static __global__ __launch_bounds__(BS_WG) void brick_starts_kernel(int *__restrict__ count, int n,
-                                                                    const int *__restrict__ bsum,
-                                                                    int *__restrict__ start, int *__restrict__ istart,
-                                                                    int *__restrict__ item) {
-    __shared__ int sh[2 * BS_WG / 64];
-    __shared__ int si[BS_CHUNK + 1];
+static __global__ __launch_bounds__(BS_WG) void brick_sums_kernel(BrickScan S, int n) {
+    __shared__ int sh[3 * BS_WG / 64];
     const int base = blockIdx.x * BS_CHUNK + threadIdx.x * BS_PER;
-    int c[BS_PER], a = 0, b = 0, ta, tb;
+    int a[3] = {0, 0, 0}, tot[3];
 #pragma unroll
     for (int k = 0; k < BS_PER; ++k) {
-        c[k] = base + k < n ? count[base + k] : 0;
-        a += c[k];
-        b += (c[k] + BRK_ITEM - 1) / BRK_ITEM;
+        int v[3];
+        brick_sizes(S, base + k < n ? S.count[base + k] : 0, v);
+        for (int q = 0; q < 3; ++q) a[q] += v[q];
     }
-    int oa = 0, ob = 0;  // totals of the blocks before this one
-    if (blockIdx.x > 0) {
-        int pa = 0, pb = 0;
-        for (int k = threadIdx.x; k < (int)blockIdx.x; k += BS_WG) {
-            pa += bsum[2 * k];
-            pb += bsum[2 * k + 1];
+    block_scan<BS_WG>(a, tot, sh);
+    if (S.chunk && blockIdx.x == 0 && threadIdx.x == 0) S.nchunk[0] = 0;
+    if (threadIdx.x < 3) S.bsum[3 * blockIdx.x + threadIdx.x] = threadIdx.x == 0 ? tot[0] : (threadIdx.x == 1 ? tot[1] : tot[2]);
+}
+
+// inclusive maxima over a workgroup: on entry the largest of the thread's own values, on exit
+// the largest of all threads before it (0 for none)
+template <int WG> __device__ __forceinline__ int block_max_before(int v, int *sh) {
+    const int lane = __lane_id(), wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(v, o);
+        if (lane >= o) v = max(v, y);
+    }
+    if (lane == 63) sh[wave] = v;
+    __syncthreads();
+    int before = 0;
+    for (int w = 0; w < wave; ++w) before = max(before, sh[w]);
+    const int up = __shfl_up(v, 1);
+    __syncthreads();
+    return lane > 0 ? max(before, up) : before;
+}
+
+static __global__ __launch_bounds__(BS_WG) void brick_starts_kernel(BrickScan S, int n) {
+    __shared__ int sh[4 * BS_WG / 64];
+    __shared__ int si[BS_CHUNK + 1];          // item starts
+    __shared__ int ss[BS_CHUNK + 1];          // starts
+    __shared__ unsigned char tk[BS_CHUNK];    // 1: a sparse brick, 2: one at the start of a row
+    __shared__ int cbase;
+    const int base = blockIdx.x * BS_CHUNK + threadIdx.x * BS_PER, l0 = threadIdx.x * BS_PER;
+    int c[BS_PER], a[4] = {0, 0, 0, 0}, tot[4];
+    int first[BS_PER], last = 0;  // first brick of the run a brick belongs to, 1-based
+#pragma unroll
+    for (int k = 0; k < BS_PER; ++k) {
+        int v[3];
+        c[k] = base + k < n ? S.count[base + k] : 0;
+        brick_sizes(S, c[k], v);
+        for (int q = 0; q < 3; ++q) a[q] += v[q];
+        if (S.chunk) {
+            const bool take = c[k] > 0 && c[k] < S.sparse_max, row = (base + k) % S.NB == 0;
+            tk[l0 + k] = take ? (row ? 2 : 1) : 0;
+            // a run begins after a brick that is not sparse, and with a row or the block
+            if (!take) last = l0 + k + 2;
+            else if (row || l0 + k == 0) last = l0 + k + 1;
+            first[k] = last;
         }
-        block_scan2<BS_WG>(pa, pb, oa, ob, sh);
     }
-    block_scan2<BS_WG>(a, b, ta, tb, sh);
-    a += oa;
-    b += ob;
+    unsigned heads = 0u;  // bricks that begin a chunk
+    if (S.chunk) {
+        const int before = block_max_before<BS_WG>(last, sh);
+#pragma unroll
+        for (int k = 0; k < BS_PER; ++k)
+            if (c[k] > 0 && c[k] < S.sparse_max) {
+                const int pos = l0 + k + 1 - max(first[k], before);
+                if (pos % S.chunk_w == 0) heads |= 1u << k;
+            }
+        a[3] = __popc(heads);
+    }
+    int off[3] = {0, 0, 0};  // totals of the blocks before this one
+    if (blockIdx.x > 0) {
+        int p[3] = {0, 0, 0};
+        for (int k = threadIdx.x; k < (int)blockIdx.x; k += BS_WG)
+            for (int q = 0; q < 3; ++q) p[q] += S.bsum[3 * k + q];
+        block_scan<BS_WG>(p, off, sh);
+    }
+    block_scan<BS_WG>(a, tot, sh);
+    for (int q = 0; q < 3; ++q) a[q] += off[q];
 #pragma unroll
     for (int k = 0; k < BS_PER; ++k) {
         const int i = base + k;
-        si[threadIdx.x * BS_PER + k] = b;
+        si[l0 + k] = a[1];
+        ss[l0 + k] = a[0];
+        int v[3];
+        brick_sizes(S, c[k], v);
         if (i < n) {
-            start[i] = a;
-            istart[i] = b;
-            count[i] = 0;
+            S.start[i] = a[0];
+            S.istart[i] = a[1];
+            S.count[i] = 0;
+            if (S.cursor) S.cursor[i] = a[0];
+            for (int g = 0; g < v[2]; ++g) S.group[a[2] + g] = make_int2(i, g);
         }
-        a += c[k];
-        b += (c[k] + BRK_ITEM - 1) / BRK_ITEM;
+        for (int q = 0; q < 3; ++q) a[q] += v[q];
     }
     if (threadIdx.x == 0) {
-        si[BS_CHUNK] = ob + tb;
+        si[BS_CHUNK] = off[1] + tot[1];
+        ss[BS_CHUNK] = off[0] + tot[0];
+        if (S.chunk) {
+            if (gridDim.x == 1) S.nchunk[0] = tot[3];
+            cbase = gridDim.x == 1 ? 0 : (tot[3] ? atomicAdd(&S.nchunk[0], tot[3]) : 0);
+        }
         if (blockIdx.x + 1 == gridDim.x) {
-            start[n] = oa + ta;
-            istart[n] = ob + tb;
+            S.start[n] = off[0] + tot[0];
+            S.istart[n] = off[1] + tot[1];
+            if (S.group) S.ngroup[0] = off[2] + tot[2];
+            if (S.chunk) S.nchunk[1] = 0;
         }
     }
     __syncthreads();
-    for (int i = ob + (int)threadIdx.x; i < ob + tb; i += BS_WG) {
+    if (S.chunk) {
+        int at = cbase + a[3];
+#pragma unroll
+        for (int k = 0; k < BS_PER; ++k) {
+            if (!((heads >> k) & 1u)) continue;
+            int e = l0 + k + 1;
+            while (e < BS_CHUNK && e < l0 + k + S.chunk_w && tk[e] == 1) ++e;
+            S.chunk[at++] = make_int4(ss[l0 + k], ss[e], base + k, e - (l0 + k));
+        }
+    }
+    for (int i = off[1] + (int)threadIdx.x; i < off[1] + tot[1]; i += BS_WG) {
         int lo = 0, hi = BS_CHUNK;  // the last brick whose first item is <= i
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
@@ -198,20 +286,19 @@ static __global__ __launch_bounds__(BS_WG) void brick_starts_kernel(int *__restr
             else hi = mid;
         }
         // bricks without items share the next brick's start: the last of them is the owner
-        item[i] = blockIdx.x * BS_CHUNK + lo;
+        S.item[i] = blockIdx.x * BS_CHUNK + lo;
     }
 }
 
 inline int brick_blocks(int64_t nbk) { return (int)((nbk + BS_CHUNK - 1) / BS_CHUNK); }
 
-// starts, items and (cleared) counts of `n` bricks
-inline int brick_scan(int *count, int n, int *bsum, int *start, int *istart, int *item, hipStream_t st) {
+inline int brick_scan(const BrickScan &S, int n, hipStream_t st) {
     const int nb = brick_blocks(n);
     if (nb > 1) {
-        brick_sums_kernel<<<nb, BS_WG, 0, st>>>(count, n, bsum);
+        brick_sums_kernel<<<nb, BS_WG, 0, st>>>(S, n);
         LF2MI_LAUNCHED();
     }
-    brick_starts_kernel<<<nb, BS_WG, 0, st>>>(count, n, bsum, start, istart, item);
+    brick_starts_kernel<<<nb, BS_WG, 0, st>>>(S, n);
     LF2MI_LAUNCHED();
     return LF2MI_OK;
 }
@@ -240,7 +327,7 @@ static __global__ __launch_bounds__(256) void brick_list_kernel(int64_t np, cons
 // the index of the particles whose cells are in `cell` and whose places are in B.rank already
 inline int brick_build_ranked(const int32_t *cell, int64_t np, int N, const BrickBuild &B, hipStream_t st) {
     const int NB = (N + BRK - 1) / BRK, lgN = is_pow2(N) ? __builtin_ctz((unsigned)N) : -1;
-    if (int rc = brick_scan(B.count, NB * NB * NB, B.bsum, B.start, B.istart, B.item, st)) return rc;
+    if (int rc = brick_scan(B.scan(), NB * NB * NB, st)) return rc;
     brick_list_kernel<<<blocks_for(np, 256), 256, 0, st>>>(np, cell, N, NB, lgN, B.start, B.rank, B.list);
     LF2MI_LAUNCHED();
     return LF2MI_OK;

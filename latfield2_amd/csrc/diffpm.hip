@@ -516,7 +516,7 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     if (!rc) rc = dp_malloc(&m->resid, fb);
     const int64_t nb = (N + BRK - 1) / BRK, nbk = nb * nb * nb, items = brick_items(nbk, np);
     // starts, item starts, counts, block totals, items, list, places
-    m->index_bytes = sizeof(int) * (size_t)(2 * (nbk + 1) + nbk + 2 * brick_blocks(nbk) + items + 2 * np);
+    m->index_bytes = sizeof(int) * (size_t)(2 * (nbk + 1) + nbk + 3 * brick_blocks(nbk) + items + 2 * np);
     if (!rc) rc = dp_malloc(&m->index_mem, m->index_bytes);
     if (!rc) {
         int *q = (int *)m->index_mem;
@@ -528,7 +528,7 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
         m->bricks.start = take(nbk + 1);
         m->bricks.istart = take(nbk + 1);
         m->bricks.count = take(nbk);
-        m->bricks.bsum = take(2 * brick_blocks(nbk));
+        m->bricks.bsum = take(3 * brick_blocks(nbk));
         m->bricks.item = take(items);
         m->bricks.list = take(np);
         m->bricks.rank = take(np);
