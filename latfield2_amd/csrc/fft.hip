@@ -253,6 +253,7 @@ template <typename T> struct StridedArgs {
     int64_t in_es, out_es;      // stride between elements of a line (transform axis)
     int64_t in_bs, out_bs;      // stride between batches (the other row axis)
     int ncols;                  // valid columns per row
+    int remap;                  // rows that are no whole lines: see the kernel
     const cplx<T> *tw;
     // Green fusion (MODE 1): element (col, e, batch) has kx = col / C, ky = e, kz = batch
     const double *green_s;      // s[k] = N^2 (2 - 2 cos(2 pi k / N)) = 4 N^2 sin^2(pi k / N), FP64 table
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(WG) void fft_strided_kernel(StridedArgs<T> A) {
     extern __shared__ unsigned char smem_raw[];
     V *lds = reinterpret_cast<V *>(smem_raw);
     int bx = blockIdx.x, by = blockIdx.y;
-    if constexpr (L * (int)sizeof(V) < 128) {
+    if (L * (int)sizeof(V) < 128 || A.remap) {
         // a tile row is part of a 128-byte line whose rest belongs to the next tiles: blocks are
         // dispatched round-robin over the 8 XCDs, so give each XCD a contiguous range of tiles
         // and the whole line one L2
@@ -391,6 +392,25 @@ __global__ __launch_bounds__(WG) void fft_x_r2c_kernel(XArgs<T> A) {
     tile_fft_io<T, N, L, ES, WG, -1, 1, false, true>(lds, A.tw, rload, lstore);
     // split the two half spectra: A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = -i (Z[k] - conj Z[N-k]) / 2
     constexpr int H = N / 2 + 1;
+    if constexpr (CC == 1 && N < 256) {
+        // short rows: the (row, kx) items spread over all threads (a row of N/2 + 1 values
+        // leaves half to three quarters of them idle: x pass 9.7 -> 6.4 us at 64^3, 10.8 -> 9.4 at
+        // 128^3, FP64 at 32^3 6.8 -> 5.2; from 256 the rows one by one are as fast or faster)
+        for (int i = threadIdx.x; i < 2 * L * H; i += WG) {
+            const int rr = i / H, kx = i - rr * H, p = rr >> 1, ab = rr & 1;
+            const int64_t pr = pair0 + p;
+            if (pr >= npairs) break;
+            const V zk = lds[kx * ES + p];
+            const V zm = lds[(kx == 0 ? 0 : N - kx) * ES + p];
+            V r;
+            r.x = (T)0.5 * (ab == 0 ? zk.x + zm.x : zk.y + zm.y);
+            r.y = (T)0.5 * (ab == 0 ? zk.y - zm.y : zm.x - zk.x);
+            const int row = (int)(2 * pr) + ab;
+            const int y = row % N, z = row / N;
+            A.kout[A.k_col0 + (int64_t)z * A.k_s1 + (int64_t)y * A.k_s2 + kx] = r;
+        }
+        return;
+    }
     if constexpr (CC == 1) {
         // one output row at a time (its base address uniform), threads along kx
         for (int rr = 0; rr < 2 * L; ++rr) {
@@ -693,8 +713,12 @@ template <> struct Tune<float> {
     template <int N> static constexpr int x_L() { return N >= 512 ? 4 : (N >= 128 ? 12 : 24); }
     template <int N> static constexpr int x_L_max() { return N >= 512 ? 6 : (N >= 128 ? 12 : 24); }
     // x pass workgroup: 512 threads at N = 1024 (1024^3 forward / backward x passes 2.87 / 2.63
-    // -> 2.41 / 2.35 ms for one component, 21.6 / 23.1 -> 20.6 / 20.9 ms for six)
-    template <int N> static constexpr int x_WG() { return N >= 1024 ? 512 : 256; }
+    // -> 2.41 / 2.35 ms for one component, 21.6 / 23.1 -> 20.6 / 20.9 ms for six); at 256 and 512
+    // one radix-8 butterfly of the tile per thread, so that no round is half empty (forward
+    // transform, 512^3 six components 5.57 -> 5.08 ms, 256^3 three 318 -> 297 us, six 688 -> 648)
+    template <int N, int L> static constexpr int x_WG() {
+        return N >= 1024 ? 512 : (N == 256 || N == 512 ? L * N / 8 : 256);
+    }
     // C2C z pass: 128-byte column reads (padded LDS tile N x (L+1), up to 136 KB at 1024)
     template <int N> static constexpr int c2c_z_L() { return 16; }
     // C2C x pass: lines per tile (8 at N >= 512: 1.65 -> 1.55 ms forward at 512^3)
@@ -706,7 +730,7 @@ template <> struct Tune<double> {
     template <int N> static constexpr int green_L() { return N >= 1024 ? 4 : 8; }
     template <int N> static constexpr int x_L() { return N >= 512 ? 3 : (N >= 128 ? 6 : 12); }
     template <int N> static constexpr int x_L_max() { return N >= 512 ? 3 : (N >= 128 ? 6 : 12); }
-    template <int N> static constexpr int x_WG() { return 256; }
+    template <int N, int L> static constexpr int x_WG() { return 256; }
     template <int N> static constexpr int c2c_z_L() { return 8; }
     template <int N> static constexpr int c2c_x_L() { return x_L_max<N>(); }
 };
@@ -730,7 +754,16 @@ struct lf2mi_fft_plan_s {
 namespace lf2mi {
 
 template <typename T, int N>
-static int launch_strided(const StridedArgs<T> &A, int S, int mode, int nbatch, hipStream_t st) {
+static int launch_strided(StridedArgs<T> A, int S, int mode, int nbatch, hipStream_t st) {
+    // Tiles whose rows are not whole 128-byte lines share lines with their neighbours: as with
+    // the narrow tiles, give each XCD a contiguous range of them, so that the parts of a line
+    // meet in one L2 (512^3 forward, y pass into the unpadded k-field: one component 0.92 ->
+    // 0.89 ms for the whole transform, three 3.04 -> 2.66, six 6.47 -> 5.57; FP64 one component
+    // 1.97 -> 1.75).  For rows only read so, below 512, where the field stays in the last-level
+    // cache (256^3 backward 90 -> 81 us; at 512^3 0.78 -> 0.82 ms with it).
+    const int64_t line = 128 / (int64_t)sizeof(cplx<T>);
+    A.remap = (A.out_es | A.out_bs | A.out_col0) % line != 0 ||
+              (N < 512 && (A.in_es | A.in_bs | A.in_col0) % line != 0);
     constexpr int WG = Tune<T>::WG;
     constexpr int L = Tune<T>::template strided_L<N>();
     constexpr int LG = Tune<T>::template green_L<N>();
@@ -759,7 +792,7 @@ static int launch_strided(const StridedArgs<T> &A, int S, int mode, int nbatch, 
 
 template <typename T, int N, int L>
 static int launch_x_tile(const XArgs<T> &A, int S, hipStream_t st) {
-    constexpr int WG = Tune<T>::template x_WG<N>();
+    constexpr int WG = Tune<T>::template x_WG<N, L>();
     const int P = L / A.C;
     const int64_t npairs = (int64_t)N * N / 2;
     const unsigned grid = (unsigned)((npairs + P - 1) / P);
