@@ -16,9 +16,10 @@
 //                        phi-bar = sum_d D_d F-bar_d          (D_d is antisymmetric)
 //                        rho-bar = G phi-bar                  (G is symmetric: the same FFT solve)
 //                        lambda_x += q N grad_X interp(rho-bar)(X_p)   (deposit weights)
-// Particles keep their order so gradients stay attached to them; a brick index (bricks.hpp)
-// of the state at hand lets the deposits and gathers work brick by brick.  The starting state of every step is checkpointed in HBM and the fields are recomputed
-// on the way back.  Positions are kept as (cell, offset in cell units) and re-anchored
+// A particle keeps its place in all states, so gradients stay attached to it; a brick index
+// (bricks.hpp) of every state lets the deposits and gathers work brick by brick.  The starting
+// state of every step is checkpointed in HBM and the fields are recomputed on the way back.
+// Positions are kept as (cell, offset in cell units) and re-anchored
 // in FP64 after each drift, as in the PM step.  T = float or double selects the
 // precision of the whole path (fields, FFTs, offsets, velocities, adjoints).
 #include <algorithm>
@@ -78,27 +79,73 @@ template <typename T> __device__ __forceinline__ void anchor(double X, int N, in
 
 template <typename T> __device__ __forceinline__ T wsel(int i, T u) { return i ? u : (T)1 - u; }
 
-template <typename T, typename I>
-__global__ void dp_init_kernel(DpState<T> s, const I *__restrict__ pos, const I *__restrict__ vel) {
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
-        int c[3];
-        for (int d = 0; d < 3; ++d) {
-            T o;
-            anchor<T>(mul_nc((double)pos[3 * p + d], (double)s.N), s.N, c[d], o);
-            s.off[d][p] = o;
-            s.vel[d][p] = vel ? (T)vel[3 * p + d] : (T)0;
-        }
-        s.cell[p] = c[0] + s.N * (c[1] + s.N * c[2]);
+// clears up to two fields on the side of a launch that covers the chip: beside a small mesh the
+// launches count (32^3: about 3 us each), beside a large one the clears hide behind the
+// particles' latency
+template <typename T> struct DpClear {
+    T *a, *b;  // may be null
+    int64_t n;
+};
+template <typename T> __device__ __forceinline__ void dp_clear(const DpClear<T> &c) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < c.n; i += stride) {
+        if (c.a) c.a[i] = (T)0;
+        if (c.b) c.b[i] = (T)0;
     }
 }
 
-template <typename T, typename I> __global__ void dp_state_out_kernel(DpState<T> s, I *__restrict__ pos, I *__restrict__ vel) {
+// The states hold the particles in the brick order of the initial positions (slot[i]: the place
+// of the caller's particle i): the particles move a few cells over a run, so the brick lists of
+// every state read memory nearly in order, whatever order the caller's arrays have (128^3 FP32
+// lattice, 10 steps: adjoint 86 -> 68 us a launch, density 41 -> 33; 64^3 in random order: the
+// whole evaluation 7.0 -> 1.6 ms against particles in the caller's order with global atomics).
+// Here: the initial cells and the particles' places in their bricks.
+template <typename T, typename I>
+__global__ __launch_bounds__(DP_WG) void dp_cells_kernel(int64_t np, const I *__restrict__ pos, int N, int NB,
+                                                         int *__restrict__ count, int *__restrict__ rank, DpClear<T> clear,
+                                                         double *__restrict__ loss) {
+    const int64_t p = (int64_t)blockIdx.x * DP_WG + threadIdx.x;
+    const bool in = p < np;
+    int c[3] = {0, 0, 0};
+    if (in)
+        for (int d = 0; d < 3; ++d) {
+            T o;
+            anchor<T>(mul_nc((double)pos[3 * p + d], (double)N), N, c[d], o);
+        }
+    const int r = brick_rank(count, brick_of(c[0], c[1], c[2], NB), in);
+    if (in) rank[p] = r;
+    if (p == 0) *loss = 0.0;
+    dp_clear(clear);
+}
+
+template <typename T, typename I>
+__global__ void dp_init_kernel(DpState<T> s, const I *__restrict__ pos, const I *__restrict__ vel, int NB,
+                               const int *__restrict__ start, const int *__restrict__ rank, int *__restrict__ slot,
+                               int *__restrict__ list) {
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
         int c[3];
-        decode(s.cell[p], s.N, c);
+        T o[3];
+        for (int d = 0; d < 3; ++d) anchor<T>(mul_nc((double)pos[3 * p + d], (double)s.N), s.N, c[d], o[d]);
+        const int j = start[brick_of(c[0], c[1], c[2], NB)] + rank[p];
+        slot[p] = j;
+        list[j] = j;
         for (int d = 0; d < 3; ++d) {
-            if (pos) pos[3 * p + d] = (I)(add_nc((double)c[d], (double)s.off[d][p]) / (double)s.N);
-            if (vel) vel[3 * p + d] = (I)s.vel[d][p];
+            s.off[d][j] = o[d];
+            s.vel[d][j] = vel ? (T)vel[3 * p + d] : (T)0;
+        }
+        s.cell[j] = c[0] + s.N * (c[1] + s.N * c[2]);
+    }
+}
+
+template <typename T, typename I>
+__global__ void dp_state_out_kernel(DpState<T> s, const int *__restrict__ slot, I *__restrict__ pos, I *__restrict__ vel) {
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = slot[p];
+        int c[3];
+        decode(s.cell[j], s.N, c);
+        for (int d = 0; d < 3; ++d) {
+            if (pos) pos[3 * p + d] = (I)(add_nc((double)c[d], (double)s.off[d][j]) / (double)s.N);
+            if (vel) vel[3 * p + d] = (I)s.vel[d][j];
         }
     }
 }
@@ -109,7 +156,7 @@ static constexpr int DP_FW = BRK + 1, DP_F3 = DP_FW * DP_FW * DP_FW;  // nodes [
 static constexpr int DP_PW = BRK + 3, DP_P3 = DP_PW * DP_PW * DP_PW;  // nodes [o - 1, o + 9]
 
 // density: the brick's terms q w summed in an FP64 window, its nodes added to rho (128^3 FP32
-// particles in lattice order: 390 us with 8 global atomics per particle)
+// particles in lattice order: 33 us; 390 us with 8 global atomics per particle)
 template <typename T>
 __global__ __launch_bounds__(DP_WG) void dp_density_kernel(DpState<T> s, BrickIndex V, T *__restrict__ rho, T q) {
     __shared__ double win[DP_F3];
@@ -174,9 +221,10 @@ __device__ __forceinline__ void brick_forces(const T *__restrict__ phi, int N, c
 // v += dt a(X); X += dt N v; re-anchor: state s -> state t (the particles keep their numbers)
 template <typename T>
 __global__ __launch_bounds__(DP_WG) void dp_step_kernel(DpState<T> s, DpState<T> t, BrickIndex V,
-                                                        const T *__restrict__ phi, T dt) {
+                                                        const T *__restrict__ phi, T dt, DpClear<T> clear) {
     __shared__ T phw[DP_P3];
     __shared__ T frc[3][DP_F3];
+    dp_clear(clear);
     BrickRange r;
     if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
     const int N = s.N;
@@ -256,9 +304,10 @@ __device__ __forceinline__ void interp_grad(const T *__restrict__ g, int N, cons
             }
 }
 
-// lambda_x (AoS, np*3) = (init ? 0 : lambda_x) + qN grad_X interp(g)
+// lambda_x (AoS, np*3) = (init ? 0 : lambda_x) + qN grad_X interp(g); init: lambda_v = 0 too
 template <typename T>
-__global__ void dp_pos_grad_kernel(DpState<T> s, const T *__restrict__ g, T qN, T *__restrict__ lx, int init) {
+__global__ void dp_pos_grad_kernel(DpState<T> s, const T *__restrict__ g, T qN, T *__restrict__ lx, T *__restrict__ lv,
+                                   int init, DpClear<T> clear) {
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < s.np; p += (int64_t)gridDim.x * blockDim.x) {
         int c[3];
         decode(s.cell[p], s.N, c);
@@ -266,16 +315,20 @@ __global__ void dp_pos_grad_kernel(DpState<T> s, const T *__restrict__ g, T qN, 
         T gr[3];
         interp_grad(g, s.N, c, u, gr);
 #pragma unroll
-        for (int d = 0; d < 3; ++d) lx[3 * p + d] = (init ? (T)0 : lx[3 * p + d]) + qN * gr[d];
+        for (int d = 0; d < 3; ++d) {
+            lx[3 * p + d] = (init ? (T)0 : lx[3 * p + d]) + qN * gr[d];
+            if (init) lv[3 * p + d] = (T)0;
+        }
     }
+    dp_clear(clear);
 }
 
 // One backward step's particle part, and phi-bar = sum_d D_d F-bar_d with
 // F-bar_d = sum_p mu_d W: F-bar is summed per brick in three FP64 LDS windows and its
 // differences are formed there, so that a brick adds one value to each node of its
 // [o - 1, o + 9] window of phi-bar instead of 24 terms per particle to a three-component
-// field (128^3 FP32 particles: 1960 us with global atomics, and a pass over the field for the
-// differences).
+// field (128^3 FP32 particles: 68 us; 1960 us with global atomics, and a pass over the field for
+// the differences).
 template <typename T>
 __global__ __launch_bounds__(DP_WG) void dp_adj_kernel(DpState<T> s, BrickIndex V, const T *__restrict__ phi, T dt,
                                                        T *__restrict__ lx, T *__restrict__ lv, T *__restrict__ phib) {
@@ -337,12 +390,17 @@ __global__ __launch_bounds__(DP_WG) void dp_adj_kernel(DpState<T> s, BrickIndex 
     }
 }
 
-template <typename T> __global__ void dp_fill_kernel(T *__restrict__ p, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) p[i] = (T)0;
-}
-
-template <typename T, typename I> __global__ void dp_convert_kernel(const T *__restrict__ src, I *__restrict__ dst, int64_t n) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) dst[i] = (I)src[i];
+// the adjoints in the caller's order (gv may be null)
+template <typename T, typename I>
+__global__ void dp_grad_out_kernel(int64_t np, const int *__restrict__ slot, const T *__restrict__ lx,
+                                   const T *__restrict__ lv, I *__restrict__ gp, I *__restrict__ gv) {
+    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < np; p += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = slot[p];
+        for (int d = 0; d < 3; ++d) {
+            gp[3 * p + d] = (I)lx[3 * j + d];
+            if (gv) gv[3 * p + d] = (I)lv[3 * j + d];
+        }
+    }
 }
 
 }  // namespace
@@ -356,9 +414,13 @@ struct lf2mi_diffpm_s {
     size_t tsize;   // sizeof(T)
     void *ck_mem;   // nsteps + 1 particle states (cell, off[3], vel[3])
     void *rho, *phi, *resid, *phib, *rhob;  // (N+2)^3 fields of T
-    void *index_mem;  // brick index of one state (rebuilt for every state it is needed for)
+    void *index_mem;  // brick indexes, scratch of their builds, slots
     size_t index_bytes;
-    lf2mi::BrickBuild bricks;
+    lf2mi::BrickBuild bricks;  // index of the first state
+    int *index_more;           // in index_mem: an index for each further state, or null: then the
+                               // states share the first, rebuilt on the way back
+    int64_t index_ints;        // size of one index
+    int *slot;        // place of the caller's particles in the states
     void *lx, *lv;  // adjoints, np*3 of T
     double *loss_dev;
     bool forward_done;
@@ -391,48 +453,69 @@ int dp_malloc(void **p, size_t bytes) {
     return LF2MI_OK;
 }
 
+// the arrays of state k's brick index
+BrickBuild dp_index(const lf2mi_diffpm_s *m, int k) {
+    BrickBuild B = m->bricks;
+    if (k > 0 && m->index_more) {
+        int *q = m->index_more + (int64_t)(k - 1) * m->index_ints;
+        const int *q0 = m->bricks.start;  // the first index is in one piece, in the same order
+        B.start = q;
+        B.istart = q + (m->bricks.istart - q0);
+        B.item = q + (m->bricks.item - q0);
+        B.list = q + (m->bricks.list - q0);
+    }
+    return B;
+}
+
 unsigned dp_bricks_grid(const lf2mi_diffpm_s *m) {
     const int64_t nb = (m->N + BRK - 1) / BRK;
     return (unsigned)brick_items(nb * nb * nb, m->np);
 }
 
-// the brick index of state s and its density in m->rho
-template <typename T> int dp_density(lf2mi_diffpm_s *m, const DpState<T> &s, hipStream_t st) {
-    if (int rc = brick_build(s.cell, m->np, m->N, m->bricks, st)) return rc;
-    dp_fill_kernel<T><<<dp_grid(m->G3), DP_WG, 0, st>>>((T *)m->rho, m->G3);
-    LF2MI_LAUNCHED();
+// a thread per particle, and enough to clear fields beside few particles
+unsigned dp_clear_grid(const lf2mi_diffpm_s *m) {
+    return std::max(blocks_for(m->np, DP_WG), std::min(blocks_for(m->G3, DP_WG), 2048u));
+}
+
+// density of state k, whose brick index is at hand, in m->rho (cleared before)
+template <typename T> int dp_density(lf2mi_diffpm_s *m, int k, hipStream_t st) {
     const double n3 = (double)m->N * m->N * m->N;
-    dp_density_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(s, brick_view(m->bricks, m->N), (T *)m->rho,
-                                                              (T)(m->mass * n3));
+    dp_density_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(dp_view<T>(m, k), brick_view(dp_index(m, k), m->N),
+                                                              (T *)m->rho, (T)(m->mass * n3));
     LF2MI_LAUNCHED();
     return LF2MI_OK;
 }
 
-// index, density and potential of state s
-template <typename T> int dp_potential(lf2mi_diffpm_s *m, const DpState<T> &s, hipStream_t st) {
-    if (int rc = dp_density<T>(m, s, st)) return rc;
+// density and potential of state k
+template <typename T> int dp_potential(lf2mi_diffpm_s *m, int k, hipStream_t st) {
+    if (int rc = dp_density<T>(m, k, st)) return rc;
     const double n3 = (double)m->N * m->N * m->N;
     return lf2mi_poisson_solve(m->plan, m->rho, m->phi, m->mass * (double)m->np, 1.0 / n3, st);
 }
 
 template <typename T, typename I>
 int dp_forward(lf2mi_diffpm_s *m, const I *pos0, const I *vel0, const I *target, I *rho_out, double *loss, hipStream_t st) {
-    dp_init_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, 0), pos0, vel0);
+    const int N = m->N, NB = (N + BRK - 1) / BRK;
+    const DpClear<T> clear_rho{(T *)m->rho, nullptr, m->G3};
+    dp_cells_kernel<T, I><<<dp_clear_grid(m), DP_WG, 0, st>>>(m->np, pos0, N, NB, m->bricks.count, m->bricks.rank,
+                                                              clear_rho, m->loss_dev);
+    LF2MI_LAUNCHED();
+    if (int rc = brick_scan(m->bricks.scan(), NB * NB * NB, st)) return rc;
+    dp_init_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, 0), pos0, vel0, NB, m->bricks.start,
+                                                           m->bricks.rank, m->slot, m->bricks.list);
     LF2MI_LAUNCHED();
     for (int s = 0; s < m->nsteps; ++s) {
-        const DpState<T> xs = dp_view<T>(m, s);
-        if (int rc = dp_potential<T>(m, xs, st)) return rc;
-        dp_step_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, dp_view<T>(m, s + 1), brick_view(m->bricks, m->N),
-                                                               (const T *)m->phi, (T)m->dt);
+        const DpState<T> xs = dp_view<T>(m, s), xn = dp_view<T>(m, s + 1);
+        if (int rc = dp_potential<T>(m, s, st)) return rc;
+        dp_step_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, xn, brick_view(dp_index(m, s), N),
+                                                               (const T *)m->phi, (T)m->dt, clear_rho);
         LF2MI_LAUNCHED();
+        if (int rc = brick_build(xn.cell, m->np, N, dp_index(m, s + 1), st)) return rc;
     }
-    const DpState<T> fin = dp_view<T>(m, m->nsteps);
-    if (int rc = dp_density<T>(m, fin, st)) return rc;
-    dp_fill_kernel<double><<<1, DP_WG, 0, st>>>(m->loss_dev, 1);
-    LF2MI_LAUNCHED();
-    const double n3 = (double)m->N * m->N * m->N;
+    if (int rc = dp_density<T>(m, m->nsteps, st)) return rc;
+    const double n3 = (double)N * N * N;
     dp_resid_kernel<T, I><<<std::min<unsigned>(dp_grid((int64_t)n3), 1024), DP_WG, 0, st>>>(
-        (const T *)m->rho, target, (T *)m->resid, rho_out, m->N, m->loss_dev);
+        (const T *)m->rho, target, (T *)m->resid, rho_out, N, m->loss_dev);
     LF2MI_LAUNCHED();
     if (loss) {
         LF2MI_HIP(hipMemcpyAsync(loss, m->loss_dev, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -445,33 +528,29 @@ template <typename T, typename I> int dp_backward(lf2mi_diffpm_s *m, I *grad_pos
     const double n3 = (double)m->N * m->N * m->N;
     const T qN = (T)(m->mass * n3 * m->N);
     T *lx = (T *)m->lx, *lv = (T *)m->lv;
-    dp_fill_kernel<T><<<dp_grid(3 * m->np), DP_WG, 0, st>>>(lv, 3 * m->np);
-    LF2MI_LAUNCHED();
-    dp_pos_grad_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, m->nsteps), (const T *)m->resid, qN, lx, 1);
+    const DpClear<T> clear{(T *)m->rho, (T *)m->phib, m->G3};
+    dp_pos_grad_kernel<T><<<dp_clear_grid(m), DP_WG, 0, st>>>(dp_view<T>(m, m->nsteps), (const T *)m->resid, qN, lx, lv, 1,
+                                                            clear);
     LF2MI_LAUNCHED();
     for (int s = m->nsteps - 1; s >= 0; --s) {
         const DpState<T> xs = dp_view<T>(m, s);
-        if (int rc = dp_potential<T>(m, xs, st)) return rc;  // recompute phi of step s
-        dp_fill_kernel<T><<<dp_grid(m->G3), DP_WG, 0, st>>>((T *)m->phib, m->G3);
-        LF2MI_LAUNCHED();
-        dp_adj_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, brick_view(m->bricks, m->N), (const T *)m->phi,
-                                                              (T)m->dt, lx, lv, (T *)m->phib);
+        if (!m->index_more)
+            if (int rc = brick_build(xs.cell, m->np, m->N, m->bricks, st)) return rc;
+        if (int rc = dp_potential<T>(m, s, st)) return rc;  // recompute phi of step s
+        dp_adj_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, brick_view(dp_index(m, s), m->N),
+                                                              (const T *)m->phi, (T)m->dt, lx, lv, (T *)m->phib);
         LF2MI_LAUNCHED();
         if (int rc = lf2mi_poisson_solve(m->plan, m->phib, m->rhob, 0.0, 1.0 / n3, st)) return rc;
-        dp_pos_grad_kernel<T><<<dp_grid(m->np), DP_WG, 0, st>>>(xs, (const T *)m->rhob, qN, lx, 0);
+        dp_pos_grad_kernel<T><<<dp_clear_grid(m), DP_WG, 0, st>>>(xs, (const T *)m->rhob, qN, lx, lv, 0, clear);
         LF2MI_LAUNCHED();
     }
-    dp_convert_kernel<T, I><<<dp_grid(3 * m->np), DP_WG, 0, st>>>(lx, grad_pos, 3 * m->np);
+    dp_grad_out_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(m->np, m->slot, lx, lv, grad_pos, grad_vel);
     LF2MI_LAUNCHED();
-    if (grad_vel) {
-        dp_convert_kernel<T, I><<<dp_grid(3 * m->np), DP_WG, 0, st>>>(lv, grad_vel, 3 * m->np);
-        LF2MI_LAUNCHED();
-    }
     return LF2MI_OK;
 }
 
 template <typename T, typename I> int dp_state(lf2mi_diffpm_s *m, int step, I *pos, I *vel, hipStream_t st) {
-    dp_state_out_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, step), pos, vel);
+    dp_state_out_kernel<T, I><<<dp_grid(m->np), DP_WG, 0, st>>>(dp_view<T>(m, step), m->slot, pos, vel);
     LF2MI_LAUNCHED();
     return LF2MI_OK;
 }
@@ -515,9 +594,22 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     if (!rc) rc = dp_malloc(&m->phi, fb);
     if (!rc) rc = dp_malloc(&m->resid, fb);
     const int64_t nb = (N + BRK - 1) / BRK, nbk = nb * nb * nb, items = brick_items(nbk, np);
-    // starts, item starts, counts, block totals, items, list, places
-    m->index_bytes = sizeof(int) * (size_t)(2 * (nbk + 1) + nbk + 3 * brick_blocks(nbk) + items + 2 * np);
-    if (!rc) rc = dp_malloc(&m->index_mem, m->index_bytes);
+    // an index: starts, item starts, items, list; once: counts, block totals, ranks, slots
+    m->index_ints = 2 * (nbk + 1) + items + np;
+    m->index_bytes = sizeof(int) * (size_t)(m->index_ints + nbk + 3 * brick_blocks(nbk) + 2 * np);
+    if (!rc && nsteps > 0) {
+        // if there is room, the indexes of the further states are kept for the way back (about
+        // 4 bytes per particle and state)
+        const size_t more = sizeof(int) * (size_t)m->index_ints * (size_t)nsteps;
+        if (hipMalloc(&m->index_mem, m->index_bytes + more) == hipSuccess) {
+            m->index_more = (int *)((char *)m->index_mem + m->index_bytes);
+            m->index_bytes += more;
+        } else {
+            (void)hipGetLastError();
+            m->index_mem = nullptr;
+        }
+    }
+    if (!rc && !m->index_mem) rc = dp_malloc(&m->index_mem, m->index_bytes);
     if (!rc) {
         int *q = (int *)m->index_mem;
         auto take = [&q](int64_t n) {
@@ -527,11 +619,12 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
         };
         m->bricks.start = take(nbk + 1);
         m->bricks.istart = take(nbk + 1);
-        m->bricks.count = take(nbk);
-        m->bricks.bsum = take(3 * brick_blocks(nbk));
         m->bricks.item = take(items);
         m->bricks.list = take(np);
+        m->bricks.count = take(nbk);
+        m->bricks.bsum = take(3 * brick_blocks(nbk));
         m->bricks.rank = take(np);
+        m->slot = take(np);
         hipError_t e = hipMemset(m->bricks.count, 0, sizeof(int) * (size_t)nbk);
         if (e != hipSuccess) rc = hip_fail(e, "hipMemset(diffpm)", __FILE__, __LINE__);
     }

@@ -229,3 +229,30 @@ def test_diffpm_errors():
         raw.call("lf2mi_diffpm_backward", m.h, g.data_ptr(), None, None)
     with pytest.raises(lf.Lf2miError):
         DiffPM(12, 64, 1, 1.0, 0.01, lf.F32)  # N must be a power of two
+
+
+@pytest.mark.parametrize("N,np_", [(8, 1), (8, 67), (16, 5001), (32, 3000)])
+def test_diffpm_any_particle_order(N, np_):
+    """Particles without order, in counts that fill no wavefront or brick, against the oracle:
+    states and gradients come in the caller's order, also from a second evaluation.  FP64 sums
+    of at most some hundred terms, each rounded at 1e-16, over a few steps: the bounds are those
+    of the ordered FP64 run above."""
+    lf, DiffPM, _ = _lib()
+    import oracle as orc
+    announce(f"diffpm unordered N={N} np={np_}")
+    nsteps, dt, mass = 2, 0.02, 1.0 / np_
+    rng = np.random.default_rng(70 + np_)
+    m = DiffPM(N, np_, nsteps, mass, dt, lf.F64)
+    for _ in range(2):
+        pos0, vel0, tpos = rng.random((np_, 3)), rng.normal(0.0, 0.05, (np_, 3)), rng.random((np_, 3))
+        target = orc.cic_density(tpos, N, mass)
+        L, gp, gv = orc.diffpm_loss_grad(pos0, vel0, N, mass, dt, nsteps, target)
+        fpos, fvel = orc.diffpm_forward(pos0, vel0, N, mass, dt, nsteps)
+        gL = m.forward(dev(pos0), dev(vel0), dev(target.ravel()))
+        ggp, ggv = m.backward()
+        pos, vel = m.state(nsteps)
+        torch.cuda.synchronize()
+        dpos = np.mod(pos.cpu().numpy() - fpos + 0.5, 1.0) - 0.5
+        assert abs(gL - L) / L <= 1e-11
+        assert np.abs(dpos).max() * N <= 1e-10 and rel_l2(vel.cpu().numpy(), fvel) <= 1e-11
+        assert rel_l2(ggp.cpu().numpy(), gp) <= 1e-9 and rel_l2(ggv.cpu().numpy(), gv) <= 1e-9
