@@ -349,6 +349,37 @@ __global__ void upload_f64_kernel(int64_t np, const double *__restrict__ pos, co
     for (int w = 0; w < plw; ++w) dst.pl[j * plw + w] = pl[i * plw + w];
 }
 
+// ---------------------------------------------------------------- drift
+// Drift in FP64 cell units and re-anchoring: X = (c + u) + fl(dt v) N, then the sequential
+// periodic wrap of Particles.hpp:2028-2032 and re-binning to (cell, FP32 offset o).  Returns the
+// new cell.  The kick (which counts the new buckets) and the scatter (which moves the particles
+// there) both evaluate it from the stored state, so every operation is pinned: the two agree in
+// every bit.  Both kernels are bound by the particles' bytes; moved by the kick, the new
+// positions were written once more, 16 of 112 bytes per particle and step (a step of 256^3
+// particles on 256^3: 746 -> 703 us).
+__device__ __forceinline__ int drift_cell(int N, double dt, int cx, int cy, int cz, const float u[3], const float v[3],
+                                          float o[3]) {
+    int c3[3] = {cx, cy, cz};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        double X = add_rn((double)c3[d], (double)u[d]);
+        X = add_rn(X, mul_rn(mul_rn(dt, (double)v[d]), (double)N));
+        if (X < 0.0) X = add_rn(X, (double)N);
+        if (X >= (double)N) X = sub_rn(X, (double)N);
+        // beyond the reference's range (|dt v| >= box) wrap fully so the cell stays valid
+        if (X < 0.0 || X >= (double)N) X = __builtin_fma(-(double)N, floor(X / (double)N), X);
+        const double fl = floor(X);
+        int cn = (int)fl;
+        if (cn >= N) cn = N - 1;
+        if (cn < 0) cn = 0;
+        float on = (float)sub_rn(X, fl);
+        if (!(on < 1.0f)) on = 0x1.fffffep-1f;
+        c3[d] = cn;
+        o[d] = on;
+    }
+    return c3[0] + N * (c3[1] + N * c3[2]);
+}
+
 // ---------------------------------------------------------------- scatter (counting sort)
 // Counting-sort scatter, SCAT_PER particles per thread (1024 per block): every load is in
 // flight before the slots are claimed.  Slots: per wave, lanes with equal new buckets form
@@ -361,8 +392,9 @@ __global__ void upload_f64_kernel(int64_t np, const double *__restrict__ pos, co
 static constexpr int SCAT_PER = 4;
 static constexpr int SCAT_HT = 2048;
 
+template <bool DRIFT>
 __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa32 dst, Geo g,
-                                                      int *__restrict__ cursor, int plw) {
+                                                      int *__restrict__ cursor, int plw, double dt) {
     __shared__ int hkey[SCAT_HT];
     __shared__ int hval[SCAT_HT];  // group counts, then the bucket's reserved base
     for (int i = threadIdx.x; i < SCAT_HT; i += 256) {
@@ -387,6 +419,16 @@ __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa
             }
             if (src.mass) m[k] = src.mass[i];
             if (src.id) id[k] = src.id[i];
+        }
+    }
+    if constexpr (DRIFT) {
+#pragma unroll
+        for (int k = 0; k < SCAT_PER; ++k) {
+            if (cell[k] < 0) continue;
+            int cx, cy, cz;
+            decode_cell(cell[k], g, cx, cy, cz);
+            const float u[3] = {o[k][0], o[k][1], o[k][2]};
+            cell[k] = drift_cell(g.N, dt, cx, cy, cz, u, v[k], o[k]);
         }
     }
     __syncthreads();
@@ -1447,42 +1489,17 @@ struct GkdArgs {
     int drift;              // 0: a kick only; positions, cells and buckets stay
 };
 
-// kick with the gathered acceleration, drift in FP64 cell units, re-anchor and store:
-// X = (c + u) + fl(dt v) N, then the sequential periodic wrap of Particles.hpp:2028-2032
-// and re-binning to (cell, FP32 offset).  Returns the new cell.
-__device__ __forceinline__ int kick_drift_store(const GkdArgs &A, int p, int cx, int cy, int cz, const float u[3],
-                                                const float vin[3], const float a[3], float &vmax) {
-    const int N = A.g.N;
-    float v[3];
-    int c3[3] = {cx, cy, cz};
-    float o[3];
+// kick with the gathered acceleration, store the velocity; returns the cell after the drift
+__device__ __forceinline__ int kick_store(const GkdArgs &A, int p, int cx, int cy, int cz, const float u[3],
+                                          const float vin[3], const float a[3], float &vmax) {
+    float v[3], o[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         v[d] = vin[d] + A.dt_kick * a[d];
-        double X = add_rn((double)c3[d], (double)u[d]);
-        X = add_rn(X, mul_rn(A.dt_drift, (double)v[d]) * (double)N);
-        if (X < 0.0) X = add_rn(X, (double)N);
-        if (X >= (double)N) X = sub_rn(X, (double)N);
-        // beyond the reference's range (|dt v| >= box) wrap fully so the cell stays valid
-        if (X < 0.0 || X >= (double)N) X -= (double)N * floor(X / (double)N);
-        const double fl = floor(X);
-        int cn = (int)fl;
-        if (cn >= N) cn = N - 1;
-        if (cn < 0) cn = 0;
-        float on = (float)(X - fl);
-        if (!(on < 1.0f)) on = 0x1.fffffep-1f;
-        c3[d] = cn;
-        o[d] = on;
-    }
-    const int newcell = c3[0] + N * (c3[1] + N * c3[2]);
-    if (A.drift) A.s.cell[p] = newcell;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (A.drift) A.s.off[d][p] = o[d];
         A.s.vel[d][p] = v[d];
     }
     vmax = fmaxf(vmax, v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
-    return newcell;
+    return A.drift ? drift_cell(A.g.N, A.dt_drift, cx, cy, cz, u, v, o) : 0;
 }
 
 // CIC interpolation of F = -grad phi (centred differences, N/2 per unit of phi) at a
@@ -1609,7 +1626,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) {
                 const float vin[3] = {A.s.vel[0][p], A.s.vel[1][p], A.s.vel[2][p]};
                 float a[3] = {0.f, 0.f, 0.f};
                 if (A.phi) gather_direct(A, cx, cy, cz, u, a);
-                newcell = kick_drift_store(A, p, cx, cy, cz, u, vin, a, vmax);
+                newcell = kick_store(A, p, cx, cy, cz, u, vin, a, vmax);
             }
             if (A.drift) gkd_hist_add(A, r.b, h27, act, newcell);
         }
@@ -1685,7 +1702,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) {
                             a[1] += w * frc[1][n];
                             a[2] += w * frc[2][n];
                         }
-                newcell = kick_drift_store(A, p, cx, cy, cz, u, vin, a, vmax);
+                newcell = kick_store(A, p, cx, cy, cz, u, vin, a, vmax);
             }
             if (A.drift) gkd_hist_add(A, r.b, h27, act, newcell);
         }
@@ -1810,7 +1827,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4
             const int zs[4] = {lz - 1, lz, lz + 1, lz + 2};
             float a[3];
             cic_force([&](int x, int y, int z) { return win[x + wx * (y + wy * z)]; }, xs, ys, zs, hn, u, a);
-            const int newcell = kick_drift_store(A, p, cx, cy, cz, u, vin, a, vmax);
+            const int newcell = kick_store(A, p, cx, cy, cz, u, vin, a, vmax);
             if (!A.drift) continue;
             // new bucket relative to the chunk: x in [-1, nbx], y and z in [-1, 1] (periodic)
             int nx, ny, nz;
@@ -2706,12 +2723,14 @@ static int scan_buckets(lf2mi_parts_s *p, hipStream_t st) {
     return brick_scan(S, (int)n, st);
 }
 
-// counting sort of buffer `src` (counts already in bcount) into buffer 1 - src
-static int sort_into_other(lf2mi_parts_s *p, int src, int64_t nsrc, hipStream_t st) {
+// counting sort of buffer `src` (counts already in bcount) into buffer 1 - src; drift: the
+// particles move by dt on the way
+static int sort_into_other(lf2mi_parts_s *p, int src, int64_t nsrc, bool drift, double dt, hipStream_t st) {
     if (int rc = scan_buckets(p, st)) return rc;
     LF2MI_PROF("rebucket_scatter", st);
-    scatter_kernel<<<grid1(nsrc, 256 * SCAT_PER), 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor,
-                                                                  p->plw);
+    const unsigned grid = grid1(nsrc, 256 * SCAT_PER);
+    if (drift) scatter_kernel<true><<<grid, 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor, p->plw, dt);
+    else scatter_kernel<false><<<grid, 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor, p->plw, dt);
     LF2MI_LAUNCHED();
     p->cur = 1 - src;
     return LF2MI_OK;
@@ -2868,7 +2887,7 @@ static int ic_common(lf2mi_parts_s *p, IcArgs &A, hipStream_t st) {
         LF2MI_LAUNCHED();
         if (p->plw && A.np > 0)
             LF2MI_HIP(hipMemsetAsync(p->b32[src].pl, 0, (size_t)A.np * p->plw * sizeof(unsigned long long), st));
-        if (int rc = sort_into_other(p, src, A.np, st)) return rc;
+        if (int rc = sort_into_other(p, src, A.np, false, 0.0, st)) return rc;
         if (int rc = read_total(p, st, &p->np)) return rc;
     } else {
         p->np = A.np;
@@ -3175,7 +3194,7 @@ static int upload_impl(lf2mi_parts p, int64_t np, const double *pos, const doubl
                                                              p->bcount);
                 if ((e = hipGetLastError()) != hipSuccess) rc = hip_fail(e, "bin_upload_kernel", __FILE__, __LINE__);
             }
-            if (!rc) rc = sort_into_other(p, src, nk, st);
+            if (!rc) rc = sort_into_other(p, src, nk, false, 0.0, st);
             if (!rc) rc = read_total(p, st, &p->np);
         } else {
             p->np = nk;
@@ -3899,7 +3918,7 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
     }
     // (the scan clears the claims)
     if (A.drift) {
-        if (int rc = sort_into_other(p, p->cur, p->np, st)) return rc;
+        if (int rc = sort_into_other(p, p->cur, p->np, true, dt_drift, st)) return rc;
     } else if (A.chunked) {
         if (int rc = fill_int(p->nchunk + 1, 1, 0, st)) return rc;
     }
