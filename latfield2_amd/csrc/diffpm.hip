@@ -18,8 +18,9 @@
 //                        lambda_x += q N grad_X interp(rho-bar)(X_p)   (deposit weights)
 // A particle keeps its place in all states, so gradients stay attached to it; a brick index
 // (bricks.hpp) of every state lets the deposits and gathers work brick by brick.  The starting
-// state of every step is checkpointed in HBM and the fields are recomputed on the way back.
-// Positions are kept as (cell, offset in cell units) and re-anchored
+// state and the potential of every step are checkpointed in HBM; where that has no room for the
+// potentials and indexes (8 bytes beside a particle's 28 or 52), they are computed again on the
+// way back.  Positions are kept as (cell, offset in cell units) and re-anchored
 // in FP64 after each drift, as in the PM step.  T = float or double selects the
 // precision of the whole path (fields, FFTs, offsets, velocities, adjoints).
 #include <algorithm>
@@ -420,6 +421,7 @@ struct lf2mi_diffpm_s {
     int *index_more;           // in index_mem: an index for each further state, or null: then the
                                // states share the first, rebuilt on the way back
     int64_t index_ints;        // size of one index
+    char *phi_kept;            // in index_mem: the potentials of the steps, or null with index_more
     int *slot;        // place of the caller's particles in the states
     void *lx, *lv;  // adjoints, np*3 of T
     double *loss_dev;
@@ -467,6 +469,11 @@ BrickBuild dp_index(const lf2mi_diffpm_s *m, int k) {
     return B;
 }
 
+// the potential of step k
+template <typename T> T *dp_phi(const lf2mi_diffpm_s *m, int k) {
+    return (T *)(m->phi_kept ? m->phi_kept + (size_t)k * m->G3 * m->tsize : (char *)m->phi);
+}
+
 unsigned dp_bricks_grid(const lf2mi_diffpm_s *m) {
     const int64_t nb = (m->N + BRK - 1) / BRK;
     return (unsigned)brick_items(nb * nb * nb, m->np);
@@ -490,7 +497,7 @@ template <typename T> int dp_density(lf2mi_diffpm_s *m, int k, hipStream_t st) {
 template <typename T> int dp_potential(lf2mi_diffpm_s *m, int k, hipStream_t st) {
     if (int rc = dp_density<T>(m, k, st)) return rc;
     const double n3 = (double)m->N * m->N * m->N;
-    return lf2mi_poisson_solve(m->plan, m->rho, m->phi, m->mass * (double)m->np, 1.0 / n3, st);
+    return lf2mi_poisson_solve(m->plan, m->rho, dp_phi<T>(m, k), m->mass * (double)m->np, 1.0 / n3, st);
 }
 
 template <typename T, typename I>
@@ -508,7 +515,7 @@ int dp_forward(lf2mi_diffpm_s *m, const I *pos0, const I *vel0, const I *target,
         const DpState<T> xs = dp_view<T>(m, s), xn = dp_view<T>(m, s + 1);
         if (int rc = dp_potential<T>(m, s, st)) return rc;
         dp_step_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, xn, brick_view(dp_index(m, s), N),
-                                                               (const T *)m->phi, (T)m->dt, clear_rho);
+                                                               dp_phi<T>(m, s), (T)m->dt, clear_rho);
         LF2MI_LAUNCHED();
         if (int rc = brick_build(xn.cell, m->np, N, dp_index(m, s + 1), st)) return rc;
     }
@@ -528,17 +535,18 @@ template <typename T, typename I> int dp_backward(lf2mi_diffpm_s *m, I *grad_pos
     const double n3 = (double)m->N * m->N * m->N;
     const T qN = (T)(m->mass * n3 * m->N);
     T *lx = (T *)m->lx, *lv = (T *)m->lv;
-    const DpClear<T> clear{(T *)m->rho, (T *)m->phib, m->G3};
+    const DpClear<T> clear{m->phi_kept ? nullptr : (T *)m->rho, (T *)m->phib, m->G3};
     dp_pos_grad_kernel<T><<<dp_clear_grid(m), DP_WG, 0, st>>>(dp_view<T>(m, m->nsteps), (const T *)m->resid, qN, lx, lv, 1,
                                                             clear);
     LF2MI_LAUNCHED();
     for (int s = m->nsteps - 1; s >= 0; --s) {
         const DpState<T> xs = dp_view<T>(m, s);
-        if (!m->index_more)
+        if (!m->phi_kept) {  // nor its index
             if (int rc = brick_build(xs.cell, m->np, m->N, m->bricks, st)) return rc;
-        if (int rc = dp_potential<T>(m, s, st)) return rc;  // recompute phi of step s
-        dp_adj_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, brick_view(dp_index(m, s), m->N),
-                                                              (const T *)m->phi, (T)m->dt, lx, lv, (T *)m->phib);
+            if (int rc = dp_potential<T>(m, s, st)) return rc;
+        }
+        dp_adj_kernel<T><<<dp_bricks_grid(m), DP_WG, 0, st>>>(xs, brick_view(dp_index(m, s), m->N), dp_phi<T>(m, s),
+                                                              (T)m->dt, lx, lv, (T *)m->phib);
         LF2MI_LAUNCHED();
         if (int rc = lf2mi_poisson_solve(m->plan, m->phib, m->rhob, 0.0, 1.0 / n3, st)) return rc;
         dp_pos_grad_kernel<T><<<dp_clear_grid(m), DP_WG, 0, st>>>(xs, (const T *)m->rhob, qN, lx, lv, 0, clear);
@@ -566,7 +574,7 @@ int lf2mi_diffpm_bytes(lf2mi_diffpm m, int64_t *bytes) {
     if (!m || !bytes) return fail(LF2MI_EINVAL, "lf2mi_diffpm_bytes: null argument");
     int64_t fft = 0;
     if (int rc = lf2mi_fft_plan_bytes(m->plan, &fft)) return rc;
-    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + 5 * (size_t)m->G3 * m->tsize + m->index_bytes +
+    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + (m->phi ? 5 : 4) * (size_t)m->G3 * m->tsize + m->index_bytes +
                        6 * (size_t)m->np * m->tsize + sizeof(double)) + fft;
     return LF2MI_OK;
 }
@@ -591,25 +599,27 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     int rc = lf2mi_fft_plan_create(N, 1, 1, 0, dtype, &m->plan);
     if (!rc) rc = dp_malloc(&m->ck_mem, dp_state_bytes(np, m->tsize) * (size_t)(nsteps + 1));
     if (!rc) rc = dp_malloc(&m->rho, fb);
-    if (!rc) rc = dp_malloc(&m->phi, fb);
     if (!rc) rc = dp_malloc(&m->resid, fb);
     const int64_t nb = (N + BRK - 1) / BRK, nbk = nb * nb * nb, items = brick_items(nbk, np);
     // an index: starts, item starts, items, list; once: counts, block totals, ranks, slots
     m->index_ints = 2 * (nbk + 1) + items + np;
     m->index_bytes = sizeof(int) * (size_t)(m->index_ints + nbk + 3 * brick_blocks(nbk) + 2 * np);
     if (!rc && nsteps > 0) {
-        // if there is room, the indexes of the further states are kept for the way back (about
-        // 4 bytes per particle and state)
-        const size_t more = sizeof(int) * (size_t)m->index_ints * (size_t)nsteps;
-        if (hipMalloc(&m->index_mem, m->index_bytes + more) == hipSuccess) {
-            m->index_more = (int *)((char *)m->index_mem + m->index_bytes);
-            m->index_bytes += more;
+        // if there is room, the potentials of the steps and the indexes of the further states are
+        // kept for the way back
+        const size_t own = (m->index_bytes + 255) / 256 * 256, phis = fb * (size_t)nsteps;
+        const size_t all = own + phis + sizeof(int) * (size_t)m->index_ints * (size_t)nsteps;
+        if (hipMalloc(&m->index_mem, all) == hipSuccess) {
+            m->phi_kept = (char *)m->index_mem + own;
+            m->index_more = (int *)(m->phi_kept + phis);
+            m->index_bytes = all;
         } else {
             (void)hipGetLastError();
             m->index_mem = nullptr;
         }
     }
     if (!rc && !m->index_mem) rc = dp_malloc(&m->index_mem, m->index_bytes);
+    if (!rc && !m->phi_kept) rc = dp_malloc(&m->phi, fb);
     if (!rc) {
         int *q = (int *)m->index_mem;
         auto take = [&q](int64_t n) {
@@ -636,6 +646,7 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     if (!rc) {
         // the ghosts of these fields are never written by the kernels here; keep them defined
         for (void *p : {m->rho, m->phi, m->resid, m->phib, m->rhob}) {
+            if (!p) continue;
             hipError_t e = hipMemset(p, 0, fb);
             if (e != hipSuccess) {
                 rc = hip_fail(e, "hipMemset(diffpm)", __FILE__, __LINE__);
