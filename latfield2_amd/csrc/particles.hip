@@ -1967,22 +1967,30 @@ __global__ void deposit_f64_kernel(Dep64Args A) {
 
 // ---- brick windows
 // One workgroup per group of consecutive particles of a brick: every particle's terms go into
-// an LDS window of the brick's nodes, all components interleaved as in the field, and the
-// window's non-zero values then go to the field with one atomic each, consecutive lanes on
-// consecutive addresses.  The window sums are FP64 (W = double), or int64 of terms quantised
-// one by one (W = unsigned long long, the fixed-point deposit).  No sort: a wave's particles
-// rarely share a node.  int64 windows of scaled sums, whose LDS atomics are twice as fast but
-// need a pass for the scale and conversions, measured equal to 25 % slower: the flush bounds
-// it, at 300-350 G atomics/s.  (FP32
-// container at 256^3, 512 particles per brick, microseconds, against sorting a brick's items
-// by cell and summing runs in registers first: scalar 247 -> 218, vector 710 -> 466, VecVec
-// 1572 -> 893, CIC-NGP 580 -> 387 / 1188 -> 692.)
+// an LDS window of the brick's nodes, and the window's non-zero values then go to the field with
+// one atomic each, consecutive lanes on consecutive addresses.  The window sums are FP64
+// (W = double), or int64 of terms quantised one by one (W = unsigned long long, the fixed-point
+// deposit).  No sort: a wave's particles rarely share a node, and nearly sorted ones would more
+// often (LDS atomics of random cells 1500 G/s, of neighbouring ones 1290-1380).  FP32 container
+// at 256^3, 512 particles per brick, microseconds, against sorting a brick's items by cell and
+// summing runs in registers first: scalar 247 -> 218, vector 710 -> 466, VecVec 1572 -> 831,
+// CIC-NGP 580 -> 387 and 1188 -> 692.  What bounds it: of VecVec's 945 us before the layout below
+// the LDS atomics were 560 and the flush 59; of the FP64 container's 280 for a scalar the flush
+// is half.  Without gain: int64 windows of scaled sums, whose LDS atomics are twice as fast but
+// need a pass for the scale and conversions (equal to 25 % slower); nodes that only one window
+// covers added to without atomics (280 -> 442, 945 -> 1066: loads at each workgroup's end).
 // 512 threads for six components, whose window leaves room for three workgroups per CU.
 template <int KIND> constexpr int bw_wg() { return KindC<KIND>::C == 6 ? 512 : 256; }
 template <int KIND> constexpr int bw_edge() { return BRK + 1 - KindC<KIND>::LO; }
 template <int KIND> constexpr int bw_size() {
     return bw_edge<KIND>() * bw_edge<KIND>() * bw_edge<KIND>() * KindC<KIND>::C;
 }
+
+// window values from a node to the next: components interleaved, or, of six, one after the other
+// (interleaved their nodes lie 12 banks apart, and random nodes meet in a third of the banks:
+// 1129 G atomics/s against 1505; 256^3 VecVec 945 -> 831 us; three interleaved components have no
+// such conflict)
+template <int KIND> constexpr int bw_stride() { return KindC<KIND>::C == 6 ? 1 : KindC<KIND>::C; }
 
 template <typename T> struct BwParticle {
     int l[3];                // cell in the brick
@@ -2018,7 +2026,7 @@ __device__ __forceinline__ void bw_term(unsigned long long *p, float q, float w0
 
 template <int KIND, int COMP, typename W, typename T>
 __device__ __forceinline__ void bw_add(W *__restrict__ win, const BwParticle<T> &P, T q, const double *fxs) {
-    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP, C = KindC<KIND>::C, E = bw_edge<KIND>();
+    constexpr int M = Comp<KIND, COMP>::MASK, G = Comp<KIND, COMP>::NGP, E = bw_edge<KIND>();
     int b[3];
     T w[3][2];
     constexpr int n[3] = {(G & 1) ? 1 : 2, (G & 2) ? 1 : 2, (G & 4) ? 1 : 2};
@@ -2029,14 +2037,15 @@ __device__ __forceinline__ void bw_add(W *__restrict__ win, const BwParticle<T> 
         w[d][0] = ngp ? (T)1 : (link ? P.lw[d][0] : P.vw[d][0]);
         w[d][1] = ngp ? (T)0 : (link ? P.lw[d][1] : P.vw[d][1]);
     }
-    W *o = win + C * (b[0] + E * (b[1] + E * b[2])) + COMP;
+    constexpr int SN = bw_stride<KIND>();
+    W *o = win + SN * (b[0] + E * (b[1] + E * b[2])) + COMP * (SN == 1 ? E * E * E : 1);
 #pragma unroll
     for (int k = 0; k < n[2]; ++k)
 #pragma unroll
         for (int j = 0; j < n[1]; ++j)
 #pragma unroll
             for (int i = 0; i < n[0]; ++i)
-                bw_term(&o[C * (i + E * (j + E * k))], q, w[0][i], w[1][j], w[2][k], fxs[COMP]);
+                bw_term(&o[SN * (i + E * (j + E * k))], q, w[0][i], w[1][j], w[2][k], fxs[COMP]);
 }
 
 // a particle's terms of every component
@@ -2065,9 +2074,9 @@ __device__ __forceinline__ void bw_flush(const W *__restrict__ win, F *__restric
                                          int ox, int oy, int oz) {
     constexpr int C = KindC<KIND>::C, LO = KindC<KIND>::LO, E = bw_edge<KIND>();
     for (int i = threadIdx.x; i < bw_size<KIND>(); i += bw_wg<KIND>()) {
-        const W v = win[i];
-        if (v == W(0)) continue;
         const int c = i % C, n = i / C;
+        const W v = bw_stride<KIND>() == 1 ? win[n + E * E * E * c] : win[i];
+        if (v == W(0)) continue;
         int gx = ox + n % E + LO, gy = oy + (n / E) % E + LO, gz = oz + n / (E * E) + LO;
         if (tgt == LF2MI_DEP_PERIODIC) {
             gx = wrapi(gx, N);
