@@ -1741,11 +1741,14 @@ static_assert((DEP_WG / 64) * GKD_STAGE >= (MAXB + 3) * (MAXB + 3), "one batch o
 // GKD_CHUNK_B bricks), the following one while this one's particles are processed.  Chunks cut
 // at fixed borders instead, a workgroup each, cost 0.74 ms against 0.62 at 512^3 (blobs): a
 // fourth more of them.
-template <int BC>
+// ONE: chunks of one brick each and no more of them than workgroups (small lattices): nothing to
+// claim, and a small window, whose 11-value rows would leave most of a wave idle (64^3 with 64
+// particles per brick 15.7 -> 6.5 us; both forms in one kernel cost the wide one a tenth).
+template <int BC, bool ONE>
 __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4 *__restrict__ chunks,
                                                            int *__restrict__ nchunk) {
-    constexpr int WXM = GKD_CHUNK_B * MAXB + 3, WYM = MAXB + 3;
-    constexpr int NHM = (GKD_CHUNK_B + 2) * 9;
+    constexpr int WXM = (ONE ? 1 : GKD_CHUNK_B) * MAXB + 3, WYM = MAXB + 3;
+    constexpr int NHM = ((ONE ? 1 : GKD_CHUNK_B) + 2) * 9;
     __shared__ float win[WXM * WYM * WYM];
     __shared__ int hist[NHM];
     __shared__ unsigned int red;
@@ -1781,10 +1784,27 @@ __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4
             }
         };
         fetch(ch.x);
-        // rows (y, z) of the window, one wave per row: the row's base index is wave-uniform,
-        // a lane holds x = lane and x = lane + 64; every row's loads are issued before the
-        // LDS stores (a load-store loop would wait out one HBM round trip per row)
-        {
+        if constexpr (ONE) {
+            // one brick: four rows (y, z) per wave
+            constexpr int RB = DEP_WG / 16, ST = (WYM * WYM + RB - 1) / RB;
+            const int x = threadIdx.x & 15, gx = wrapi(ox - 1 + min(x, wx - 1), N);
+            float v[ST];
+#pragma unroll
+            for (int k = 0; k < ST; ++k) {
+                const int row = (int)(threadIdx.x >> 4) + RB * k;
+                v[k] = 0.0f;
+                if (row < wy * wy)
+                    v[k] = A.phi[site_index(N, A.h, gx, wrapi(oy - 1 + row % wy, N), wrapi(oz - 1 + row / wy, N))];
+            }
+#pragma unroll
+            for (int k = 0; k < ST; ++k) {
+                const int row = (int)(threadIdx.x >> 4) + RB * k;
+                if (x < wx && row < wy * wy) win[x + wx * row] = v[k];
+            }
+        } else {
+            // rows (y, z) of the window, one wave per row: the row's base index is wave-uniform,
+            // a lane holds x = lane and x = lane + 64; every row's loads are issued before the
+            // LDS stores (a load-store loop would wait out one HBM round trip per row)
             const int nrows = wy * wy;
             const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
             const int lane = threadIdx.x & 63;
@@ -1818,7 +1838,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4
             }
         }
         __syncthreads();
-        if (threadIdx.x == 0) claim = (int)gridDim.x + atomicAdd(&nchunk[1], 1);
+        if (!ONE && threadIdx.x == 0) claim = (int)gridDim.x + atomicAdd(&nchunk[1], 1);
         for (int q0 = ch.x; q0 < ch.y; q0 += ITEM_P) {
         if (q0 != ch.x) fetch(q0);
 #pragma unroll
@@ -1865,6 +1885,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4
             const int bbx = (bx0 + ex + NB) % NB, bby = (by + ey + NB) % NB, bbz = (bz + ez + NB) % NB;
             atomicAdd(&A.next_counts[bbx + NB * (bby + NB * bbz)], c);
         }
+        if constexpr (ONE) break;
         ci = claim;
         __syncthreads();
     }
@@ -2713,6 +2734,14 @@ static int b64_fill(lf2mi_parts_s *p, const double *pos, const double *vel, cons
     return LF2MI_OK;
 }
 
+// bricks per chunk of the sparse gather: fewer on small lattices, while that leaves less than 1024
+// chunks (four workgroups per CU)
+static int chunk_width(const lf2mi_parts_s *p) {
+    int w = GKD_CHUNK_B;
+    while (w > 1 && p->g.nbk / w < 1024) w /= 2;
+    return w;
+}
+
 // exclusive scans of bcount -> bstart and the cursors, items -> istart, and the dense bricks'
 // groups; bcount comes out cleared
 static int scan_buckets(lf2mi_parts_s *p, hipStream_t st) {
@@ -2734,10 +2763,7 @@ static int scan_buckets(lf2mi_parts_s *p, hipStream_t st) {
     S.nchunk = p->nchunk;
     S.NB = p->g.NB;
     S.sparse_max = GKD_DIRECT_MAX;
-    // narrower chunks on small lattices, while that leaves fewer than 1024 of them (four
-    // workgroups per CU)
-    S.chunk_w = GKD_CHUNK_B;
-    while (S.chunk_w > 1 && n / S.chunk_w < 1024) S.chunk_w /= 2;
+    S.chunk_w = chunk_width(p);
     return brick_scan(S, (int)n, st);
 }
 
@@ -3927,11 +3953,17 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
         LF2MI_LAUNCHED();
     }
     if (A.chunked) {
-        // persistent: a few workgroups per CU walk the chunk list
         LF2MI_PROF("gkd_f32_chunks", st);
-        const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(p->g.nbk, 2048));
-        if (b8) gkd_chunk_kernel<8><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
-        else gkd_chunk_kernel<0><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+        if (chunk_width(p) == 1) {
+            const unsigned grid = (unsigned)p->g.nbk;
+            if (b8) gkd_chunk_kernel<8, true><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+            else gkd_chunk_kernel<0, true><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+        } else {
+            // persistent: a few workgroups per CU walk the chunk list
+            const unsigned grid = (unsigned)std::min<int64_t>(p->g.nbk, 2048);
+            if (b8) gkd_chunk_kernel<8, false><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+            else gkd_chunk_kernel<0, false><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+        }
         LF2MI_LAUNCHED();
     }
     // (the scan clears the claims)

@@ -37,3 +37,31 @@ def test_drift_moves_every_particle_once(N, n, speed):
         off = b["pos"] * N - np.stack([c % N, c // N % N, c // N ** 2], axis=1)
         assert np.min(off) >= -1e-12 and np.max(off) <= 1.0
         assert np.array_equal(parts.cell_counts().cpu().numpy(), np.bincount(c, minlength=N ** 3))
+
+
+@pytest.mark.parametrize("N", [8, 20, 64, 96, 104])
+def test_sparse_gather_matches_fp64(N):
+    """Bricks of few particles, in chunks of one brick (up to 12^3 bricks of 8^3 cells) and of
+    several (from 13^3), against the FP64 container.  White noise as the potential: its
+    differences cancel nothing, so a velocity carries some 30 FP32 roundings of 6e-8."""
+    announce(f"sparse gather N={N}")
+    n = 20 * ((N + 7) // 8) ** 3 + 3
+    rng = np.random.default_rng(N)
+    pos, vel = rng.random((n, 3)), rng.standard_normal((n, 3))
+    lat = lf.Lattice(3, N, 1)
+    out = {}
+    f32 = lf.Field(lat, 1, lf.F32)
+    f32.t.normal_(generator=torch.Generator(device="cuda").manual_seed(N))
+    f64 = lf.Field(lat, 1, lf.F64)
+    f64.t.copy_(f32.t)
+    for code, phi in ((lf.F32, f32), (lf.F64, f64)):
+        parts = lf.Particles(N, n, code, ids=True)
+        assert parts.addParticles(pos, vel, ids=np.arange(n, dtype=np.int64)) == n
+        parts.gather_kick_drift(phi, 1.0 / N, 0.01)
+        d = parts.download()
+        i = np.argsort(d["id"])
+        out[code] = (d["vel"][i], d["pos"][i])
+    dv = out[lf.F32][0] - out[lf.F64][0]
+    assert np.linalg.norm(dv) / np.linalg.norm(out[lf.F64][0]) <= 2e-6
+    dx = np.abs(out[lf.F32][1] - out[lf.F64][1])
+    assert np.max(np.minimum(dx, 1.0 - dx)) * N <= 1e-4
