@@ -381,32 +381,33 @@ __device__ __forceinline__ int drift_cell(int N, double dt, int cx, int cy, int 
 }
 
 // ---------------------------------------------------------------- scatter (counting sort)
-// Counting-sort scatter, SCAT_PER particles per thread (1024 per block): every load is in
+// Counting-sort scatter, PER particles per thread (1024 or 256 per block): every load is in
 // flight before the slots are claimed.  Slots: per wave, lanes with equal new buckets form
 // groups (leader loop) whose leader adds the group size to the bucket's entry in an LDS hash
 // table (one CAS to insert the key); after a barrier one global atomic per distinct bucket of
 // the block reserves the range, and after a second barrier every particle stores at
 // start[b] + base + rank.  A re-bucketing block sees a few buckets (the source is bucket
-// ordered); a block of an unordered source (initial sort) at most 1024, for which the
-// 2048-slot table has room.
-static constexpr int SCAT_PER = 4;
-static constexpr int SCAT_HT = 2048;
-
-template <bool DRIFT>
+// ordered); a block of an unordered source (initial sort) at most one per particle, for which the
+// table of twice as many slots has room.  Four per thread, or one where that fills less than
+// the chip (sort_into_other).
+template <bool DRIFT, int PER>
 __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa32 dst, Geo g,
                                                       int *__restrict__ cursor, int plw, double dt) {
-    __shared__ int hkey[SCAT_HT];
-    __shared__ int hval[SCAT_HT];  // group counts, then the bucket's reserved base
-    for (int i = threadIdx.x; i < SCAT_HT; i += 256) {
+    constexpr int HT = 512 * PER;
+    constexpr int HASH = PER == 4 ? 21 : 23;  // the key's top bits
+    static_assert(HT == 1 << (32 - HASH), "table size");
+    __shared__ int hkey[HT];
+    __shared__ int hval[HT];  // group counts, then the bucket's reserved base
+    for (int i = threadIdx.x; i < HT; i += 256) {
         hkey[i] = -1;
         hval[i] = 0;
     }
-    const int64_t i0 = (int64_t)blockIdx.x * (256 * SCAT_PER) + threadIdx.x;
-    int cell[SCAT_PER];
-    float o[SCAT_PER][3], v[SCAT_PER][3], m[SCAT_PER];
-    int64_t id[SCAT_PER];
+    const int64_t i0 = (int64_t)blockIdx.x * (256 * PER) + threadIdx.x;
+    int cell[PER];
+    float o[PER][3], v[PER][3], m[PER];
+    int64_t id[PER];
 #pragma unroll
-    for (int k = 0; k < SCAT_PER; ++k) {
+    for (int k = 0; k < PER; ++k) {
         const int64_t i = i0 + k * 256;
         cell[k] = i < np ? src.cell[i] : -1;
         m[k] = 0.f;
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa
     }
     if constexpr (DRIFT) {
 #pragma unroll
-        for (int k = 0; k < SCAT_PER; ++k) {
+        for (int k = 0; k < PER; ++k) {
             if (cell[k] < 0) continue;
             int cx, cy, cz;
             decode_cell(cell[k], g, cx, cy, cz);
@@ -433,9 +434,9 @@ __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa
     }
     __syncthreads();
     const int lane = lane_id();
-    int bk[SCAT_PER], ent[SCAT_PER], rank[SCAT_PER];
+    int bk[PER], ent[PER], rank[PER];
 #pragma unroll
-    for (int k = 0; k < SCAT_PER; ++k) {
+    for (int k = 0; k < PER; ++k) {
         const bool act = cell[k] >= 0;
         bk[k] = act ? bucket_of(cell[k], g) : 0;
         ent[k] = 0;
@@ -447,11 +448,11 @@ __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa
             const unsigned long long grp = __ballot(act && bk[k] == lkey);
             int e = 0, r0 = 0;
             if (lane == leader) {
-                e = (int)(((unsigned)lkey * 2654435761u) >> 21) & (SCAT_HT - 1);
+                e = (int)(((unsigned)lkey * 2654435761u) >> HASH) & (HT - 1);
                 for (;;) {
                     const int old = atomicCAS(&hkey[e], -1, lkey);
                     if (old == -1 || old == lkey) break;
-                    e = (e + 1) & (SCAT_HT - 1);
+                    e = (e + 1) & (HT - 1);
                 }
                 r0 = atomicAdd(&hval[e], __popcll(grp));
             }
@@ -465,13 +466,13 @@ __global__ __launch_bounds__(256) void scatter_kernel(int64_t np, Soa32 src, Soa
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < SCAT_HT; i += 256) {
+    for (int i = threadIdx.x; i < HT; i += 256) {
         const int key = hkey[i];
         if (key >= 0) hval[i] = atomicAdd(&cursor[key], hval[i]);
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < SCAT_PER; ++k) {
+    for (int k = 0; k < PER; ++k) {
         if (cell[k] < 0) continue;
         const int64_t j = (int64_t)hval[ent[k]] + rank[k];
         dst.cell[j] = cell[k];
@@ -2767,14 +2768,24 @@ static int scan_buckets(lf2mi_parts_s *p, hipStream_t st) {
     return brick_scan(S, (int)n, st);
 }
 
+static constexpr int64_t SCAT_FULL = 256 * 1024;  // four particles per thread fill 256 CUs
+
 // counting sort of buffer `src` (counts already in bcount) into buffer 1 - src; drift: the
 // particles move by dt on the way
 static int sort_into_other(lf2mi_parts_s *p, int src, int64_t nsrc, bool drift, double dt, hipStream_t st) {
     if (int rc = scan_buckets(p, st)) return rc;
     LF2MI_PROF("rebucket_scatter", st);
-    const unsigned grid = grid1(nsrc, 256 * SCAT_PER);
-    if (drift) scatter_kernel<true><<<grid, 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor, p->plw, dt);
-    else scatter_kernel<false><<<grid, 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor, p->plw, dt);
+    auto launch = [&](auto kernel, int per) {
+        kernel<<<grid1(nsrc, 256 * per), 256, 0, st>>>(nsrc, p->b32[src], p->b32[1 - src], p->g, p->cursor, p->plw, dt);
+    };
+    // one particle per thread while four leave CUs without a block (32^3 particles: 10.1 -> 4.9 us)
+    if (nsrc < SCAT_FULL) {
+        if (drift) launch(scatter_kernel<true, 1>, 1);
+        else launch(scatter_kernel<false, 1>, 1);
+    } else {
+        if (drift) launch(scatter_kernel<true, 4>, 4);
+        else launch(scatter_kernel<false, 4>, 4);
+    }
     LF2MI_LAUNCHED();
     p->cur = 1 - src;
     return LF2MI_OK;

@@ -13,7 +13,7 @@ from gpu_util import announce  # noqa: E402
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("N,n", [(8, 1), (8, 1023), (20, 4097), (64, 70001)])
+@pytest.mark.parametrize("N,n", [(8, 1), (8, 1023), (20, 4097), (64, 70001), (64, 300001)])
 @pytest.mark.parametrize("speed", [0.01, 3.0])
 def test_drift_moves_every_particle_once(N, n, speed):
     announce(f"drift N={N} n={n} speed={speed}")
