@@ -1502,7 +1502,7 @@ __device__ __forceinline__ int kick_store(const GkdArgs &A, int p, int cx, int c
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         v[d] = vin[d] + A.dt_kick * a[d];
-        A.s.vel[d][p] = v[d];
+        if (A.phi) A.s.vel[d][p] = v[d];  // a drift alone leaves it (1.5M particles: 29 -> 21 us)
     }
     vmax = fmaxf(vmax, v[0] * v[0] + v[1] * v[1] + v[2] * v[2]);
     return A.drift ? drift_cell(A.g.N, A.dt_drift, cx, cy, cz, u, v, o) : 0;
