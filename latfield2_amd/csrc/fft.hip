@@ -354,6 +354,64 @@ __global__ __launch_bounds__(WG) void fft_strided_kernel(StridedArgs<T> A) {
     }
 }
 
+// ---------------------------------------------------------------- small lattices: whole planes
+// One workgroup per column, whose N x N plane stays in LDS: MODE 0 the forward z and y transforms,
+// 2 the inverse y and z ones, 1 the Poisson solve's forward, Green and inverse ones.  Below N = 64
+// a strided pass is a launch's latency; their sums against this kernel, microseconds: solve, FP32 /
+// FP64, N = 16 8.4 -> 4.3 / 9.2 -> 4.5, 32 9.2 -> 6.0 / 9.9 -> 6.2, 40 10.4 -> 8.4 / 10.4 -> 9.4, 48
+// 11.3 -> 11.2 / 10.7 -> 13.9, 64 (FP32) 11.1 -> 13.5.  A column's values lie one to a 128-byte
+// line, which bounds it; neighbouring columns go to one XCD, whose L2 then has the line.
+// in_es / out_es are the strides of y, in_bs / out_bs those of z.
+template <typename T, int N, int WG, int MODE>
+__global__ __launch_bounds__(WG) void fft_plane_kernel(StridedArgs<T> A) {
+    using V = cplx<T>;
+    constexpr int ES = N + 1;
+    extern __shared__ unsigned char smem_raw[];
+    V *lds = reinterpret_cast<V *>(smem_raw), *twl = lds + N * ES;
+    const int per = gridDim.x / 8, rem = gridDim.x % 8, xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
+    const int col = xcd * per + min(xcd, rem) + slot;
+    const V *in = A.in + A.in_col0 + col;
+    V *out = A.out + A.out_col0 + col;
+    // the first pass uses no twiddles, and the barrier after it orders these stores
+    for (int i = threadIdx.x; i < N; i += WG) twl[i] = A.tw[i];
+    // the tile is [z][y] for the z transforms (line y) and [y][z] for the y transforms (line z):
+    // the last pass of the transform before writes it the other way round
+    auto ld = [lds](int l, int e) { return lds[e * ES + l]; };
+    auto turn = [lds](int l, int e, V v) { lds[l * ES + e] = v; };
+    auto load_z = [&](int y, int z) { return in[y * A.in_es + z * A.in_bs]; };
+    auto load_y = [&](int z, int y) { return in[y * A.in_es + z * A.in_bs]; };
+    auto store_z = [&](int y, int z, V v) { out[y * A.out_es + z * A.out_bs] = v; };
+    auto store_y = [&](int z, int y, V v) { out[y * A.out_es + z * A.out_bs] = v; };
+    if constexpr (MODE == 0) {
+        tile_fft_io<T, N, N, ES, WG, -1, 0, false, true>(lds, twl, load_z, turn);
+        tile_fft_io<T, N, N, ES, WG, -1, 0, true, false>(lds, twl, ld, store_y);
+    } else if constexpr (MODE == 2) {
+        tile_fft_io<T, N, N, ES, WG, +1, 0, false, true>(lds, twl, load_y, turn);
+        tile_fft_io<T, N, N, ES, WG, +1, 0, true, false>(lds, twl, ld, store_z);
+    } else {
+        const int kx = col / A.C;
+        const T sx = sizeof(T) == 4 ? (T)A.green_sf[kx] : (T)A.green_s[kx];
+        const T gsc = (T)A.green_scale;
+        auto green_store = [&](int z, int y, V v) {  // as the strided pass
+            const T sy = sizeof(T) == 4 ? (T)A.green_sf[y] : (T)A.green_s[y];
+            const T sz = sizeof(T) == 4 ? (T)A.green_sf[z] : (T)A.green_s[z];
+            const T k2 = sx + sy + sz;
+            T g = T(0);
+            if (k2 > T(0)) {
+                if constexpr (sizeof(T) == 4) g = -gsc * __builtin_amdgcn_rcpf(k2);
+                else g = -gsc / k2;
+            }
+            v.x *= g;
+            v.y *= g;
+            lds[y * ES + z] = v;
+        };
+        tile_fft_io<T, N, N, ES, WG, -1, 0, false, true>(lds, twl, load_z, turn);
+        tile_fft_io<T, N, N, ES, WG, -1, 0, true, true>(lds, twl, ld, green_store);
+        tile_fft_io<T, N, N, ES, WG, +1, 0, true, true>(lds, twl, ld, turn);
+        tile_fft_io<T, N, N, ES, WG, +1, 0, true, false>(lds, twl, ld, store_z);
+    }
+}
+
 // ---------------------------------------------------------------- x pass, R2C
 // Block = P row pairs x C components = P*C complex lines; line (p, c) carries rows
 // (2p, 2p+1) of component c as re/im.  Row r = y + N z of the real interior.
@@ -790,6 +848,26 @@ static int launch_strided(StridedArgs<T> A, int S, int mode, int nbatch, hipStre
     return LF2MI_OK;
 }
 
+// lattices whose y and z transforms run on whole planes (figures at the kernel)
+static constexpr int PLANE_N = 40;
+
+template <typename T, int N>
+static int launch_plane(const StridedArgs<T> &A, int mode, hipStream_t st) {
+    if constexpr (N <= PLANE_N) {
+        constexpr int WG = N <= 32 ? 256 : 512;
+        LF2MI_PROF(mode == 1 ? "fft_plane_green" : (mode == 0 ? "fft_plane_fwd" : "fft_plane_inv"), st);
+        const size_t shm = sizeof(cplx<T>) * (N * (N + 1) + N);
+        const unsigned grid = (unsigned)A.ncols;
+        if (mode == 0) fft_plane_kernel<T, N, WG, 0><<<grid, WG, shm, st>>>(A);
+        else if (mode == 1) fft_plane_kernel<T, N, WG, 1><<<grid, WG, shm, st>>>(A);
+        else fft_plane_kernel<T, N, WG, 2><<<grid, WG, shm, st>>>(A);
+        LF2MI_LAUNCHED();
+        return LF2MI_OK;
+    } else {
+        return fail(LF2MI_EUNSUPPORTED, "no plane pass for N = %d", N);
+    }
+}
+
 template <typename T, int N, int L>
 static int launch_x_tile(const XArgs<T> &A, int S, hipStream_t st) {
     constexpr int WG = Tune<T>::template x_WG<N, L>();
@@ -890,6 +968,9 @@ static int launch_c2c(const C2CArgs<T> &A, int pass, int S, hipStream_t st) {
 template <typename T> static int strided(int N, const StridedArgs<T> &A, int S, int mode, int nb, hipStream_t st) {
     LF2MI_DISPATCH_N(N, (launch_strided<T, NN>(A, S, mode, nb, st)));
 }
+template <typename T> static int plane(int N, const StridedArgs<T> &A, int mode, hipStream_t st) {
+    LF2MI_DISPATCH_N(N, (launch_plane<T, NN>(A, mode, st)));
+}
 template <typename T> static int xpass(int N, const XArgs<T> &A, int S, hipStream_t st) {
     LF2MI_DISPATCH_N(N, (launch_x<T, NN>(A, S, st)));
 }
@@ -950,6 +1031,15 @@ static int forward(lf2mi_fft_plan_s *p, const void *rfield, cplx<T> *kout, KGeo 
     A.ncols = (N / 2 + 1) * p->C;
     A.tw = (const cplx<T> *)p->tw;
     A.C = p->C;
+    if (N <= PLANE_N) {
+        A.out = kout;
+        A.out_col0 = kg.col0;
+        A.in_es = wg.s2;
+        A.in_bs = wg.s1;
+        A.out_es = kg.s2;
+        A.out_bs = kg.s1;
+        return plane<T>(N, A, 0, st);
+    }
     // z pass in place on W: along slot1, batches over slot2
     A.in_es = A.out_es = wg.s1;
     A.in_bs = A.out_bs = wg.s2;
@@ -982,13 +1072,17 @@ static int backward(lf2mi_fft_plan_s *p, const cplx<T> *kin, KGeo kg, void *rfie
     A.out_es = wg.s2;
     A.in_bs = kg.s1;
     A.out_bs = wg.s1;
-    if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
-    // z pass in place on W along slot1
-    A.in = W;
-    A.in_col0 = wg.col0;
-    A.in_es = A.out_es = wg.s1;
-    A.in_bs = A.out_bs = wg.s2;
-    if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
+    if (N <= PLANE_N) {
+        if (int rc = plane<T>(N, A, 2, st)) return rc;
+    } else {
+        if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
+        // z pass in place on W along slot1
+        A.in = W;
+        A.in_col0 = wg.col0;
+        A.in_es = A.out_es = wg.s1;
+        A.in_bs = A.out_bs = wg.s2;
+        if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
+    }
     XArgs<T> X{};
     X.kin = W;
     X.real_out = (T *)rfield;
@@ -1082,18 +1176,24 @@ static int poisson(lf2mi_fft_plan_s *p, const void *rho, void *phi, double shift
     A.green_s = p->green_s;
     A.green_sf = p->green_sf;
     A.green_scale = scale;
-    // z forward along slot1
-    A.in_es = A.out_es = wg.s1;
-    A.in_bs = A.out_bs = wg.s2;
-    if (int rc = strided<T>(N, A, -1, 0, N, st)) return rc;
-    // y forward + Green + y inverse along slot2 (batch = slot1 = kz)
-    A.in_es = A.out_es = wg.s2;
-    A.in_bs = A.out_bs = wg.s1;
-    if (int rc = strided<T>(N, A, -1, 1, N, st)) return rc;
-    // z inverse along slot1
-    A.in_es = A.out_es = wg.s1;
-    A.in_bs = A.out_bs = wg.s2;
-    if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
+    if (N <= PLANE_N) {
+        A.in_es = A.out_es = wg.s2;
+        A.in_bs = A.out_bs = wg.s1;
+        if (int rc = plane<T>(N, A, 1, st)) return rc;
+    } else {
+        // z forward along slot1
+        A.in_es = A.out_es = wg.s1;
+        A.in_bs = A.out_bs = wg.s2;
+        if (int rc = strided<T>(N, A, -1, 0, N, st)) return rc;
+        // y forward + Green + y inverse along slot2 (batch = slot1 = kz)
+        A.in_es = A.out_es = wg.s2;
+        A.in_bs = A.out_bs = wg.s1;
+        if (int rc = strided<T>(N, A, -1, 1, N, st)) return rc;
+        // z inverse along slot1
+        A.in_es = A.out_es = wg.s1;
+        A.in_bs = A.out_bs = wg.s2;
+        if (int rc = strided<T>(N, A, +1, 0, N, st)) return rc;
+    }
     XArgs<T> X{};
     X.kin = W;
     X.real_out = (T *)phi;

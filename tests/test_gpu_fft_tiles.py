@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("prec,tol", [("f64", 1e-12), ("f32", 2e-6)])
 @pytest.mark.parametrize("N,h,kh,C", [(8, 0, 1, 3), (48, 1, 1, 6), (96, 1, 0, 3), (128, 0, 1, 1), (192, 1, 0, 1),
-                                      (256, 1, 1, 3), (256, 0, 0, 1)])
+                                      (256, 1, 1, 3), (256, 0, 0, 1), (40, 1, 1, 6), (10, 2, 0, 3)])
 def test_fft_tiles_both_ways_match_oracle(prec, tol, N, h, kh, C):
     announce(f"fft tiles {prec} N={N} h={h} kh={kh} C={C}")
     code = lf.F32 if prec == "f32" else lf.F64
@@ -40,3 +40,23 @@ def test_fft_tiles_both_ways_match_oracle(prec, tol, N, h, kh, C):
     orc.fft_c2r(np.ascontiguousarray(kin), ref, N, h, kh)
     assert close(real_np(r), ref)
     assert np.array_equal(kfield_np(k), kin)
+
+
+@pytest.mark.parametrize("prec,tol", [("f64", 1e-12), ("f32", 2e-6)])
+@pytest.mark.parametrize("N", [8, 10, 12, 20, 24, 32, 40, 48])
+def test_small_solves_match_numpy(prec, tol, N):
+    """the solve on whole planes (up to 40) and on strided passes against the FP64 transform"""
+    announce(f"small solve {prec} N={N}")
+    code = lf.F32 if prec == "f32" else lf.F64
+    lat = lf.Lattice(3, N, 1)
+    rho, phi = lf.Field(lat, 1, code), lf.Field(lat, 1, code)
+    rho.t.normal_()
+    s = slice(1, N + 1)
+    x = real_np(rho)[s, s, s].astype(np.float64)
+    lf.poisson_solve(lf.PlanFFT(rho, None), rho, phi, 0.25, 1.0 / N ** 3)
+    torch.cuda.synchronize()
+    sn = 4.0 * N ** 2 * np.sin(np.pi * np.arange(N) / N) ** 2
+    k2 = sn[:, None, None] + sn[None, :, None] + sn[None, None, :]
+    k2[0, 0, 0] = np.inf
+    want = np.fft.ifftn(-np.fft.fftn(x - 0.25, axes=(0, 1, 2)) / k2[..., None], axes=(0, 1, 2)).real
+    assert rel_l2(real_np(phi)[s, s, s], want) <= tol
