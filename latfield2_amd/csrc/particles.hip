@@ -592,7 +592,7 @@ static constexpr int DEP_MERGE = 8;  // items one deposit workgroup takes
 //    then written once, TILE_X consecutive x per row (stored, or added to the field).  The layer
 //    that belongs to the bricks above in y or z goes to two shell buffers and the tile's last
 //    x = 8 plane to a seam buffer, one value per node.  No global atomics, no sort.
-//  * dense_groups_kernel + dense_body: the bricks with dense_min or more particles,
+//  * the work list of brick_starts_kernel + dense_body: the bricks with dense_min or more particles,
 //    in groups of up to DEP_MERGE items (a work list shared out statically among persistent
 //    workgroups); each particle's 8 terms go straight into a 9^3 LDS window (no sort: a
 //    wave's 64 particles of a crowded brick rarely share a cell), added to the field with one
@@ -1449,23 +1449,40 @@ struct FxScales {
     double inv[6];
 };
 
-// field += fixed-point sums (set: = them), which are cleared for the next deposit on the way.
-// Clearing both before every deposit took two more launches and passes (128^3: 10.6 of 162 us
-// of a step).
-template <bool SET>
-__device__ __forceinline__ void fixed_take(unsigned long long *__restrict__ fx, float *__restrict__ f, int64_t i, double scale) {
-    const long long q = (long long)fx[i];
-    if (q) fx[i] = 0ull;
-    if (SET) f[i] = (float)((double)q * scale);
-    else if (q) f[i] += (float)((double)q * scale);
+// field += fixed-point sums (SET: = them), which are cleared for the next deposit on the way
+// (clear; the tiles deposit stores every sum, and leaves that out).  Clearing both before every
+// deposit took two more launches and passes (a step at 128^3 162 -> 147 us; added to a field,
+// 128^3 43 -> 32, 256^3 229 -> 198, its vector kind 741 -> 423, 512^3 1720 -> 1490).
+// scale(i): the units of value i; FX_PER loads of a thread in flight together.
+static constexpr int FX_PER = 4;
+template <bool SET, class Scale>
+__device__ __forceinline__ void fixed_take(unsigned long long *__restrict__ fx, float *__restrict__ f, int64_t n, int clear,
+                                           Scale &&scale) {
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i0 < n; i0 += FX_PER * stride) {
+        long long q[FX_PER];
+        float old[FX_PER];
+#pragma unroll
+        for (int k = 0; k < FX_PER; ++k) {
+            const int64_t i = i0 + k * stride;
+            q[k] = i < n ? (long long)fx[i] : 0;
+            old[k] = !SET && i < n ? f[i] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < FX_PER; ++k) {
+            const int64_t i = i0 + k * stride;
+            if (i >= n) break;
+            if (clear && q[k]) fx[i] = 0ull;
+            if (SET) f[i] = (float)((double)q[k] * scale(i));
+            else if (q[k]) f[i] = old[k] + (float)((double)q[k] * scale(i));
+        }
+    }
 }
 // component c of site i at fx[i C + c], in units of 1 / S.inv[c]
 template <bool SET>
 __global__ void fixed_to_field_c_kernel(unsigned long long *__restrict__ fx, float *__restrict__ f, int64_t n, int C,
-                                        FxScales S) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
-        fixed_take<SET>(fx, f, i, S.inv[i % C]);
+                                        int clear, FxScales S) {
+    fixed_take<SET>(fx, f, n, clear, [&](int64_t i) { return S.inv[i % C]; });
 }
 __global__ void fill_u64_kernel(unsigned long long *__restrict__ p, int64_t n) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -1473,9 +1490,9 @@ __global__ void fill_u64_kernel(unsigned long long *__restrict__ p, int64_t n) {
 }
 
 template <bool SET>
-__global__ void fixed_to_field_kernel(unsigned long long *__restrict__ fx, float *__restrict__ f, int64_t n, double scale) {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) fixed_take<SET>(fx, f, i, scale);
+__global__ void fixed_to_field_kernel(unsigned long long *__restrict__ fx, float *__restrict__ f, int64_t n, int clear,
+                                      double scale) {
+    fixed_take<SET>(fx, f, n, clear, [scale](int64_t) { return scale; });
 }
 
 // ---------------------------------------------------------------- gather + kick + drift (F32)
@@ -2153,7 +2170,7 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Arg
 
 // The same windows for the FP32 container, whose buckets are its bricks (any edge up to 8):
 // one workgroup per group of up to DEP_MERGE items of a brick, or a share of the groups of a
-// work list (dense_groups_kernel).  The terms' products are FP32.
+// work list (brick_starts_kernel).  The terms' products are FP32.
 template <int KIND, typename ACC>
 __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs A, const int2 *__restrict__ groups,
                                                                         const int *__restrict__ ngroups) {
@@ -2614,6 +2631,7 @@ struct lf2mi_parts_s {
     unsigned long long *fx;
     int64_t fx_n;
     int fx_used;  // fx is not cleared (new, or an error between a deposit and its taking)
+    int fx_halo;  // -1, or the halo of a tiles deposit whose interior sums fx may still hold
     void *shell;          // shell and seam buffers of the tiles deposit kernel (grown on demand)
     int64_t shell_bytes;
     unsigned int *vmax_f32;
@@ -3796,13 +3814,16 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
             LF2MI_HIP(hipMalloc((void **)&p->fx, n * sizeof(unsigned long long)));
             p->fx_n = n;
             p->fx_used = 1;
+            p->fx_halo = -1;
         }
-        // every deposit leaves the buffer cleared; a captured one, which runs later and perhaps
-        // after one that failed, clears it first
+        // a deposit leaves the buffer cleared, or, by the tiles, with the interior that the next
+        // such deposit stores again; a captured one, which runs later and perhaps after one that
+        // failed, clears it first and leaves it cleared
+        const bool tiles = tiles_path(p, kind, target, pm);
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         LF2MI_HIP(hipStreamIsCapturing(st, &cap));
         const bool captured = cap != hipStreamCaptureStatusNone;
-        if (p->fx_used || captured) {
+        if (p->fx_used || captured || (p->fx_halo >= 0 && !(tiles && p->fx_halo == halo))) {
             fill_u64_kernel<<<(unsigned)std::min<int64_t>(grid1(p->fx_n), 65536), 256, 0, st>>>(p->fx, p->fx_n);
             LF2MI_LAUNCHED();
         }
@@ -3852,8 +3873,8 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
                                                    "deposit_f32_vecvec_fixed64", "deposit_f32_vector_ngp_fixed64",
                                                    "deposit_f32_symtensor_ngp_fixed64"};
             LF2MI_PROF(namesfx[kind], st);
-            if (tiles_path(p, kind, target, pm)) {
-                // the fixed-point buffer starts cleared, so its interior can be stored
+            if (tiles) {
+                // the sums of the interior are stored
                 if (int rc = launch_tiles_dense<unsigned long long>(p, A, true, false, st)) return rc;
             } else {
                 switch (kind) {
@@ -3868,14 +3889,18 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
         }
         {
             LF2MI_PROF("fixed_to_field", st);
-            const unsigned gf = (unsigned)std::min<int64_t>(grid1(n), 65536);
+            const unsigned gf = (unsigned)std::min<int64_t>(grid1(n, 256 * FX_PER), 65536);
             float *f = (float *)field;
-            if (C == 1 && overwrite) fixed_to_field_kernel<true><<<gf, 256, 0, st>>>(p->fx, f, n, S.inv[0]);
-            else if (C == 1) fixed_to_field_kernel<false><<<gf, 256, 0, st>>>(p->fx, f, n, S.inv[0]);
-            else if (overwrite) fixed_to_field_c_kernel<true><<<gf, 256, 0, st>>>(p->fx, f, n, C, S);
-            else fixed_to_field_c_kernel<false><<<gf, 256, 0, st>>>(p->fx, f, n, C, S);
+            const int clear = captured || !tiles;
+            if (C == 1 && overwrite) fixed_to_field_kernel<true><<<gf, 256, 0, st>>>(p->fx, f, n, clear, S.inv[0]);
+            else if (C == 1) fixed_to_field_kernel<false><<<gf, 256, 0, st>>>(p->fx, f, n, clear, S.inv[0]);
+            else if (overwrite) fixed_to_field_c_kernel<true><<<gf, 256, 0, st>>>(p->fx, f, n, C, clear, S);
+            else fixed_to_field_c_kernel<false><<<gf, 256, 0, st>>>(p->fx, f, n, C, clear, S);
             LF2MI_LAUNCHED();
-            if (!captured) p->fx_used = 0;
+            if (!captured) {
+                p->fx_used = 0;
+                p->fx_halo = tiles ? halo : -1;
+            }
         }
         return LF2MI_OK;
     }

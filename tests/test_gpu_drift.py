@@ -65,3 +65,33 @@ def test_sparse_gather_matches_fp64(N):
     assert np.linalg.norm(dv) / np.linalg.norm(out[lf.F64][0]) <= 2e-6
     dx = np.abs(out[lf.F32][1] - out[lf.F64][1])
     assert np.max(np.minimum(dx, 1.0 - dx)) * N <= 1e-4
+
+
+def test_fixed_deposits_leave_nothing_behind():
+    """The fixed-point sums stay in the container between deposits: after one of any kind, target
+    and halo, the next must be bit for bit that of a container without a past (integer sums do
+    not depend on the order of the particles).  Few particles that move, so that most nodes with
+    a value have none the next time."""
+    N, n = 64, 4001
+    announce("fixed deposits one after the other")
+    rng = np.random.default_rng(5)
+    parts = lf.Particles(N, n, lf.F32, mass=0.5)
+    assert parts.addParticles(rng.random((n, 3)), rng.standard_normal((n, 3))) == n
+    fields = {}
+    for kind, C, target, halo in ((lf.PROJ_SCALAR, 1, lf.DEP_PERIODIC, 1), (lf.PROJ_SCALAR, 1, lf.DEP_PERIODIC, 1),
+                                  (lf.PROJ_SCALAR, 1, lf.DEP_PERIODIC_SET, 2), (lf.PROJ_VECTOR, 3, lf.DEP_PERIODIC, 1),
+                                  (lf.PROJ_SCALAR, 1, lf.DEP_PERIODIC_SET, 1), (lf.PROJ_SCALAR, 1, lf.DEP_UNFOLDED, 1),
+                                  (lf.PROJ_SCALAR, 1, lf.DEP_PERIODIC, 2), (lf.PROJ_VECVEC, 6, lf.DEP_UNFOLDED, 1),
+                                  (lf.PROJ_VECTOR, 3, lf.DEP_PERIODIC_SET, 2)):
+        parts.gather_kick_drift(None, 0.0, 0.01)
+        d = parts.download()
+        new = lf.Particles(N, n, lf.F32, mass=0.5)
+        assert new.addParticles(d["pos"], d["vel"]) == n
+        got, want = (lf.Field(lf.Lattice(3, N, halo), C, lf.F32) for _ in range(2))
+        start = 3.0 if target == lf.DEP_PERIODIC_SET else 0.0
+        for p, f in ((parts, got), (new, want)):
+            f.t.fill_(start)
+            p.deposit(kind, f, target, lf.ACC_FIXED64)
+        torch.cuda.synchronize()
+        assert torch.equal(got.t, want.t), (kind, target, halo)
+        assert float(want.t.abs().max()) > 0 and float((want.t == 0).double().mean()) > 0.3, (kind, target, halo)
