@@ -41,15 +41,15 @@ BRICK = 8
 # each scaled by what the counter reads for the run's 1 GiB device copy: FETCH_SIZE 256.1 MiB (factor 1024 / 256.1), WRITE_SIZE 1024.0 MiB
 # (factor 1).  Registry name -> (FETCH_SIZE, WRITE_SIZE) summed over the kernels it times.
 TRAFFIC_MIB = {
-    "rebucket_scatter": (1803.7, 3761.8),
-    "gkd_f32": (1818.8, 3011.8),
-    "gkd_f32_chunks": (1022.2, 668.7),
-    "deposit_f32_scalar": (619.1 + 920.7 + 0.5 + 0.1, 685.2 + 247.6 + 0.2 + 14.2),
+    "rebucket_scatter": (1794.2, 3760.3),
+    "gkd_f32": (1821.1, 1281.6),
+    "gkd_f32_chunks": (1017.1, 291.0),
+    "deposit_f32_scalar": (619.1 + 916.9, 685.2 + 252.5),
     "fft_x_r2c": (266.8, 520.0),
     "fft_x_c2r": (272.0, 515.0),
     "fft_strided_fwd": (272.1, 520.0),
     "fft_strided_inv": (272.1, 520.0),
-    "fft_y_green": (272.3, 586.0),
+    "fft_y_green": (275.2, 592.4),
 }
 FETCH_FACTOR, WRITE_FACTOR = 1024.0 / 256.1, 1.0
 
@@ -65,14 +65,15 @@ def measured_traffic(name: str) -> float | None:
 def algorithmic_bytes(name: str, N: int, Np: int, esz: int, np_sparse: int = 0) -> float | None:
     """compulsory HBM bytes of one launch of `name` (reads + writes of its data); the
     gather's item kernel takes the particles of bricks with at least GKD_DIRECT_MAX of
-    them and reads phi once, its chunk kernel the other np_sparse particles"""
+    them and reads phi once, its chunk kernel the other np_sparse particles; both read a
+    particle and write its velocity, the scatter evaluates the drift and moves it"""
     M = (N // 2 + 1) * N * N
     c = 2 * esz  # complex element
     table = {
         "deposit_f32_scalar": 16 * Np + 4 * N ** 3,
         "deposit_f64_scalar": 24 * Np + 8 * N ** 3,
-        "gkd_f32": 4 * N ** 3 + 56 * (Np - np_sparse),
-        "gkd_f32_chunks": 56 * np_sparse,
+        "gkd_f32": 4 * N ** 3 + 40 * (Np - np_sparse),
+        "gkd_f32_chunks": 40 * np_sparse,
         "gkd_f64": 8 * N ** 3 + 96 * Np,
         "fft_x_r2c": esz * N ** 3 + c * M,
         "fft_x_c2r": c * M + esz * N ** 3,
@@ -337,11 +338,11 @@ def main():
         v["GBps"] = round(b / (v["avg_ms"] * 1e-3) / 1e9, 1) if b else None
         v["avg_ms"] = round(v["avg_ms"], 4)
         v["ms_per_step"] = round(v["ms_per_step"], 4)
-    # the gather + kick + drift stage as a whole (chunk list, item kernel, chunk kernel)
-    gk = [k for k in ("gkd_chunk_list", "gkd_f32", "gkd_f32_chunks") if k in kernels]
+    # the gather + kick stage as a whole (item kernel, chunk kernel)
+    gk = [k for k in ("gkd_f32", "gkd_f32_chunks") if k in kernels]
     gms = sum(kernels[k]["ms_per_step"] for k in gk)
     gather_stage = {"kernels": gk, "ms_per_step": round(gms, 4), "sparse_particles": np_sparse,
-                    "GBps": round((4 * N ** 3 + 56 * Np) / (gms * 1e-3) / 1e9, 1) if gms else None}
+                    "GBps": round((4 * N ** 3 + 40 * Np) / (gms * 1e-3) / 1e9, 1) if gms else None}
     # the clustered deposit timed both ways on the same particles: FP32 float atomics and
     # int64 fixed point (2^-32 units, run-to-run reproducible, converted to FP32 after)
     dep = {}
