@@ -1617,8 +1617,7 @@ __device__ __forceinline__ void gkd_hist_flush(const GkdArgs &A, int b, const in
     atomicAdd(&A.next_counts[bx + NB * (by + NB * bz)], h27[t]);
 }
 
-template <int BC>
-__global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) {
+template <int BC> __device__ __forceinline__ void gkd_dense(const GkdArgs &A, int it) {
     constexpr int PW = MAXB + 3;  // phi window [o-1, o+B+1]
     constexpr int FW = MAXB + 1;  // force nodes [o, o+B]
     __shared__ float phw[PW * PW * PW];
@@ -1626,7 +1625,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) {
     __shared__ unsigned int red;
     __shared__ int h27[27];
     ItemRange r;
-    if (!item_range(blockIdx.x, A.start, A.istart, A.item_bucket, A.g, r)) return;
+    if (!item_range(it, A.start, A.istart, A.item_bucket, A.g, r)) return;
     if (A.chunked && A.start[r.b + 1] - A.start[r.b] < GKD_DIRECT_MAX) return;
     if (A.phi) {
         // one workgroup per GKD_MERGE consecutive items of a brick: one phi window and force
@@ -1745,6 +1744,8 @@ __global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) {
     if (A.vmax2 && threadIdx.x == 0) atomicMax(A.vmax2, red);
 }
 
+template <int BC> __global__ __launch_bounds__(DEP_WG) void gkd_f32_kernel(GkdArgs A) { gkd_dense<BC>(A, blockIdx.x); }
+
 // ---- sparse bricks: chunks along x
 // Runs of consecutive non-empty bricks of one brick row (same y, z) whose counts are below
 // GKD_DIRECT_MAX form chunks of at most GKD_CHUNK_B bricks (their particles are contiguous in
@@ -1768,8 +1769,7 @@ static_assert((DEP_WG / 64) * GKD_STAGE >= (MAXB + 3) * (MAXB + 3), "one batch o
 // claim, and a small window, whose 11-value rows would leave most of a wave idle (64^3 with 64
 // particles per brick 15.7 -> 6.5 us; both forms in one kernel cost the wide one a tenth).
 template <int BC, bool ONE>
-__global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4 *__restrict__ chunks,
-                                                           int *__restrict__ nchunk) {
+__device__ __forceinline__ void gkd_chunk(const GkdArgs &A, const int4 *__restrict__ chunks, int *__restrict__ nchunk) {
     constexpr int WXM = (ONE ? 1 : GKD_CHUNK_B) * MAXB + 3, WYM = MAXB + 3;
     constexpr int NHM = ((ONE ? 1 : GKD_CHUNK_B) + 2) * 9;
     __shared__ float win[WXM * WYM * WYM];
@@ -1917,6 +1917,22 @@ __global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4
         __syncthreads();
         if (threadIdx.x == 0) atomicMax(A.vmax2, red);
     }
+}
+
+template <int BC>
+__global__ __launch_bounds__(DEP_WG) void gkd_chunk_kernel(GkdArgs A, const int4 *__restrict__ chunks,
+                                                           int *__restrict__ nchunk) {
+    gkd_chunk<BC, false>(A, chunks, nchunk);
+}
+
+// small lattices: one launch, a workgroup per brick for the chunks, then those of the dense items
+// (one launch of two costs 4.5 us of a step: 64^3 lattice, 32^3 particles, two steps 109 -> 100)
+template <int BC>
+__global__ __launch_bounds__(DEP_WG) void gkd_small_kernel(GkdArgs A, const int4 *__restrict__ chunks,
+                                                           int *__restrict__ nchunk) {
+    const int nbk = (int)A.g.nbk;
+    if ((int)blockIdx.x < nbk) gkd_chunk<BC, true>(A, chunks, nchunk);
+    else gkd_dense<BC>(A, (int)blockIdx.x - nbk);
 }
 
 // ---------------------------------------------------------------- F64 plain path
@@ -3999,25 +4015,28 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
     A.drift = dt_drift != 0.0;
     if (vmax2) LF2MI_HIP(hipMemsetAsync(p->vmax_f32, 0, sizeof(unsigned int), st));
     const bool b8 = p->g.B == 8;
-    {
+    const unsigned items = (unsigned)item_grid(p);
+    if (A.chunked && chunk_width(p) == 1) {
         LF2MI_PROF("gkd_f32", st);
-        if (b8) gkd_f32_kernel<8><<<(unsigned)item_grid(p), DEP_WG, 0, st>>>(A);
-        else gkd_f32_kernel<0><<<(unsigned)item_grid(p), DEP_WG, 0, st>>>(A);
+        const unsigned grid = (unsigned)p->g.nbk + items;
+        if (b8) gkd_small_kernel<8><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+        else gkd_small_kernel<0><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
         LF2MI_LAUNCHED();
-    }
-    if (A.chunked) {
-        LF2MI_PROF("gkd_f32_chunks", st);
-        if (chunk_width(p) == 1) {
-            const unsigned grid = (unsigned)p->g.nbk;
-            if (b8) gkd_chunk_kernel<8, true><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
-            else gkd_chunk_kernel<0, true><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
-        } else {
-            // persistent: a few workgroups per CU walk the chunk list
-            const unsigned grid = (unsigned)std::min<int64_t>(p->g.nbk, 2048);
-            if (b8) gkd_chunk_kernel<8, false><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
-            else gkd_chunk_kernel<0, false><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+    } else {
+        {
+            LF2MI_PROF("gkd_f32", st);
+            if (b8) gkd_f32_kernel<8><<<items, DEP_WG, 0, st>>>(A);
+            else gkd_f32_kernel<0><<<items, DEP_WG, 0, st>>>(A);
+            LF2MI_LAUNCHED();
         }
-        LF2MI_LAUNCHED();
+        if (A.chunked) {
+            // persistent: a few workgroups per CU walk the chunk list
+            LF2MI_PROF("gkd_f32_chunks", st);
+            const unsigned grid = (unsigned)std::min<int64_t>(p->g.nbk, 2048);
+            if (b8) gkd_chunk_kernel<8><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+            else gkd_chunk_kernel<0><<<grid, DEP_WG, 0, st>>>(A, p->chunks, p->nchunk);
+            LF2MI_LAUNCHED();
+        }
     }
     // (the scan clears the claims)
     if (A.drift) {
