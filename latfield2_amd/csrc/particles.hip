@@ -1765,7 +1765,7 @@ static_assert((DEP_WG / 64) * GKD_STAGE >= (MAXB + 3) * (MAXB + 3), "one batch o
 // GKD_CHUNK_B bricks), the following one while this one's particles are processed.  Chunks cut
 // at fixed borders instead, a workgroup each, cost 0.74 ms against 0.62 at 512^3 (blobs): a
 // fourth more of them.
-// ONE: chunks of one brick each and no more of them than workgroups (small lattices): nothing to
+// ONE: chunks of one brick each, and a workgroup for every brick (small lattices): nothing to
 // claim, and a small window, whose 11-value rows would leave most of a wave idle (64^3 with 64
 // particles per brick 15.7 -> 6.5 us; both forms in one kernel cost the wide one a tenth).
 template <int BC, bool ONE>
@@ -2775,13 +2775,11 @@ static int b64_fill(lf2mi_parts_s *p, const double *pos, const double *vel, cons
     return LF2MI_OK;
 }
 
-// bricks per chunk of the sparse gather: fewer on small lattices, while that leaves less than 1024
-// chunks (four workgroups per CU)
-static int chunk_width(const lf2mi_parts_s *p) {
-    int w = GKD_CHUNK_B;
-    while (w > 1 && p->g.nbk / w < 1024) w /= 2;
-    return w;
-}
+// bricks per chunk of the sparse gather: one below 8192 bricks, where more would leave fewer than
+// four chunks per CU or need the launch of their own (two steps, chunks of one and of four: 128^3
+// uniform 210 against 232 us, clustered 289 / 313, 160^3 clustered 498 / 525, dense 276 / 277;
+// of one and of eight: 192^3 uniform 421 / 399, 256^3 uniform 825 / 745)
+static int chunk_width(const lf2mi_parts_s *p) { return p->g.nbk < 8192 ? 1 : GKD_CHUNK_B; }
 
 // exclusive scans of bcount -> bstart and the cursors, items -> istart, and the dense bricks'
 // groups; bcount comes out cleared

@@ -39,10 +39,10 @@ def test_drift_moves_every_particle_once(N, n, speed):
         assert np.array_equal(parts.cell_counts().cpu().numpy(), np.bincount(c, minlength=N ** 3))
 
 
-@pytest.mark.parametrize("N", [8, 20, 64, 96, 104])
+@pytest.mark.parametrize("N", [8, 20, 64, 160, 168])
 def test_sparse_gather_matches_fp64(N):
-    """Bricks of few particles, in chunks of one brick (up to 12^3 bricks of 8^3 cells) and of
-    several (from 13^3), against the FP64 container.  White noise as the potential: its
+    """Bricks of few particles, in chunks of one brick (up to 20^3 bricks of 8^3 cells) and of
+    several (from 21^3), against the FP64 container.  White noise as the potential: its
     differences cancel nothing, so a velocity carries some 30 FP32 roundings of 6e-8."""
     announce(f"sparse gather N={N}")
     n = 20 * ((N + 7) // 8) ** 3 + 3
