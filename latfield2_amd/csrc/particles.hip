@@ -2150,6 +2150,10 @@ __device__ __forceinline__ void bw_flush(const W *__restrict__ win, F *__restric
 // below this many particles per brick the index, the windows' zeroing and their flush cost an
 // FP64 container more than its particles' own atomics
 static constexpr int64_t B64_OCC = 24;
+// and below this many particles altogether the index's launches cost more than the atomics: two
+// steps, by bricks and particle by particle, 20 000 particles on 32^3 129 and 105 us, on 40^3 126
+// and 100; 40 000 on 32^3 139 / 144, on 64^3 127 / 122; 80 000 on 64^3 138 / 172, on 96^3 163 / 200
+static constexpr int64_t B64_NP = 40000;
 static constexpr int B64_MERGE = 8;  // items per workgroup
 
 template <int KIND>
@@ -2704,7 +2708,9 @@ static int64_t b64_bricks(int N) {
     return nb * nb * nb;
 }
 // whether the F64 container's brick index is kept for its particles
-static bool b64_used(const lf2mi_parts_s *p) { return p->bricks && p->np >= B64_OCC * b64_bricks(p->N); }
+static bool b64_used(const lf2mi_parts_s *p) {
+    return p->bricks && p->np >= std::max(B64_NP, B64_OCC * b64_bricks(p->N));
+}
 template <typename T> static int reorder_one(lf2mi_parts_s *p, T *a, int stride, hipStream_t st) {
     const unsigned g = grid1(p->np);
     reorder_gather_kernel<T><<<g, 256, 0, st>>>(p->np, a, stride, p->bb.list, (T *)p->tmp);
@@ -3157,7 +3163,7 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
         A((void **)&p->vmax_f64, sizeof(unsigned long long));
         // the windows need distinct images of a brick's nodes, the scans at most 4096 blocks
         const int64_t nbk = b64_bricks(N);
-        p->bricks = N >= 16 && brick_blocks(nbk) <= 4096;
+        p->bricks = N >= 16 && brick_blocks(nbk) <= 4096 && capacity >= B64_NP;
         if (p->bricks) {
             A((void **)&p->bb.start, (size_t)(nbk + 1) * sizeof(int));
             A((void **)&p->bb.istart, (size_t)(nbk + 1) * sizeof(int));

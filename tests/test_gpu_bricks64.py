@@ -1,7 +1,7 @@
 """FP64 container with its brick index (LDS windows of the deposits and of the gather) against
-the FP64 oracle, on both sides of the particles-per-brick rule, with bricks that are partial
-at the upper faces (N not a multiple of 8), through several steps that move particles across
-bricks.  Bars: PM steps 1e-10 (FP64 sums in another order, carried through the solve),
+the FP64 oracle, on both sides of the rules on particles per brick and in all, with bricks that
+are partial at the upper faces (N not a multiple of 8), through several steps that move particles
+across bricks.  Bars: PM steps 1e-10 (FP64 sums in another order, carried through the solve),
 deposits 1e-12."""
 import numpy as np
 import pytest
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("N,n", [(16, 24 * 8 - 1), (16, 24 * 8), (16, 9000), (20, 24 * 27), (20, 30011),
-                                 (40, 24 * 125 - 1), (40, 70001)])
+                                 (40, 24 * 125 - 1), (40, 70001), (16, 39999), (16, 40000), (20, 45011)])
 def test_f64_steps_and_projections_match_oracle(N, n):
     announce(f"F64 bricks N={N} n={n}")
     rng = np.random.default_rng(N + n)
@@ -76,7 +76,7 @@ def test_f64_reordering_keeps_structs_and_upload_order():
     """more drifts than the container waits between two reorderings, with IDs, masses and a
     payload: everything comes back in upload order, and a captured run of steps that holds a
     reordering replays like eager steps"""
-    N, n, dt, mass = 16, 5003, 0.01, 1.0 / 5003
+    N, n, dt, mass = 16, 42001, 0.01, 1.0 / 42001
     announce(f"F64 reorder N={N} n={n}")
     rng = np.random.default_rng(3)
     part = np.dtype([("ID", "<i8"), ("pos", "<f8", 3), ("vel", "<f8", 3), ("tag", "<f8")])
