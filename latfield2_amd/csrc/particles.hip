@@ -2274,15 +2274,18 @@ __device__ __forceinline__ void kick_drift64(const Gkd64Args &A, int64_t p, cons
     if (A.drift) A.s.cell[p] = cn[0] + N * (cn[1] + N * cn[2]);
 }
 
-// largest |v|^2 of the workgroup into vmax2, one atomic (256 threads)
-__device__ __forceinline__ void vmax64(const Gkd64Args &A, double v2) {
-    __shared__ double wm[4];
+// bits of |v|^2: as unsigned integers they are ordered like the values, a NaN above all of them, so
+// that a maximum over them keeps a NaN (fmax drops it)
+__device__ __forceinline__ unsigned long long v2_bits(double v2) { return (unsigned long long)__double_as_longlong(v2); }
+
+// largest |v|^2 of the workgroup (its bits) into vmax2, one atomic (256 threads)
+__device__ __forceinline__ void vmax64(const Gkd64Args &A, unsigned long long m) {
+    __shared__ unsigned long long wm[4];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v2 = fmax(v2, __shfl_xor(v2, o));
-    if (lane_id() == 0) wm[threadIdx.x >> 6] = v2;
+    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
+    if (lane_id() == 0) wm[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0)
-        atomicMax(A.vmax2, (unsigned long long)__double_as_longlong(fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]))));
+    if (threadIdx.x == 0) atomicMax(A.vmax2, max(max(wm[0], wm[1]), max(wm[2], wm[3])));
 }
 
 // one workgroup per group of items of a brick: the brick's window of phi, then its force
@@ -2342,7 +2345,7 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
         frc[2][i] = -(phw[c + PW * PW] - phw[c - PW * PW]) * hn;
     }
     __syncthreads();
-    double vmax = 0.0;
+    unsigned long long vmax = 0ull;
     for (int j0 = r.p0; j0 < r.p1; j0 += RP) {
         if (j0 != r.p0) fetch(j0);
 #pragma unroll
@@ -2373,7 +2376,7 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
                     }
             double v2;
             kick_drift64(A, p[q], x[q], vin[q], a, v2);
-            vmax = fmax(vmax, v2);
+            vmax = max(vmax, v2_bits(v2));
         }
     }
     if (A.vmax2) vmax64(A, vmax);
@@ -2415,7 +2418,7 @@ __global__ __launch_bounds__(256) void gkd_f64_kernel(Gkd64Args A) {
         }
         kick_drift64(A, p, x, vin, a, v2);
     }
-    if (A.vmax2) vmax64(A, v2);
+    if (A.vmax2) vmax64(A, v2_bits(v2));
 }
 
 // ---------------------------------------------------------------- download / counts
