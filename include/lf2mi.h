@@ -382,8 +382,8 @@ int lf2mi_pm_step(lf2mi_parts p, lf2mi_fft_plan plan, void *rho, void *phi, int 
  *   rho = CIC deposit of q = mass N^3 per particle; phi = G rho, G = -1/K^2, G(0) = 0;
  *   F = -grad phi (central differences); v += dt * gather(F); x += dt * v (wrapped);
  *   loss = sum_cells (rho(x_final) - target)^2 over the N^3 interior.
- * The starting state of every step is checkpointed on the device; the backward pass
- * recomputes each step's fields and runs the hand-written adjoint: the gather's
+ * The starting state of every step is checkpointed on the device, its potential too where
+ * there is room; the backward pass takes or recomputes it and runs the hand-written adjoint: the gather's
  * transpose is a CIC deposit, the central difference is antisymmetric, G is symmetric
  * (the same FFT solve), and the CIC weights' position derivatives give the direct
  * terms.  dtype (F32/F64) is the precision of the whole path. */
@@ -391,6 +391,12 @@ typedef struct lf2mi_diffpm_s *lf2mi_diffpm;
 
 int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, int dtype,
                         lf2mi_diffpm *out);
+/* The same with a bound on what the handle may spend, beside the buffers that it needs, on keeping
+ * every step's potential and index for the backward pass instead of computing them again: keep_bytes,
+ * or, below 0 (lf2mi_diffpm_create), an eighth of the device memory that is free after the others.
+ * All is kept or nothing (0: nothing). */
+int lf2mi_diffpm_create_keep(int N, int64_t np, int nsteps, double mass, double dt, int dtype,
+                             int64_t keep_bytes, lf2mi_diffpm *out);
 int lf2mi_diffpm_destroy(lf2mi_diffpm m);
 /* device bytes held by the handle (checkpoints, fields, adjoints, FFT workspace) */
 int lf2mi_diffpm_bytes(lf2mi_diffpm m, int64_t *bytes);

@@ -82,6 +82,7 @@ SIGNATURES = {
     "lf2mi_parts_reduce": [_vp, _i, _i32p, _i32p, _dp, _vp],
     "lf2mi_pm_step": [_vp, _vp, _vp, _vp, _i, _d, _d, _i, _vp],
     "lf2mi_diffpm_create": [_i, _i64, _i, _d, _d, _i, ctypes.POINTER(_vp)],
+    "lf2mi_diffpm_create_keep": [_i, _i64, _i, _d, _d, _i, _i64, ctypes.POINTER(_vp)],
     "lf2mi_diffpm_destroy": [_vp],
     "lf2mi_diffpm_bytes": [_vp, _i64p],
     "lf2mi_diffpm_forward": [_vp, _vp, _vp, _vp, _i, _vp, _dp, _vp],

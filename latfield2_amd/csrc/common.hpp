@@ -59,6 +59,18 @@ __host__ __device__ inline int64_t site_index(int N, int h, int x, int y, int z)
 
 inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
+// What an object may spend on memory that it can do without (results kept for later, indexes), beside
+// the buffers it needs: an eighth of what is free once those are made, so that the caller's own tensors,
+// a second object and the staging of transfers find nearly the room they had without it.
+inline size_t spare_bytes() {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return free_b / 8;
+}
+
 inline bool is_pow2(int n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // Optional per-kernel timing with HIP events recorded on the launch stream

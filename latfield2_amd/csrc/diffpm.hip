@@ -18,10 +18,10 @@
 //                        lambda_x += q N grad_X interp(rho-bar)(X_p)   (deposit weights)
 // A particle keeps its place in all states, so gradients stay attached to it; a brick index
 // (bricks.hpp) of every state lets the deposits and gathers work brick by brick.  The starting
-// state and the potential of every step are checkpointed in HBM; where that has no room for the
-// potentials and indexes (8 bytes beside a particle's 28 or 52), they are computed again on the
-// way back.  Positions are kept as (cell, offset in cell units) and re-anchored
-// in FP64 after each drift, as in the PM step.  T = float or double selects the
+// state of every step is checkpointed in HBM, and so are its potential and its index (4 bytes
+// beside a particle's 28 or 52) where the memory left over has room for them (spare_bytes); else
+// these are computed again on the way back.  Positions are kept as (cell, offset in cell units)
+// and re-anchored in FP64 after each drift, as in the PM step.  T = float or double selects the
 // precision of the whole path (fields, FFTs, offsets, velocities, adjoints).
 #include <algorithm>
 #include <cmath>
@@ -415,13 +415,16 @@ struct lf2mi_diffpm_s {
     size_t tsize;   // sizeof(T)
     void *ck_mem;   // nsteps + 1 particle states (cell, off[3], vel[3])
     void *rho, *phi, *resid, *phib, *rhob;  // (N+2)^3 fields of T
-    void *index_mem;  // brick indexes, scratch of their builds, slots
+    void *index_mem;  // the first state's brick index, scratch of the builds, slots
     size_t index_bytes;
     lf2mi::BrickBuild bricks;  // index of the first state
-    int *index_more;           // in index_mem: an index for each further state, or null: then the
-                               // states share the first, rebuilt on the way back
     int64_t index_ints;        // size of one index
-    char *phi_kept;            // in index_mem: the potentials of the steps, or null with index_more
+    // kept for the way back where there is room, else null: the potentials of the steps after the
+    // first, then an index for each state after the first.  Without it the states share the first
+    // index and one potential, and both are made again on the way back.
+    char *phi_kept;
+    int *index_more;
+    size_t kept_bytes;
     int *slot;        // place of the caller's particles in the states
     void *lx, *lv;  // adjoints, np*3 of T
     double *loss_dev;
@@ -471,7 +474,7 @@ BrickBuild dp_index(const lf2mi_diffpm_s *m, int k) {
 
 // the potential of step k
 template <typename T> T *dp_phi(const lf2mi_diffpm_s *m, int k) {
-    return (T *)(m->phi_kept ? m->phi_kept + (size_t)k * m->G3 * m->tsize : (char *)m->phi);
+    return k > 0 && m->phi_kept ? (T *)m->phi_kept + (size_t)(k - 1) * m->G3 : (T *)m->phi;
 }
 
 unsigned dp_bricks_grid(const lf2mi_diffpm_s *m) {
@@ -574,12 +577,17 @@ int lf2mi_diffpm_bytes(lf2mi_diffpm m, int64_t *bytes) {
     if (!m || !bytes) return fail(LF2MI_EINVAL, "lf2mi_diffpm_bytes: null argument");
     int64_t fft = 0;
     if (int rc = lf2mi_fft_plan_bytes(m->plan, &fft)) return rc;
-    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + (m->phi ? 5 : 4) * (size_t)m->G3 * m->tsize + m->index_bytes +
-                       6 * (size_t)m->np * m->tsize + sizeof(double)) + fft;
+    *bytes = (int64_t)(dp_state_bytes(m->np, m->tsize) * (size_t)(m->nsteps + 1) + 5 * (size_t)m->G3 * m->tsize + m->index_bytes +
+                       m->kept_bytes + 6 * (size_t)m->np * m->tsize + sizeof(double)) + fft;
     return LF2MI_OK;
 }
 
 int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, int dtype, lf2mi_diffpm *out) {
+    return lf2mi_diffpm_create_keep(N, np, nsteps, mass, dt, dtype, -1, out);
+}
+
+int lf2mi_diffpm_create_keep(int N, int64_t np, int nsteps, double mass, double dt, int dtype, int64_t keep_bytes,
+                             lf2mi_diffpm *out) {
     if (!out) return fail(LF2MI_EINVAL, "lf2mi_diffpm_create: null output");
     *out = nullptr;
     if (N < 8 || !is_pow2(N) || np < 1 || np > INT32_MAX || nsteps < 0 || !(mass > 0) || !std::isfinite(dt))
@@ -599,27 +607,13 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     int rc = lf2mi_fft_plan_create(N, 1, 1, 0, dtype, &m->plan);
     if (!rc) rc = dp_malloc(&m->ck_mem, dp_state_bytes(np, m->tsize) * (size_t)(nsteps + 1));
     if (!rc) rc = dp_malloc(&m->rho, fb);
+    if (!rc) rc = dp_malloc(&m->phi, fb);
     if (!rc) rc = dp_malloc(&m->resid, fb);
     const int64_t nb = (N + BRK - 1) / BRK, nbk = nb * nb * nb, items = brick_items(nbk, np);
     // an index: starts, item starts, items, list; once: counts, block totals, ranks, slots
     m->index_ints = 2 * (nbk + 1) + items + np;
     m->index_bytes = sizeof(int) * (size_t)(m->index_ints + nbk + 3 * brick_blocks(nbk) + 2 * np);
-    if (!rc && nsteps > 0) {
-        // if there is room, the potentials of the steps and the indexes of the further states are
-        // kept for the way back
-        const size_t own = (m->index_bytes + 255) / 256 * 256, phis = fb * (size_t)nsteps;
-        const size_t all = own + phis + sizeof(int) * (size_t)m->index_ints * (size_t)nsteps;
-        if (hipMalloc(&m->index_mem, all) == hipSuccess) {
-            m->phi_kept = (char *)m->index_mem + own;
-            m->index_more = (int *)(m->phi_kept + phis);
-            m->index_bytes = all;
-        } else {
-            (void)hipGetLastError();
-            m->index_mem = nullptr;
-        }
-    }
-    if (!rc && !m->index_mem) rc = dp_malloc(&m->index_mem, m->index_bytes);
-    if (!rc && !m->phi_kept) rc = dp_malloc(&m->phi, fb);
+    if (!rc) rc = dp_malloc(&m->index_mem, m->index_bytes);
     if (!rc) {
         int *q = (int *)m->index_mem;
         auto take = [&q](int64_t n) {
@@ -646,11 +640,25 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
     if (!rc) {
         // the ghosts of these fields are never written by the kernels here; keep them defined
         for (void *p : {m->rho, m->phi, m->resid, m->phib, m->rhob}) {
-            if (!p) continue;
             hipError_t e = hipMemset(p, 0, fb);
             if (e != hipSuccess) {
                 rc = hip_fail(e, "hipMemset(diffpm)", __FILE__, __LINE__);
                 break;
+            }
+        }
+    }
+    if (!rc && nsteps > 0) {
+        // last, so that nothing the model needs can fail for it
+        const size_t phis = fb * (size_t)(nsteps - 1);
+        const size_t kept = phis + sizeof(int) * (size_t)m->index_ints * (size_t)nsteps;
+        void *p = nullptr;
+        if (kept <= (keep_bytes < 0 ? spare_bytes() : (size_t)keep_bytes)) {
+            if (hipMalloc(&p, kept) == hipSuccess) {
+                m->phi_kept = (char *)p;
+                m->index_more = (int *)((char *)p + phis);
+                m->kept_bytes = kept;
+            } else {
+                (void)hipGetLastError();
             }
         }
     }
@@ -665,7 +673,7 @@ int lf2mi_diffpm_create(int N, int64_t np, int nsteps, double mass, double dt, i
 int lf2mi_diffpm_destroy(lf2mi_diffpm m) {
     if (!m) return LF2MI_OK;
     if (m->plan) lf2mi_fft_plan_destroy(m->plan);
-    for (void *p : {m->ck_mem, m->index_mem, m->rho, m->phi, m->resid, m->phib, m->rhob, m->lx, m->lv, (void *)m->loss_dev})
+    for (void *p : {m->ck_mem, m->index_mem, (void *)m->phi_kept, m->rho, m->phi, m->resid, m->phib, m->rhob, m->lx, m->lv, (void *)m->loss_dev})
         if (p) (void)hipFree(p);
     delete m;
     return LF2MI_OK;
