@@ -18,6 +18,7 @@
 // divide N.
 #pragma once
 
+#include "brick_run.hpp"
 #include "common.hpp"
 
 namespace lf2mi {
@@ -357,7 +358,7 @@ inline int64_t brick_items(int64_t nbk, int64_t np) { return nbk + np / BRK_ITEM
 // a group of MERGE consecutive items of one brick: the workgroup of the first takes them all.
 // Uniform over the workgroup; false when there is nothing to do.
 struct BrickRange {
-    int b, p0, p1, ox, oy, oz;
+    int b, p0, n, ox, oy, oz;  // list entries p0 + [0, n)
 };
 template <int MERGE>
 __device__ __forceinline__ bool brick_range(const BrickIndex &V, int it, BrickRange &r) {
@@ -365,8 +366,9 @@ __device__ __forceinline__ bool brick_range(const BrickIndex &V, int it, BrickRa
     r.b = V.item[it];
     const int k = it - V.istart[r.b];
     if (k % MERGE != 0) return false;
-    r.p0 = V.start[r.b] + k * BRK_ITEM;
-    r.p1 = min(r.p0 + MERGE * BRK_ITEM, V.start[r.b + 1]);
+    const BrickRun e = brick_run(V.start[r.b], V.start[r.b + 1], k * BRK_ITEM, MERGE * BRK_ITEM);
+    r.p0 = e.p0;
+    r.n = e.n;
     r.ox = (r.b % V.NB) * BRK;
     r.oy = ((r.b / V.NB) % V.NB) * BRK;
     r.oz = (r.b / (V.NB * V.NB)) * BRK;

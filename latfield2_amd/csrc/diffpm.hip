@@ -166,8 +166,8 @@ __global__ __launch_bounds__(DP_WG) void dp_density_kernel(DpState<T> s, BrickIn
     const int N = s.N;
     for (int i = threadIdx.x; i < DP_F3; i += DP_WG) win[i] = 0.0;
     __syncthreads();
-    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
-        const int p = V.list[j];
+    for (int j = threadIdx.x; j < r.n; j += DP_WG) {
+        const int p = V.list[r.p0 + j];
         int c[3];
         brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};
@@ -230,8 +230,8 @@ __global__ __launch_bounds__(DP_WG) void dp_step_kernel(DpState<T> s, DpState<T>
     if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
     const int N = s.N;
     brick_forces(phi, N, r, phw, frc);
-    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
-        const int p = V.list[j];
+    for (int j = threadIdx.x; j < r.n; j += DP_WG) {
+        const int p = V.list[r.p0 + j];
         int c[3];
         brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};
@@ -342,8 +342,8 @@ __global__ __launch_bounds__(DP_WG) void dp_adj_kernel(DpState<T> s, BrickIndex 
     brick_forces(phi, N, r, reinterpret_cast<T *>(&fb[0][0]), frc);
     for (int i = threadIdx.x; i < 3 * DP_F3; i += DP_WG) (&fb[0][0])[i] = 0.0;
     __syncthreads();
-    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += DP_WG) {
-        const int p = V.list[j];
+    for (int j = threadIdx.x; j < r.n; j += DP_WG) {
+        const int p = V.list[r.p0 + j];
         int c[3];
         brick_decode(s.cell[p], N, V.lgN, c[0], c[1], c[2]);
         const T u[3] = {s.off[0][p], s.off[1][p], s.off[2][p]};

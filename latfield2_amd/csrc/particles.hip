@@ -2166,8 +2166,8 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Arg
     __syncthreads();
     const int N = A.N;
     const double none[6] = {};
-    for (int j = r.p0 + (int)threadIdx.x; j < r.p1; j += WG) {
-        const int p = V.list[j];
+    for (int j = threadIdx.x; j < r.n; j += WG) {
+        const int p = V.list[r.p0 + j];
         const int o[3] = {r.ox, r.oy, r.oz};
         BwParticle<double> P;
 #pragma unroll
@@ -2306,7 +2306,7 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
 #pragma unroll
         for (int k = 0; k < G64_PER; ++k) {
             const int j = j0 + (int)threadIdx.x + 256 * k;
-            p[k] = j < r.p1 ? V.list[j] : -1;
+            p[k] = j < r.n ? V.list[r.p0 + j] : -1;
         }
 #pragma unroll
         for (int k = 0; k < G64_PER; ++k)
@@ -2319,7 +2319,7 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
             }
     };
     // the first round's particles in flight while the window loads
-    fetch(r.p0);
+    fetch(0);
     {
         constexpr int WK = (PW * PW * PW + 255) / 256;
         double w[WK];
@@ -2346,8 +2346,8 @@ __global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickInde
     }
     __syncthreads();
     unsigned long long vmax = 0ull;
-    for (int j0 = r.p0; j0 < r.p1; j0 += RP) {
-        if (j0 != r.p0) fetch(j0);
+    for (int j0 = 0; j0 < r.n; j0 += RP) {
+        if (j0 != 0) fetch(j0);
 #pragma unroll
         for (int q = 0; q < G64_PER; ++q) {
             if (p[q] < 0) continue;
