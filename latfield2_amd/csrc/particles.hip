@@ -186,7 +186,7 @@ struct IcArgs {
     const int64_t *bstart;   // nblobs + 1 prefix of blob occupancies
 };
 
-__device__ __forceinline__ void ic_particle(const IcArgs &A, int64_t i, double p[3], double v[3]) {
+__device__ __forceinline__ void ic_pos(const IcArgs &A, int64_t i, double p[3]) {
     if (A.kind == 0) {
         const int64_t ng = A.ng;
         const int64_t ix = i % ng, iy = (i / ng) % ng, iz = i / (ng * ng);
@@ -207,8 +207,10 @@ __device__ __forceinline__ void ic_particle(const IcArgs &A, int64_t i, double p
     for (int d = 0; d < 3; ++d) {
         p[d] -= floor(p[d]);  // periodic wrap into [0, 1)
         if (p[d] >= 1.0) p[d] = 0.0;
-        v[d] = A.sigma_v * grand(A.seed, i, 12 + d);
     }
+}
+__device__ __forceinline__ void ic_vel(const IcArgs &A, int64_t i, double v[3]) {
+    for (int d = 0; d < 3; ++d) v[d] = A.sigma_v * grand(A.seed, i, 12 + d);
 }
 
 __global__ void ic_f32_kernel(IcArgs A, Soa32 dst, Geo g, int *__restrict__ counts) {
@@ -217,7 +219,8 @@ __global__ void ic_f32_kernel(IcArgs A, Soa32 dst, Geo g, int *__restrict__ coun
     int cell = -1;
     if (in) {
         double p[3], v[3];
-        ic_particle(A, i, p, v);
+        ic_pos(A, i, p);
+        ic_vel(A, i, v);
         float off[3];
         bin_one(p, g.N, cell, off);
         dst.cell[i] = cell;
@@ -255,15 +258,17 @@ __device__ __forceinline__ int cell64(const double p[3], int N) {
 // hundred steps single particles of them (256^3 step: gather 1.1 -> 1.8 ms).  `slot` maps the
 // upload order to the place.  (256^3 step in brick order, lists in particle order: gather
 // 0.44 ms, 2.0 GB moved at 4.5 TB/s.)
+// The place comes from the cell that was counted (`cell`, in upload order), never from a second
+// evaluation of the position: one that differed in a bit would put a particle on another's place.
 struct Order64 {
-    const int *start, *rank;  // null: upload order
+    const int *start, *rank, *cell;  // null: upload order
     int *slot;
     int N, NB, lgN;
 };
-__device__ __forceinline__ int64_t order64(const Order64 &O, int64_t i, int cell) {
+__device__ __forceinline__ int64_t order64(const Order64 &O, int64_t i) {
     if (!O.start) return i;
     int x, y, z;
-    brick_decode(cell, O.N, O.lgN, x, y, z);
+    brick_decode(O.cell[i], O.N, O.lgN, x, y, z);
     const int j = O.start[brick_of(x, y, z, O.NB)] + O.rank[i];
     O.slot[i] = j;
     return j;
@@ -297,16 +302,11 @@ __global__ void reorder_slot_kernel(int64_t np, const int *__restrict__ place, i
     list[i] = (int)i;
 }
 
-// the cells of staged positions (pos: AoS) or, without them, of the synthetic particles
-__global__ void cells64_kernel(int64_t np, const double *__restrict__ pos, IcArgs A, int N, int *__restrict__ cell) {
+// the cells of staged positions (pos: AoS)
+__global__ void cells64_kernel(int64_t np, const double *__restrict__ pos, int N, int *__restrict__ cell) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
-    double p[3], v[3];
-    if (pos) {
-        for (int d = 0; d < 3; ++d) p[d] = pos[3 * i + d];
-    } else {
-        ic_particle(A, i, p, v);
-    }
+    const double p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
     cell[i] = cell64(p, N);
 }
 
@@ -315,20 +315,48 @@ __global__ void iota_kernel(int *__restrict__ p, int64_t n) {
     if (i < n) p[i] = (int)i;
 }
 
-__global__ void ic_f64_kernel(IcArgs A, Soa64 dst, int N, Order64 O) {
+// synthetic particles in their own order
+__global__ void ic_f64_kernel(IcArgs A, Soa64 dst, int N) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= A.np) return;
     double p[3], v[3];
-    ic_particle(A, i, p, v);
-    const int cell = cell64(p, N);
-    const int64_t j = order64(O, i, cell);
+    ic_pos(A, i, p);
+    ic_vel(A, i, v);
     for (int d = 0; d < 3; ++d) {
-        dst.pos[d][j] = p[d];
-        dst.vel[d][j] = v[d];
+        dst.pos[d][i] = p[d];
+        dst.vel[d][i] = v[d];
     }
-    dst.cell[j] = cell;
+    dst.cell[i] = cell64(p, N);
+    if (dst.mass) dst.mass[i] = 1.0;
+    if (dst.id) dst.id[i] = i;
+}
+
+// In brick order: the positions are evaluated once, into the velocities' arrays, with their cells;
+// counted and scanned, they go to their places, and then the velocities to theirs.
+__global__ void ic_stage64_kernel(IcArgs A, Soa64 dst, int N, int *__restrict__ cell) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= A.np) return;
+    double p[3];
+    ic_pos(A, i, p);
+    for (int d = 0; d < 3; ++d) dst.vel[d][i] = p[d];
+    cell[i] = cell64(p, N);
+}
+__global__ void ic_place64_kernel(int64_t np, Soa64 dst, Order64 O) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= np) return;
+    const int64_t j = order64(O, i);
+    for (int d = 0; d < 3; ++d) dst.pos[d][j] = dst.vel[d][i];
+    dst.cell[j] = O.cell[i];
     if (dst.mass) dst.mass[j] = 1.0;
     if (dst.id) dst.id[j] = i;
+}
+__global__ void ic_vel64_kernel(IcArgs A, Soa64 dst, const int *__restrict__ slot) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= A.np) return;
+    double v[3];
+    ic_vel(A, i, v);
+    const int64_t j = slot[i];
+    for (int d = 0; d < 3; ++d) dst.vel[d][j] = v[d];
 }
 
 __global__ void upload_f64_kernel(int64_t np, const double *__restrict__ pos, const double *__restrict__ vel,
@@ -337,8 +365,8 @@ __global__ void upload_f64_kernel(int64_t np, const double *__restrict__ pos, co
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= np) return;
     const double p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
-    const int cell = cell64(p, N);
-    const int64_t j = order64(O, i, cell);
+    const int cell = O.cell ? O.cell[i] : cell64(p, N);
+    const int64_t j = order64(O, i);
     for (int d = 0; d < 3; ++d) {
         dst.pos[d][j] = p[d];
         dst.vel[d][j] = vel[3 * i + d];
@@ -2762,22 +2790,30 @@ static int b64_fill(lf2mi_parts_s *p, const double *pos, const double *vel, cons
     p->moves = 0;
     if (p->sorted) {
         const BrickIndex V = brick_view(p->bb, N);
-        cells64_kernel<<<g, 256, 0, st>>>(p->np, pos, A, N, p->bb.list);  // the list is written last
+        // the cells are kept in the list, which is written last
+        if (pos) cells64_kernel<<<g, 256, 0, st>>>(p->np, pos, N, p->bb.list);
+        else ic_stage64_kernel<<<g, 256, 0, st>>>(A, p->b64, N, p->bb.list);
         LF2MI_LAUNCHED();
         brick_count_kernel<<<g, 256, 0, st>>>(p->np, p->bb.list, N, V.NB, V.lgN, p->bb.count, p->bb.rank);
         LF2MI_LAUNCHED();
         if (int rc = brick_scan(p->bb.scan(), V.nbk, st)) return rc;
         O.start = p->bb.start;
         O.rank = p->bb.rank;
+        O.cell = p->bb.list;
         O.slot = p->slot;
         O.N = N;
         O.NB = V.NB;
         O.lgN = V.lgN;
     }
     if (pos) upload_f64_kernel<<<g, 256, 0, st>>>(p->np, pos, vel, mass, id, pl, p->plw, p->b64, N, O);
-    else ic_f64_kernel<<<g, 256, 0, st>>>(A, p->b64, N, O);
+    else if (p->sorted) ic_place64_kernel<<<g, 256, 0, st>>>(p->np, p->b64, O);
+    else ic_f64_kernel<<<g, 256, 0, st>>>(A, p->b64, N);
     LF2MI_LAUNCHED();
     if (p->sorted) {
+        if (!pos) {
+            ic_vel64_kernel<<<g, 256, 0, st>>>(A, p->b64, p->slot);
+            LF2MI_LAUNCHED();
+        }
         iota_kernel<<<g, 256, 0, st>>>(p->bb.list, p->np);
         LF2MI_LAUNCHED();
     }
