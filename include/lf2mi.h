@@ -187,7 +187,10 @@ int lf2mi_poisson_solve(lf2mi_fft_plan plan, const void *rho, void *phi, double 
  * on one device.  LF2MI_F32: each particle is kept as an int32 cell index
  * x + N(y + N z) plus an FP32 offset in cell units in [0,1) per axis and FP32
  * velocities, bucketed by 8^3-cell bricks (the analogue of the per-cell lists).
- * LF2MI_F64: absolute FP64 positions and velocities, downloaded in upload order (plain path). */
+ * LF2MI_F64: absolute FP64 positions and velocities (52 bytes a particle), downloaded in
+ * upload order.  A capacity of 40 000 particles and of 24 per 8^3-cell brick also gets a brick
+ * index (20 bytes a particle) if that takes no more than an eighth of the device memory left:
+ * its particles then lie, and are deposited and gathered, brick by brick. */
 typedef struct lf2mi_parts_s *lf2mi_parts;
 
 int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_parts *out);

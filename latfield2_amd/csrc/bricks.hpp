@@ -5,7 +5,8 @@
 // A particle's atomics into the field cost 8 to 48 global transactions (FP64: 40 G atomics/s
 // on particles in lattice order, 23 on random ones); summed in an LDS window per brick first
 // (1500 G FP64 LDS atomics/s on random nodes, against 200 for FP32 ones), only the window's
-// nodes go to the field, in rows (100 G atomics/s).  The index costs 12 bytes per particle.
+// nodes go to the field, in rows (100 G atomics/s).  The index costs 8 bytes per particle (list and
+// rank) and about 16 per brick, an order of the particles beside it 4 (their places) to 12.
 //
 // Building it: brick_count_kernel counts the cells in particle order (brick_rank: the
 // particle's place among its brick's, one global atomic per brick and wave), one or two scan
