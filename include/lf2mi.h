@@ -334,7 +334,10 @@ int lf2mi_deposit(lf2mi_parts p, int kind, void *field, int halo, int target, in
  *   (reads the interior of phi only); vel += dt_kick * sum_corners w F(corner) with the
  *   scalar-deposit weights; pos += dt_drift * vel, wrapped (:2028-2032) and re-keyed.
  * In F32 the new position is formed in FP64 from (cell, offset, vel) and re-anchored to
- * (cell, FP32 offset).  The container is re-bucketed afterwards.  vmax2 (host, may be
+ * (cell, FP32 offset).  The container is re-bucketed afterwards; a F64 one with a brick index
+ * brings that up to date and puts its particles into brick order with every 32nd drift, of
+ * eager ones and of those in one capture apart: a graph of fewer drifts that is replayed
+ * hundreds of times gathers at up to half the speed until eager drifts follow.  vmax2 (host, may be
  * NULL) receives max |v|^2 after the kick (synchronises when non-NULL).  phi may be
  * NULL when dt_kick == 0: a drift only (move_particles_simple, move_function.hpp:30). */
 int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_kick,

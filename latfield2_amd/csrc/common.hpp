@@ -59,6 +59,17 @@ __host__ __device__ inline int64_t site_index(int N, int h, int x, int y, int z)
 
 inline unsigned blocks_for(int64_t n, int threads) { return (unsigned)((n + threads - 1) / threads); }
 
+// whether launches on `st` are recorded into a graph, and the capture's id
+inline bool capturing(hipStream_t st, unsigned long long *id) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    *id = 0;
+    if (hipStreamGetCaptureInfo(st, &s, id) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return s != hipStreamCaptureStatusNone;
+}
+
 // What an object may spend on memory that it can do without (results kept for later, indexes), beside
 // the buffers it needs: an eighth of what is free once those are made, so that the caller's own tensors,
 // a second object and the staging of transfers find nearly the room they had without it.

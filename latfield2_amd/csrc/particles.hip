@@ -2678,6 +2678,8 @@ struct lf2mi_parts_s {
     int sorted;            // 1: the places are in brick order (else upload order, slot unused)
     void *tmp;             // F64: one 8-byte value per particle (reordering), with the index
     int moves;             // F64: drifts since the particles were last put into brick order
+    int cap_moves;         // the same of the drifts recorded by the capture cap_id
+    unsigned long long cap_id;
     int in_box;            // 1: every F64 position is in [0, 1) (a kick then leaves them alone)
     unsigned long long *fx;
     int64_t fx_n;
@@ -2790,13 +2792,19 @@ template <typename T> static int reorder_one(lf2mi_parts_s *p, T *a, int stride,
 // The index after a drift; every B64_REORDER drifts the particles are put into its order as
 // well.  A particle that has left the brick whose place it lies in costs whole lines for
 // single values: at 256^3 the gather slows from 0.45 to 0.9 ms over 400 steps without this;
-// a reorder takes 0.9 ms.
+// a reorder takes 0.9 ms.  A drift that is recorded runs with each replay and not now, so a
+// capture counts its own drifts from 0: what a graph holds depends on the graph alone.
 static constexpr int B64_REORDER = 32;
-static int b64_moved(lf2mi_parts_s *p, hipStream_t st) {
+static int b64_moved(lf2mi_parts_s *p, bool captured, unsigned long long cap_id, hipStream_t st) {
     Soa64 &s = p->b64;
     if (int rc = brick_build(s.cell, p->np, p->N, p->bb, st)) return rc;
-    if (++p->moves < B64_REORDER) return LF2MI_OK;
-    p->moves = 0;
+    if (captured && cap_id != p->cap_id) {
+        p->cap_id = cap_id;
+        p->cap_moves = 0;
+    }
+    int &moves = captured ? p->cap_moves : p->moves;
+    if (++moves < B64_REORDER) return LF2MI_OK;
+    moves = 0;
     int rc = reorder_one(p, s.cell, 1, st);
     for (int d = 0; d < 3 && !rc; ++d) {
         rc = reorder_one(p, s.pos[d], 1, st);
@@ -4047,10 +4055,12 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
             LF2MI_LAUNCHED();
         }
         if (A.drift) {
-            p->in_box = 1;
+            unsigned long long cap_id;
+            const bool captured = capturing(st, &cap_id);
+            if (!captured) p->in_box = 1;  // a recorded drift has moved nothing yet
             if (bricks) {
                 LF2MI_PROF("brick_index", st);
-                if (int rc = b64_moved(p, st)) return rc;
+                if (int rc = b64_moved(p, captured, cap_id, st)) return rc;
             }
         }
         if (vmax2) {
