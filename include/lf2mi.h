@@ -159,7 +159,8 @@ int lf2mi_fft_execute(lf2mi_fft_plan plan, int direction, void *rfield, void *kf
 
 /* Green's-function multiply of examples/poissonSolver.cpp:99-111 on a k-field:
  * k *= scale / lambda, lambda = 2 (cos 2pi kx/N + cos 2pi ky/N + cos 2pi kz/N - 3) / res^2,
- * zero mode set to 0; lambda and scale/lambda evaluated in FP64. */
+ * zero mode set to 0; lambda and scale/lambda evaluated in FP64.  Allocates its eigenvalue
+ * table from the stream's pool, and is refused (LF2MI_EHIP) while the stream is captured. */
 int lf2mi_poisson_green(void *kfield, int N, int C, int khalo, double res, double scale,
                         int dtype, void *stream);
 
@@ -169,7 +170,7 @@ int lf2mi_poisson_green(void *kfield, int N, int C, int khalo, double res, doubl
  * 1024 doubles (8 KiB per GPU, held until the process ends), so N <= 1024 (LF2MI_ERANGE
  * otherwise); no hipMalloc/hipFree, no host synchronisation.  Calls on one GPU share that
  * array: calls that overlap on one GPU (different streams) race.  Results equal
- * lf2mi_poisson_green's to FP64 rounding (the table is computed on the device). */
+ * lf2mi_poisson_green's. */
 int lf2mi_poisson_green_noalloc(void *kfield, int N, int C, int khalo, double res, double scale,
                                 int dtype, void *stream);
 

@@ -1407,6 +1407,9 @@ int lf2mi_poisson_green(void *kfield, int N, int C, int khalo, double res, doubl
     // (a 128^3 driver loop: 266 -> 237 us a step)
     double *s4v = nullptr;
     hipStream_t st = as_stream(stream);
+    // it allocates, which a graph is not to hold: refused, as when it waited
+    unsigned long long cap_id;
+    if (capturing(st, &cap_id)) return hip_fail(hipErrorStreamCaptureUnsupported, "lf2mi_poisson_green", __FILE__, __LINE__);
     LF2MI_HIP(hipMallocAsync((void **)&s4v, sizeof(double) * N, st));
     green_table_kernel<<<(N + 255) / 256, 256, 0, st>>>(s4v, N);
     LF2MI_LAUNCHED();
