@@ -152,7 +152,7 @@ __global__ void ghost_fill_kernel(T *__restrict__ f, int nx, int ny, int nz, int
 // other, so one thread takes a node of the interior's outer layers with all its images, reads
 // them, runs the three stages on them in order and writes back what they change, ghosts
 // included: the stages' values bit for bit, in one launch instead of three (15 -> 5 us for
-// three components at 120^3).
+// three components at 120^3).  Large lattices keep the stages (fold_one).
 // The outer layers' nodes: two z layers (all x, y), then two y layers (z inside), then two x
 // layers (y, z inside).
 template <typename T>
@@ -213,7 +213,8 @@ __global__ __launch_bounds__(256) void fold_kernel(T *__restrict__ f, int N, int
     }
 }
 
-// the same for N = 1, where 0 is also N - 1 and both images fold into it
+// The stages one by one, for large lattices and for N = 1, where 0 is also N - 1 and both images fold
+// into it.
 template <typename T>
 __global__ void fold_stage_kernel(T *__restrict__ f, int N, int h, int C, int stage, unsigned down, int klo) {
     int na, nb, a0, b0;
@@ -252,6 +253,13 @@ __global__ void fold_stage_kernel(T *__restrict__ f, int N, int h, int C, int st
         if ((down >> c) & 1u) f[dst_dn * C + c] += dn;
     }
 }
+
+// Whether a fold takes the one launch: below 256^3 two launches' latency is more than the longer
+// chain of loads of a thread with all its images, which a stage's simple rows do without (one launch
+// against three, microseconds, scalar / vector / six components without lower folds: 208^3 6.0
+// against 9.0, 8.4 / 10.6, 10.2 / 10.4; 240^3 7.5 / 8.9, 10.1 / 11.5, 12.6 / 11.4; 256^3 10.3 / 9.3, 12.7 / 12.5,
+// 15.4 / 11.8; 512^3 23.2 / 16.1, 35.6 / 27.3, 46.7 / 28.1).
+static bool fold_one(int N, int C, unsigned down) { return N >= 2 && N < (C == 6 && down == 0u ? 216 : 256); }
 
 // ---------------------------------------------------------------- reductions
 template <typename T>
@@ -442,7 +450,7 @@ int lf2mi_projection_comm(void *field, int N, int halo, int kind, int dtype, voi
     if (halo < 1) return fail(LF2MI_EINVAL, "the field has to have at least a halo of 1");
     if (!field) return fail(LF2MI_EINVAL, "lf2mi_projection_comm: null field");
     LF2MI_PROF("projection_comm", as_stream(stream));
-    if (N >= 2) {
+    if (fold_one(N, C, down)) {
         const unsigned g = grid_cap((2LL * N * N + 2LL * N * (N - 2) + 2LL * (N - 2) * (N - 2)) * C, 256);
         if (dtype == LF2MI_F32)
             fold_kernel<float><<<g, 256, 0, as_stream(stream)>>>((float *)field, N, halo, C, down, klo);
@@ -451,11 +459,12 @@ int lf2mi_projection_comm(void *field, int N, int halo, int kind, int dtype, voi
         LF2MI_LAUNCHED();
         return LF2MI_OK;
     }
+    const unsigned g = grid_cap((int64_t)(N + 2) * (N + 2) * C, 256);
     for (int stage = 0; stage < 3; ++stage) {
         if (dtype == LF2MI_F32)
-            fold_stage_kernel<float><<<1, 64, 0, as_stream(stream)>>>((float *)field, N, halo, C, stage, down, klo);
+            fold_stage_kernel<float><<<g, 256, 0, as_stream(stream)>>>((float *)field, N, halo, C, stage, down, klo);
         else
-            fold_stage_kernel<double><<<1, 64, 0, as_stream(stream)>>>((double *)field, N, halo, C, stage, down, klo);
+            fold_stage_kernel<double><<<g, 256, 0, as_stream(stream)>>>((double *)field, N, halo, C, stage, down, klo);
         LF2MI_LAUNCHED();
     }
     return LF2MI_OK;
