@@ -162,7 +162,7 @@ template <typename T>
 __global__ __launch_bounds__(DP_WG) void dp_density_kernel(DpState<T> s, BrickIndex V, T *__restrict__ rho, T q) {
     __shared__ double win[DP_F3];
     BrickRange r;
-    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
+    if (!brick_range(V, blockIdx.x, DP_MERGE, r)) return;
     const int N = s.N;
     for (int i = threadIdx.x; i < DP_F3; i += DP_WG) win[i] = 0.0;
     __syncthreads();
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(DP_WG) void dp_step_kernel(DpState<T> s, DpState<T>
     __shared__ T frc[3][DP_F3];
     dp_clear(clear);
     BrickRange r;
-    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
+    if (!brick_range(V, blockIdx.x, DP_MERGE, r)) return;
     const int N = s.N;
     brick_forces(phi, N, r, phw, frc);
     for (int j = threadIdx.x; j < r.n; j += DP_WG) {
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(DP_WG) void dp_adj_kernel(DpState<T> s, BrickIndex 
     __shared__ double fb[3][DP_F3];  // the window of phi before
     static_assert(sizeof(double) * 3 * DP_F3 >= sizeof(T) * DP_P3, "the window of phi fits");
     BrickRange r;
-    if (!brick_range<DP_MERGE>(V, blockIdx.x, r)) return;
+    if (!brick_range(V, blockIdx.x, DP_MERGE, r)) return;
     const int N = s.N;
     brick_forces(phi, N, r, reinterpret_cast<T *>(&fb[0][0]), frc);
     for (int i = threadIdx.x; i < 3 * DP_F3; i += DP_WG) (&fb[0][0])[i] = 0.0;

@@ -606,7 +606,18 @@ __device__ __forceinline__ unsigned long long fx_term(float q, float w, double f
     return (unsigned long long)llrint((double)(q * w) * fxscale);
 }
 
-static constexpr int DEP_MERGE = 8;  // items one deposit workgroup takes
+static constexpr int DEP_MERGE = 8;  // items one deposit workgroup takes, at most
+
+// The items a workgroup of a window kernel takes, `most` or fewer: a window is zeroed, filled and
+// flushed once for all of them, but the crowded bricks of few particles have to be shared out, or a few
+// workgroups work on while the chip waits (clustered particles, 8 items each against this: FP32 vector
+// unfolded, 1 M on 64^3 74 -> 29 us, VecVec 2 M on 128^3 176 -> 126; FP64 vector 0.5 M on 128^3 70 -> 50).
+static constexpr int64_t MERGE_GROUPS = 2048;
+static int merge_items(int64_t np, int most) {
+    int m = most;
+    while (m > 1 && np < MERGE_GROUPS * m * ITEM_P) m /= 2;
+    return m;
+}
 
 // ---------------------------------------------------------------- scalar deposit, periodic target
 // Three kernels, when the target is periodic, the brick edge 8, the number of bricks per row a
@@ -2182,14 +2193,12 @@ static constexpr int64_t B64_OCC = 24;
 // steps, by bricks and particle by particle, 20 000 particles on 32^3 129 and 105 us, on 40^3 126
 // and 100; 40 000 on 32^3 139 / 144, on 64^3 127 / 122; 80 000 on 64^3 138 / 172, on 96^3 163 / 200
 static constexpr int64_t B64_NP = 40000;
-static constexpr int B64_MERGE = 8;  // items per workgroup
-
 template <int KIND>
-__global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Args A, BrickIndex V) {
+__global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Args A, BrickIndex V, int merge) {
     constexpr int WG = bw_wg<KIND>();
     __shared__ double win[bw_size<KIND>()];
     BrickRange r;
-    if (!brick_range<B64_MERGE>(V, blockIdx.x, r)) return;
+    if (!brick_range(V, blockIdx.x, merge, r)) return;
     for (int i = threadIdx.x; i < bw_size<KIND>(); i += WG) win[i] = 0.0;
     __syncthreads();
     const int N = A.N;
@@ -2217,45 +2226,67 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick64_kernel(Dep64Arg
 }
 
 // The same windows for the FP32 container, whose buckets are its bricks (any edge up to 8):
-// one workgroup per group of up to DEP_MERGE items of a brick, or a share of the groups of a
-// work list (brick_starts_kernel).  The terms' products are FP32.
+// one workgroup per `merge` items of a brick, or a share of the groups of a work list
+// (brick_starts_kernel), each in parts of `merge` items.  The terms' products are FP32.
 template <int KIND, typename ACC>
 __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs A, const int2 *__restrict__ groups,
-                                                                        const int *__restrict__ ngroups) {
+                                                                        const int *__restrict__ ngroups,
+                                                                        int merge) {
     constexpr int WG = bw_wg<KIND>(), GP = DEP_MERGE * ITEM_P;
     constexpr bool FX = sizeof(ACC) == 8;
     using W = std::conditional_t<FX, unsigned long long, double>;
     __shared__ W win[bw_size<KIND>()];
     const int N = A.g.N, NB = A.g.NB, B = A.g.B;
-    auto group = [&](int b, int p0) {
-        const int p1 = min(A.start[b + 1], p0 + GP);
+    auto group = [&](int b, int p0, int len) {
+        const int p1 = min(A.start[b + 1], p0 + len);
         const int o[3] = {(b % NB) * B, ((b / NB) % NB) * B, (b / (NB * NB)) * B};
+        // A round's particles are requested before the last one's terms are added; not for six
+        // components, whose three workgroups per CU that costs registers (256^3, one round per brick:
+        // 751 -> 826 us).
+        constexpr bool AHEAD = KindC<KIND>::C < 6;
+        int cell = -1;
+        float u[3], v[3] = {0.f, 0.f, 0.f}, m = A.mass_nv;
+        auto fetch = [&](int p) {
+            cell = -1;
+            if (p >= p1) return;
+            cell = A.s.cell[p];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                u[d] = A.s.off[d][p];
+                if constexpr (KIND > 0) v[d] = A.s.vel[d][p];
+            }
+            if (A.s.mass) m = A.s.mass[p] * A.mass_nv;
+        };
+        if (AHEAD) fetch(p0 + (int)threadIdx.x);
         for (int i = threadIdx.x; i < bw_size<KIND>(); i += WG) win[i] = W(0);
         __syncthreads();
         for (int p = p0 + (int)threadIdx.x; p < p1; p += WG) {
+            if (!AHEAD) fetch(p);
             int c[3];
-            decode_cell(A.s.cell[p], A.g, c[0], c[1], c[2]);
+            decode_cell(cell, A.g, c[0], c[1], c[2]);
             BwParticle<float> P;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 P.l[d] = c[d] - o[d];
-                bw_weights(P, d, A.s.off[d][p]);
+                bw_weights(P, d, u[d]);
             }
-            const float m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
-            float v[3] = {0.f, 0.f, 0.f};
-            if constexpr (KIND > 0)
-                for (int d = 0; d < 3; ++d) v[d] = A.s.vel[d][p];
-            bw_particle<KIND>(win, P, m, v, A.fxs);
+            const float vp[3] = {v[0], v[1], v[2]}, mp = m;
+            if (AHEAD) fetch(p + WG);
+            bw_particle<KIND>(win, P, mp, vp, A.fxs);
         }
         __syncthreads();
         if constexpr (FX) bw_flush<KIND>(win, A.fx, N, A.h, A.tgt, o[0], o[1], o[2]);
         else bw_flush<KIND>(win, A.field, N, A.h, A.tgt, o[0], o[1], o[2]);
     };
     if (groups) {
-        const int total = ngroups[0];
+        // the groups' first parts, then their second ones, ...: a brick's last group need not fill
+        // all of them, and the empty ones come last
+        const int n = ngroups[0], total = n * (DEP_MERGE / merge);
         for (int gi = blockIdx.x; gi < total; gi += gridDim.x) {
-            const int2 gr = groups[gi];
-            group(gr.x, A.start[gr.x] + gr.y * GP);
+            const int2 gr = groups[gi % n];
+            const int p0 = A.start[gr.x] + gr.y * GP + gi / n * merge * ITEM_P;
+            if (p0 >= A.start[gr.x + 1]) continue;
+            group(gr.x, p0, merge * ITEM_P);
             __syncthreads();  // the window is reused
         }
         return;
@@ -2263,7 +2294,7 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs 
     const int it = blockIdx.x;
     if (it >= A.istart[A.g.nbk]) return;
     const int b = A.item_bucket[it], k = it - A.istart[b];
-    if (k % DEP_MERGE == 0) group(b, A.start[b] + k * ITEM_P);
+    if (k % merge == 0) group(b, A.start[b] + k * ITEM_P, merge * ITEM_P);
 }
 
 struct Gkd64Args {
@@ -2319,14 +2350,14 @@ __device__ __forceinline__ void vmax64(const Gkd64Args &A, unsigned long long m)
 // one workgroup per group of items of a brick: the brick's window of phi, then its force
 // nodes (the differences of gkd_f64_kernel, each formed once per node instead of once per
 // particle and corner), both in LDS
-static constexpr int G64_MERGE = 4;
+static constexpr int G64_MERGE = 4;  // items per workgroup, at most
 static constexpr int G64_PER = 2;  // particles per thread and round, their loads issued together
-__global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickIndex V) {
+__global__ __launch_bounds__(256) void gkd_brick64_kernel(Gkd64Args A, BrickIndex V, int merge) {
     constexpr int PW = BRK + 3, FW = BRK + 1, RP = 256 * G64_PER;
     __shared__ double phw[PW * PW * PW];
     __shared__ double frc[3][FW * FW * FW];
     BrickRange r;
-    if (!brick_range<G64_MERGE>(V, blockIdx.x, r)) return;
+    if (!brick_range(V, blockIdx.x, merge, r)) return;
     const int N = A.N;
     int p[G64_PER];
     double x[G64_PER][3], vin[G64_PER][3];
@@ -2930,8 +2961,9 @@ static int64_t item_grid(const lf2mi_parts_s *p) { return p->g.nbk + p->np / ITE
 
 // the brick window deposit: every brick, or (groups) those of a work list of dense ones
 template <int KIND, typename ACC>
-static void launch_bricks(const DepArgs &A, unsigned grid, const int2 *groups, const int *ngroups, hipStream_t st) {
-    deposit_brick32_kernel<KIND, ACC><<<grid, bw_wg<KIND>(), 0, st>>>(A, groups, ngroups);
+static void launch_bricks(const lf2mi_parts_s *p, const DepArgs &A, unsigned grid, const int2 *groups, const int *ngroups,
+                          hipStream_t st) {
+    deposit_brick32_kernel<KIND, ACC><<<grid, bw_wg<KIND>(), 0, st>>>(A, groups, ngroups, merge_items(p->np, DEP_MERGE));
 }
 
 // the scalar deposit of a global mass into a periodic target with 8^3 bricks
@@ -3055,7 +3087,7 @@ static int launch_tiles_c(lf2mi_parts_s *p, DepArgs A, bool pm, bool overwrite, 
         fold_edges_kernel<C><<<grid1(edges), 256, 0, st>>>(A.field, (int)N, A.h, (int)NB, F, shell, edges);
         LF2MI_LAUNCHED();
     }
-    launch_bricks<KIND, float>(A, dense_workers(p), p->dgroups, p->ndgroup, st);
+    launch_bricks<KIND, float>(p, A, dense_workers(p), p->dgroups, p->ndgroup, st);
     LF2MI_LAUNCHED();
     return LF2MI_OK;
 }
@@ -3854,12 +3886,13 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
         if (b64_used(p)) {
             const BrickIndex V = brick_view(p->bb, N);
             const unsigned gb = (unsigned)brick_items(V.nbk, p->np);
+            const int mg = merge_items(p->np, DEP_MERGE);
             switch (kind) {
-                case 0: deposit_brick64_kernel<0><<<gb, bw_wg<0>(), 0, st>>>(A, V); break;
-                case 1: deposit_brick64_kernel<1><<<gb, bw_wg<1>(), 0, st>>>(A, V); break;
-                case 2: deposit_brick64_kernel<2><<<gb, bw_wg<2>(), 0, st>>>(A, V); break;
-                case 3: deposit_brick64_kernel<3><<<gb, bw_wg<3>(), 0, st>>>(A, V); break;
-                default: deposit_brick64_kernel<4><<<gb, bw_wg<4>(), 0, st>>>(A, V); break;
+                case 0: deposit_brick64_kernel<0><<<gb, bw_wg<0>(), 0, st>>>(A, V, mg); break;
+                case 1: deposit_brick64_kernel<1><<<gb, bw_wg<1>(), 0, st>>>(A, V, mg); break;
+                case 2: deposit_brick64_kernel<2><<<gb, bw_wg<2>(), 0, st>>>(A, V, mg); break;
+                case 3: deposit_brick64_kernel<3><<<gb, bw_wg<3>(), 0, st>>>(A, V, mg); break;
+                default: deposit_brick64_kernel<4><<<gb, bw_wg<4>(), 0, st>>>(A, V, mg); break;
             }
             LF2MI_LAUNCHED();
             return LF2MI_OK;
@@ -3966,11 +3999,11 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
                 if (int rc = launch_tiles_dense<unsigned long long>(p, A, true, false, st)) return rc;
             } else {
                 switch (kind) {
-                    case 0: launch_bricks<0, unsigned long long>(A, g, nullptr, nullptr, st); break;
-                    case 1: launch_bricks<1, unsigned long long>(A, g, nullptr, nullptr, st); break;
-                    case 2: launch_bricks<2, unsigned long long>(A, g, nullptr, nullptr, st); break;
-                    case 3: launch_bricks<3, unsigned long long>(A, g, nullptr, nullptr, st); break;
-                    default: launch_bricks<4, unsigned long long>(A, g, nullptr, nullptr, st); break;
+                    case 0: launch_bricks<0, unsigned long long>(p, A, g, nullptr, nullptr, st); break;
+                    case 1: launch_bricks<1, unsigned long long>(p, A, g, nullptr, nullptr, st); break;
+                    case 2: launch_bricks<2, unsigned long long>(p, A, g, nullptr, nullptr, st); break;
+                    case 3: launch_bricks<3, unsigned long long>(p, A, g, nullptr, nullptr, st); break;
+                    default: launch_bricks<4, unsigned long long>(p, A, g, nullptr, nullptr, st); break;
                 }
             }
             LF2MI_LAUNCHED();
@@ -4006,11 +4039,11 @@ static int deposit_impl(lf2mi_parts p, int kind, void *field, int halo, int targ
         }
     }
     switch (kind) {
-        case 0: launch_bricks<0, float>(A, g, nullptr, nullptr, st); break;
-        case 1: launch_bricks<1, float>(A, g, nullptr, nullptr, st); break;
-        case 2: launch_bricks<2, float>(A, g, nullptr, nullptr, st); break;
-        case 3: launch_bricks<3, float>(A, g, nullptr, nullptr, st); break;
-        default: launch_bricks<4, float>(A, g, nullptr, nullptr, st); break;
+        case 0: launch_bricks<0, float>(p, A, g, nullptr, nullptr, st); break;
+        case 1: launch_bricks<1, float>(p, A, g, nullptr, nullptr, st); break;
+        case 2: launch_bricks<2, float>(p, A, g, nullptr, nullptr, st); break;
+        case 3: launch_bricks<3, float>(p, A, g, nullptr, nullptr, st); break;
+        default: launch_bricks<4, float>(p, A, g, nullptr, nullptr, st); break;
     }
     LF2MI_LAUNCHED();
     return LF2MI_OK;
@@ -4050,7 +4083,7 @@ int lf2mi_gather_kick_drift(lf2mi_parts p, const void *phi, int halo, double dt_
         if (vmax2) LF2MI_HIP(hipMemsetAsync(p->vmax_f64, 0, sizeof(unsigned long long), st));
         {
             LF2MI_PROF("gkd_f64", st);
-            if (bricks && phi) gkd_brick64_kernel<<<(unsigned)brick_items(V.nbk, p->np), 256, 0, st>>>(A, V);
+            if (bricks && phi) gkd_brick64_kernel<<<(unsigned)brick_items(V.nbk, p->np), 256, 0, st>>>(A, V, merge_items(p->np, G64_MERGE));
             else gkd_f64_kernel<<<grid1(p->np), 256, 0, st>>>(A);
             LF2MI_LAUNCHED();
         }
