@@ -3006,14 +3006,25 @@ static int launch_tiles_dense(lf2mi_parts_s *p, const DepArgs &A, bool overwrite
     return LF2MI_OK;
 }
 
-// the other kinds (and the scalar kind with per-particle masses) into a periodic target with
-// 8^3 bricks, four to a tile, where the tiles beat the brick windows: large lattices and, from
-// 192, sparse ones (microseconds, tiles / windows, at 1 and 1/4 particle per cell: vector
-// 160^3 149 / 119 and 106 / 99, 256^3 500 / 466 and 336 / 384, 512^3 3519 / 3643 and 2273 / 3008;
-// VecVec 256^3 977 / 893 and 659 / 664, 512^3 7135 / 7074 and 4573 / 5111)
+// The other kinds (and the scalar kind with per-particle masses) into a periodic target with 8^3
+// bricks, four to a tile.  The tiles' cost is the field's, which they store once, the windows' the
+// particles' and their bricks' flushes: tiles on large lattices with few particles per brick, all from
+// 512^3; the CIC-NGP vector, with half the terms, up to more particles.  Evenly spread particles, microseconds, windows / tiles (the tiles' sums
+// are also the same from run to run where no brick is dense):
+//                               vector          VecVec           vector NGP     tensor NGP
+//   128^3, 128 per brick          65 / 66         104 / 101        55 / 47        90 / 74
+//   160^3, 128                    117 / 98        182 / 159        99 / 67        155 / 113
+//   160^3, 512                    141 / 143       210 / 258        118 / 104      194 / 196
+//   256^3, 256                    468 / 369       825 / 727        398 / 263      711 / 557
+//   256^3, 512                    510 / 486       778 / 944        419 / 367      748 / 750
+//   256^3, 1024                   607 / 880       1267 / 1746      435 / 680      862 / 1319
+// Clustered ones take less by windows throughout (128^3, 128 per brick: vector 54 / 100, tensor NGP
+// 68 / 121; 256^3, 256: vector 400 / 475, vector NGP 325 / 328), which the host cannot know.
 static bool tiles_c_path(const lf2mi_parts_s *p, int kind, int target, bool pm) {
-    return (kind != LF2MI_PROJ_SCALAR || pm) && target == LF2MI_DEP_PERIODIC && p->g.B == 8 &&
-           p->g.NB % TC_TB == 0 && p->N <= 1024 && p->N >= 192 && (p->N >= 512 || p->np < 256 * p->g.nbk);
+    if ((kind == LF2MI_PROJ_SCALAR && !pm) || target != LF2MI_DEP_PERIODIC || p->g.B != 8 || p->g.NB % TC_TB != 0 ||
+        p->N > 1024)
+        return false;
+    return p->N >= 512 || (p->N >= 160 && p->np < (kind == LF2MI_PROJ_VECTOR_NGP ? 768 : 384) * p->g.nbk);
 }
 
 // the shell buffer of deposit_tiles_c_kernel (grown on demand), its layout, the fold and the
