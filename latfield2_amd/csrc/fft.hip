@@ -818,10 +818,14 @@ static int launch_strided(StridedArgs<T> A, int S, int mode, int nbatch, hipStre
     // meet in one L2 (512^3 forward, y pass into the unpadded k-field: one component 0.92 ->
     // 0.89 ms for the whole transform, three 3.04 -> 2.66, six 6.47 -> 5.57; FP64 one component
     // 1.97 -> 1.75).  For rows only read so, below 512, where the field stays in the last-level
-    // cache (256^3 backward 90 -> 81 us; at 512^3 0.78 -> 0.82 ms with it).
+    // cache (256^3 backward 90 -> 81 us; at 512^3 0.78 -> 0.82 ms with it).  Not where the field is about
+    // in the L2s as it is (one transform without / with it, us, by the MB of its k-field: 64^3 FP64
+    // six components, 13: 23.3 / 25.0; 80^3 FP64 three, 13: 24.3 / 27.5; 128^3 FP64 one, 17: 31.1 / 32.3;
+    // 96^3 FP32 six, 22: 35.6 / 35.1; 128^3 FP32 three, 26: 37.8 / 34.9; 160^3 FP64 one, 33: 40.9 / 37.5).
     const int64_t line = 128 / (int64_t)sizeof(cplx<T>);
-    A.remap = (A.out_es | A.out_bs | A.out_col0) % line != 0 ||
-              (N < 512 && (A.in_es | A.in_bs | A.in_col0) % line != 0);
+    const bool beyond_l2 = (int64_t)A.ncols * N * nbatch * (int64_t)sizeof(cplx<T>) >= (int64_t)20 << 20;
+    A.remap = beyond_l2 && ((A.out_es | A.out_bs | A.out_col0) % line != 0 ||
+                            (N < 512 && (A.in_es | A.in_bs | A.in_col0) % line != 0));
     constexpr int WG = Tune<T>::WG;
     constexpr int L = Tune<T>::template strided_L<N>();
     constexpr int LG = Tune<T>::template green_L<N>();
