@@ -356,7 +356,7 @@ inline BrickIndex brick_view(const BrickBuild &B, int N) {
 // items there can be, and workgroups of a kernel that takes one item each
 inline int64_t brick_items(int64_t nbk, int64_t np) { return nbk + np / BRK_ITEM + 1; }
 
-// a group of `merge` consecutive items of one brick: the workgroup of the first takes them all.
+// a group of `merge` (a power of two) consecutive items of one brick: the workgroup of the first takes them all.
 // Uniform over the workgroup; false when there is nothing to do.
 struct BrickRange {
     int b, p0, n, ox, oy, oz;  // list entries p0 + [0, n)
@@ -365,7 +365,7 @@ __device__ __forceinline__ bool brick_range(const BrickIndex &V, int it, int mer
     if (it >= V.istart[V.nbk]) return false;
     r.b = V.item[it];
     const int k = it - V.istart[r.b];
-    if (k % merge != 0) return false;
+    if ((k & (merge - 1)) != 0) return false;
     const BrickRun e = brick_run(V.start[r.b], V.start[r.b + 1], k * BRK_ITEM, merge * BRK_ITEM);
     r.p0 = e.p0;
     r.n = e.n;

@@ -2240,39 +2240,33 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs 
     auto group = [&](int b, int p0, int len) {
         const int p1 = min(A.start[b + 1], p0 + len);
         const int o[3] = {(b % NB) * B, ((b / NB) % NB) * B, (b / (NB * NB)) * B};
-        // A round's particles are requested before the last one's terms are added; not for six
-        // components, whose three workgroups per CU that costs registers (256^3, one round per brick:
-        // 751 -> 826 us).
-        constexpr bool AHEAD = KindC<KIND>::C < 6;
-        int cell = -1;
-        float u[3], v[3] = {0.f, 0.f, 0.f}, m = A.mass_nv;
-        auto fetch = [&](int p) {
-            cell = -1;
-            if (p >= p1) return;
-            cell = A.s.cell[p];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                u[d] = A.s.off[d][p];
-                if constexpr (KIND > 0) v[d] = A.s.vel[d][p];
-            }
-            if (A.s.mass) m = A.s.mass[p] * A.mass_nv;
-        };
-        if (AHEAD) fetch(p0 + (int)threadIdx.x);
         for (int i = threadIdx.x; i < bw_size<KIND>(); i += WG) win[i] = W(0);
         __syncthreads();
         for (int p = p0 + (int)threadIdx.x; p < p1; p += WG) {
-            if (!AHEAD) fetch(p);
+            // Every load before the first use of one: up to 9 % of all kinds but the native scalar, which
+            // loses that where bricks are small (172^3, 22 particles each: 145 -> 152 us).  Loads a round
+            // ahead gain nothing over it, and cost the kinds of few terms up to a fifth there.
+            constexpr bool FIRST = KIND != 0 || FX;
+            const int cell = A.s.cell[p];
+            float u[3], v[3] = {0.f, 0.f, 0.f}, m = 0.f;
+            if constexpr (FIRST) {
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    u[d] = A.s.off[d][p];
+                    if constexpr (KIND > 0) v[d] = A.s.vel[d][p];
+                }
+                m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
+            }
             int c[3];
             decode_cell(cell, A.g, c[0], c[1], c[2]);
             BwParticle<float> P;
 #pragma unroll
             for (int d = 0; d < 3; ++d) {
                 P.l[d] = c[d] - o[d];
-                bw_weights(P, d, u[d]);
+                bw_weights(P, d, FIRST ? u[d] : A.s.off[d][p]);
             }
-            const float vp[3] = {v[0], v[1], v[2]}, mp = m;
-            if (AHEAD) fetch(p + WG);
-            bw_particle<KIND>(win, P, mp, vp, A.fxs);
+            if constexpr (!FIRST) m = A.s.mass ? A.s.mass[p] * A.mass_nv : A.mass_nv;
+            bw_particle<KIND>(win, P, m, v, A.fxs);
         }
         __syncthreads();
         if constexpr (FX) bw_flush<KIND>(win, A.fx, N, A.h, A.tgt, o[0], o[1], o[2]);
@@ -2294,7 +2288,7 @@ __global__ __launch_bounds__(bw_wg<KIND>()) void deposit_brick32_kernel(DepArgs 
     const int it = blockIdx.x;
     if (it >= A.istart[A.g.nbk]) return;
     const int b = A.item_bucket[it], k = it - A.istart[b];
-    if (k % merge == 0) group(b, A.start[b] + k * ITEM_P, merge * ITEM_P);
+    if ((k & (merge - 1)) == 0) group(b, A.start[b] + k * ITEM_P, merge * ITEM_P);
 }
 
 struct Gkd64Args {
