@@ -904,8 +904,9 @@ static int launch_x(const XArgs<T> &A, int S, hipStream_t st) {
     constexpr int L = Tune<T>::template x_L<N>();
     constexpr int LMAX = Tune<T>::template x_L_max<N>();
     // the wide tile too where only that is whole components (three at 512^3, there and back: 5.14
-    // -> 5.03 ms; the narrow one leaves a fourth of its lines empty)
-    if (A.C <= L && (L % A.C == 0 || LMAX % A.C != 0)) return launch_x_tile<T, N, L>(A, S, st);
+    // -> 5.03 ms; the narrow one leaves a fourth of its lines empty), but at 1024, whose
+    // 56 KB leave two workgroups per CU (three components forward: 23.7-25.3 ms, narrow 21.8-23.3)
+    if (A.C <= L && (L % A.C == 0 || LMAX % A.C != 0 || N >= 1024)) return launch_x_tile<T, N, L>(A, S, st);
     if constexpr (LMAX > L) {
         if (A.C <= LMAX) return launch_x_tile<T, N, LMAX>(A, S, st);
     }
