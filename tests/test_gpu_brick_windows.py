@@ -98,3 +98,29 @@ def test_items_per_workgroup(n, prec, tol):
             q.addParticles(pos[half], vel[half])
             q.gather_kick_drift(phi, 0.1, 0.0)
             assert np.array_equal(q.download()["vel"], got[half])
+
+
+@pytest.mark.parametrize("N", [64, 128, 192])
+@pytest.mark.parametrize("n", [1, 700, 1500])
+def test_few_particles_in_the_scalar_tiles(N, n):
+    """few particles on a large lattice, without a dense brick and with one: the launch is then the
+    fold's, whose workgroups outnumber the particles' work"""
+    announce(f"scalar tiles N={N} n={n}")
+    rng = np.random.default_rng(n)
+    pos = rng.random((n, 3))
+    if n > 1024:
+        pos = (N // 8 - 1 + pos) * 8 / N  # all in the last brick, whose upper nodes wrap
+    parts = lf.Particles(N, n, lf.F32, mass=1.0 / n)
+    parts.addParticles(pos, np.zeros((n, 3)))
+    d = parts.download()
+    s = slice(1, N + 1)
+    ref = oracle("scalar", d, N, np.full(n, 1.0 / n), True)
+    for target, before in ((lf.DEP_PERIODIC_SET, 7.0), (lf.DEP_PERIODIC, 0.0)):
+        f = lf.Field(lf.Lattice(3, N, 1), 1, lf.F32)
+        f.t.fill_(before)
+        parts.deposit(lf.PROJ_SCALAR, f, target)
+        torch.cuda.synchronize()
+        got = real_np(f)
+        assert rel_l2(got[s, s, s], ref[s, s, s]) <= 1e-6
+        got[s, s, s] = 0.0
+        assert not got.any()  # the ghosts are cleared, or were and stay
