@@ -84,14 +84,13 @@ __device__ __forceinline__ int brick_of(int x, int y, int z, int NB) {
     return (x / BRK) + NB * ((y / BRK) + NB * (z / BRK));
 }
 
-// place of a particle among those of its brick so far: lanes of a wave with the same brick
-// share one atomic, and the groups' atomics go out together after the groups are found (one
-// round trip per wave instead of one per group: counting 16.8 M particles in lattice order,
-// 8 bricks to a wave, took 358 us that way).  Every lane of the wave calls it.
-__device__ __forceinline__ int brick_rank(int *__restrict__ count, int brick, bool active) {
+// the groups of lanes of a wave with the same brick: a lane's group's first lane, its place in the
+// group and the group's size.  Every lane of the wave calls it.
+__device__ __forceinline__ void brick_groups(int brick, bool active, int &first, int &place, int &size) {
     unsigned long long todo = __ballot(active);
     const int lane = __lane_id();
-    int first = lane, place = 0, size = 0;
+    first = lane;
+    place = size = 0;
     while (todo) {
         const int leader = __ffsll((long long)todo) - 1;
         const int key = __builtin_amdgcn_readlane(brick, leader);
@@ -103,8 +102,17 @@ __device__ __forceinline__ int brick_rank(int *__restrict__ count, int brick, bo
         }
         todo &= ~grp;
     }
+}
+
+// place of a particle among those of its brick so far: lanes of a wave with the same brick
+// share one atomic, and the groups' atomics go out together after the groups are found (one
+// round trip per wave instead of one per group: counting 16.8 M particles in lattice order,
+// 8 bricks to a wave, took 358 us that way).  Every lane of the wave calls it.
+__device__ __forceinline__ int brick_rank(int *__restrict__ count, int brick, bool active) {
+    int first, place, size;
+    brick_groups(brick, active, first, place, size);
     int base = 0;
-    if (active && lane == first) base = atomicAdd(&count[brick], size);
+    if (active && (int)__lane_id() == first) base = atomicAdd(&count[brick], size);
     return __shfl(base, first) + place;
 }
 
@@ -305,15 +313,65 @@ inline int brick_scan(const BrickScan &S, int n, hipStream_t st) {
     return LF2MI_OK;
 }
 
+// Counts and ranks of PER particles per thread.  The groups of a workgroup's waves meet in an LDS hash
+// table of their bricks (twice as many slots as there can be bricks), and a brick takes one global
+// atomic per workgroup: with one per wave the counters of crowded bricks, a few lines, were the bound
+// (2 M clustered particles on 64^3: 82 us).
+template <int PER>
 static __global__ __launch_bounds__(256) void brick_count_kernel(int64_t np, const int32_t *__restrict__ cell, int N,
                                                                  int NB, int lgN, int *__restrict__ count,
                                                                  int *__restrict__ rank) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const bool in = i < np;
-    int x = 0, y = 0, z = 0;
-    if (in) brick_decode(cell[i], N, lgN, x, y, z);
-    const int r = brick_rank(count, brick_of(x, y, z, NB), in);
-    if (in) rank[i] = r;
+    constexpr int HT = 512 * PER, HASH = PER == 4 ? 21 : 23;  // slots, and the shift to the key's top bits
+    static_assert(HT == 1 << (32 - HASH), "table size");
+    __shared__ int hkey[HT];
+    __shared__ int hval[HT];  // the bricks' particles so far, then their base in the brick
+    for (int i = threadIdx.x; i < HT; i += 256) {
+        hkey[i] = -1;
+        hval[i] = 0;
+    }
+    const int64_t i0 = (int64_t)blockIdx.x * (256 * PER) + threadIdx.x;
+    int brick[PER], ent[PER], place[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int64_t i = i0 + 256 * k;
+        brick[k] = -1;
+        if (i < np) {
+            int x, y, z;
+            brick_decode(cell[i], N, lgN, x, y, z);
+            brick[k] = brick_of(x, y, z, NB);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        int first, size, e = 0, base = 0;
+        brick_groups(brick[k], brick[k] >= 0, first, place[k], size);
+        if (brick[k] >= 0 && (int)__lane_id() == first) {
+            e = (int)(((unsigned)brick[k] * 2654435761u) >> HASH);
+            for (;;) {
+                const int old = atomicCAS(&hkey[e], -1, brick[k]);
+                if (old == -1 || old == brick[k]) break;
+                e = (e + 1) & (HT - 1);
+            }
+            base = atomicAdd(&hval[e], size);
+        }
+        ent[k] = __shfl(e, first);
+        place[k] += __shfl(base, first);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < HT; i += 256)
+        if (hkey[i] >= 0) hval[i] = atomicAdd(&count[hkey[i]], hval[i]);
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        const int64_t i = i0 + 256 * k;
+        if (i < np) rank[i] = hval[ent[k]] + place[k];
+    }
+}
+// four particles per thread where that still gives every CU four workgroups
+inline void brick_count(int64_t np, const int32_t *cell, int N, int NB, int lgN, const BrickBuild &B, hipStream_t st) {
+    if (np < 1024 * 1024) brick_count_kernel<1><<<blocks_for(np, 256), 256, 0, st>>>(np, cell, N, NB, lgN, B.count, B.rank);
+    else brick_count_kernel<4><<<blocks_for(np, 1024), 256, 0, st>>>(np, cell, N, NB, lgN, B.count, B.rank);
 }
 
 static __global__ __launch_bounds__(256) void brick_list_kernel(int64_t np, const int32_t *__restrict__ cell, int N,
@@ -336,7 +394,7 @@ inline int brick_build_ranked(const int32_t *cell, int64_t np, int N, const Bric
 }
 inline int brick_build(const int32_t *cell, int64_t np, int N, const BrickBuild &B, hipStream_t st) {
     const int NB = (N + BRK - 1) / BRK, lgN = is_pow2(N) ? __builtin_ctz((unsigned)N) : -1;
-    brick_count_kernel<<<blocks_for(np, 256), 256, 0, st>>>(np, cell, N, NB, lgN, B.count, B.rank);
+    brick_count(np, cell, N, NB, lgN, B, st);
     LF2MI_LAUNCHED();
     return brick_build_ranked(cell, np, N, B, st);
 }

@@ -2863,7 +2863,7 @@ static int b64_fill(lf2mi_parts_s *p, const double *pos, const double *vel, cons
         if (pos) cells64_kernel<<<g, 256, 0, st>>>(p->np, pos, N, p->bb.list);
         else ic_stage64_kernel<<<g, 256, 0, st>>>(A, p->b64, N, p->bb.list);
         LF2MI_LAUNCHED();
-        brick_count_kernel<<<g, 256, 0, st>>>(p->np, p->bb.list, N, V.NB, V.lgN, p->bb.count, p->bb.rank);
+        brick_count(p->np, p->bb.list, N, V.NB, V.lgN, p->bb, st);
         LF2MI_LAUNCHED();
         if (int rc = brick_scan(p->bb.scan(), V.nbk, st)) return rc;
         O.start = p->bb.start;
