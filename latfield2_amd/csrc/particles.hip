@@ -2338,7 +2338,13 @@ __device__ __forceinline__ void vmax64(const Gkd64Args &A, unsigned long long m)
     for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o));
     if (lane_id() == 0) wm[threadIdx.x >> 6] = m;
     __syncthreads();
-    if (threadIdx.x == 0) atomicMax(A.vmax2, max(max(wm[0], wm[1]), max(wm[2], wm[3])));
+    if (threadIdx.x == 0) {
+        m = max(max(wm[0], wm[1]), max(wm[2], wm[3]));
+        // the value only grows, so one that is seen to be as large needs no atomic: tens of thousands of
+        // them on one address were longer than the gather of a sparse lattice (1 M clustered particles on
+        // 256^3: 458 us with the maximum, 185 without)
+        if (m > __hip_atomic_load(A.vmax2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(A.vmax2, m);
+    }
 }
 
 // one workgroup per group of items of a brick: the brick's window of phi, then its force
