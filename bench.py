@@ -7,7 +7,7 @@ box length 1), FP32 path: zero rho -> CIC deposit -> mean-subtracted Poisson sol
 (-1/K^2, 1/N^3) -> CIC gather + kick + drift -> re-bucket.  Inputs are generated on
 the device and resident in HBM before the timed region.
 
-Also measured (outside the timed region): the plain FP64 GPU path on the same
+Also measured (outside the timed region): the FP64 GPU path on the same
 workload, the FP32-vs-FP64 potential difference, per-kernel times with HIP events on
 the launch stream (roofline of the dominant kernel), and the FP64 CPU oracle on a
 full workload, on all the host threads granted and on one (cpu_baseline).
@@ -368,7 +368,7 @@ def main():
 
     extra = {}
     if not args.no_fp64:
-        log("FP64 plain path on the same workload")
+        log("FP64 path on the same workload")
         p64, r64, f64, pl64 = make_workload(lf, N, Np, lf.F64)
         # accuracy: one step from the same IC on both paths
         lf.pm_step(p64, pl64, r64, f64, dt, dt)

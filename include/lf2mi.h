@@ -319,7 +319,8 @@ int lf2mi_parts_ic_blobs(lf2mi_parts p, int64_t np, int nblobs, double alpha,
  *   target LF2MI_DEP_UNFOLDED adds exactly what the reference _project adds (ghost
  *          nodes included, follow with lf2mi_projection_comm); LF2MI_DEP_PERIODIC adds
  *          the folded result into the interior (== _project + _comm on the interior).
- *   acc   LF2MI_ACC_NATIVE, or LF2MI_ACC_FIXED64 (F32 containers): every particle's term is
+ *   acc   LF2MI_ACC_NATIVE, whose last bits may differ from run to run (float atomics in no
+ *         fixed order), or LF2MI_ACC_FIXED64 (F32 containers): every particle's term is
  *         rounded to an int64 fixed point and summed in integers, so the result does not
  *         depend on the order of the additions (bitwise reproducible); scalar kind: 2^-32 of
  *         the mass per unit weight; vector and tensor kinds: per component 2^(e-62) with

@@ -8,8 +8,8 @@
 // nodes go to the field, in rows (100 G atomics/s).  The index costs 8 bytes per particle (list and
 // rank) and about 16 per brick, an order of the particles beside it 4 (their places) to 12.
 //
-// Building it: brick_count_kernel counts the cells in particle order (brick_rank: the
-// particle's place among its brick's, one global atomic per brick and wave), one or two scan
+// Building it: brick_count_kernel counts the cells in particle order and leaves each particle's
+// place among its brick's (one global atomic per brick and workgroup), one or two scan
 // kernels turn the counts into starts (and clear them for the next time), and
 // brick_list_kernel writes each particle's number at start + place.  Counted in particle order
 // a list consists of runs of consecutive particles, which the kernels that walk it read in

@@ -11,11 +11,11 @@
 // of the brick's nodes.  After a drift the container is re-bucketed with a counting sort
 // (histogram -> scan -> scatter into the second buffer).
 //
-// F64 representation (the plain path): absolute FP64 positions and velocities, put into brick
-// order at upload and every few drifts, with a brick index beside them (bricks.hpp): deposits
-// sum a brick's particles in an FP64 LDS window, the gather reads a brick's window of phi.
-// Where few particles fall into a brick both go particle by particle in upload order: FP64
-// atomics into the field, phi straight from HBM.  Downloads come in upload order either way.
+// F64 representation: absolute FP64 positions and velocities, put into brick order at upload and
+// every few drifts, with a brick index beside them (bricks.hpp): deposits sum a brick's particles
+// in an FP64 LDS window, the gather reads a brick's window of phi.  Where few particles fall into
+// a brick, or the index finds no room, both go particle by particle in upload order: FP64 atomics
+// into the field, phi straight from HBM.  Downloads come in upload order either way.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
@@ -1974,7 +1974,7 @@ __global__ __launch_bounds__(DEP_WG) void gkd_small_kernel(GkdArgs A, const int4
     else gkd_dense<BC>(A, (int)blockIdx.x - nbk);
 }
 
-// ---------------------------------------------------------------- F64 plain path
+// ---------------------------------------------------------------- F64
 struct Dep64Args {
     Soa64 s;
     int64_t np;
@@ -2072,8 +2072,8 @@ __global__ void deposit_f64_kernel(Dep64Args A) {
 // deposit).  No sort: a wave's particles rarely share a node, and nearly sorted ones would more
 // often (LDS atomics of random cells 1500 G/s, of neighbouring ones 1290-1380).  FP32 container
 // at 256^3, 512 particles per brick, microseconds, against sorting a brick's items by cell and
-// summing runs in registers first: scalar 247 -> 218, vector 710 -> 466, VecVec 1572 -> 831,
-// CIC-NGP 580 -> 387 and 1188 -> 692.  What bounds it: of VecVec's 945 us before the layout below
+// summing runs in registers first: scalar 247 -> 218, vector 710 -> 460, VecVec 1572 -> 710,
+// CIC-NGP 580 -> 384 and 1188 -> 675.  What bounds it: of VecVec's 945 us before the layout below
 // the LDS atomics were 560 and the flush 59; of the FP64 container's 280 for a scalar the flush
 // is half.  Without gain: int64 windows of scaled sums, whose LDS atomics are twice as fast but
 // need a pass for the scale and conversions (equal to 25 % slower); nodes that only one window

@@ -15,13 +15,11 @@ KINDS = [(lf.PROJ_SCALAR, 1, orc.scalar_comm), (lf.PROJ_VECTOR, 3, orc.vector_co
          (lf.PROJ_VECTOR_NGP, 3, orc.vector_ngp_comm), (lf.PROJ_SYMTENSOR_NGP, 6, orc.symtensor_ngp_comm)]
 
 
-@pytest.mark.parametrize("kind,C,comm", KINDS)
-@pytest.mark.parametrize("N", [215, 216, 255, 256, 257])
+AROUND = [(k, N) for k in KINDS for N in ((215, 216) if k[0] == lf.PROJ_SYMTENSOR_NGP else (255, 256, 257))]
+
+
+@pytest.mark.parametrize("kind,C,comm,N", [(*k, N) for k, N in AROUND])
 def test_fold_bit_exact_around_the_rule(kind, C, comm, N):
-    if C == 6 and (kind == lf.PROJ_VECVEC) != (N >= 255):
-        pytest.skip("this kind's line lies elsewhere")
-    if C < 6 and N < 255:
-        pytest.skip("this kind's line lies elsewhere")
     announce(f"fold N={N} kind={kind}")
     h, G = 1, N + 2
     # only the two outermost layers on each side take part: the inside is zero
