@@ -666,6 +666,9 @@ int lf2mi_diffpm_create_keep(int N, int64_t np, int nsteps, double mass, double 
         lf2mi_diffpm_destroy(m);
         return rc;
     }
+    // the counters have to be clear before the first use, which may be on a stream that does not wait
+    // for this one
+    (void)hipStreamSynchronize(nullptr);
     *out = m;
     return LF2MI_OK;
 }

@@ -3306,6 +3306,9 @@ int lf2mi_parts_create(int N, int64_t capacity, int dtype, int flags, lf2mi_part
         hipMemset(p->ndgroup, 0, sizeof(int));
         hipMemset(p->nchunk, 0, 2 * sizeof(int));
     }
+    // the counters have to be clear before the first use, which may be on a stream that does not wait
+    // for this one
+    (void)hipStreamSynchronize(nullptr);
     *out = p;
     return LF2MI_OK;
 }
